@@ -1,7 +1,7 @@
-// igemm.h -- the implicit-GEMM convolution kernels on the fp32 matrix cores,
-// shared by k_igemm.hip (the plain launchers) and k_igemm_fused.hip (the
-// launchers with a neighbouring pass folded into a kernel's operand loads or
-// epilogue).  Design notes and the MFMA lane layout: k_igemm.hip.
+// igemm.h -- the implicit-GEMM convolution kernels on the matrix cores, shared
+// by k_igemm.hip (the plain launchers) and k_igemm_fused.hip (the launchers
+// with a neighbouring pass folded into a kernel's operand loads or epilogue).
+// Design notes, the operand split and the MFMA lane layout: k_igemm.hip.
 #pragma once
 #include "nn_hip_rt.h"
 #include "nnk_common.h"
@@ -21,21 +21,148 @@ struct ConvShape {
     FastDiv wo, ho;  // output pixel decode m -> (b, oh, ow)
 };
 
-// float4 slot of (row, chunk) in a [128][8] tile.  The xor spreads any 8
-// consecutive rows of one chunk over the 8 chunk positions, and any 16
-// consecutive rows over distinct (row parity, position) pairs, so 128-bit
-// accesses whose lane groups cover 128 or 256 bytes of banks do not conflict.
-__device__ __forceinline__ int slot(int row, int chunk) {
-    return row * 8 + (chunk ^ (row & 7) ^ ((row >> 3) & 1));
+// XCD-aware tile order.  Workgroups are dispatched round-robin over the
+// device's 8 XCDs (workgroup L on XCD L % 8), each with its own L2.  Tile
+// L' = xcd_order(L) gives XCD x a contiguous range of tiles, so tiles that
+// read the same activations run in the same L2 instead of on different XCDs.  A bijection of [0, total) for any total.
+constexpr int kXcds = 8;
+__device__ __forceinline__ int xcd_order(int L, int total) {
+    const int x = L % kXcds, j = L / kXcds, q = total / kXcds, r = total % kXcds;
+    return x * q + min(x, r) + j;
 }
 
-// float offset of (k, n) in a [32][BN] B tile: rows 4..7 of every 8 rotated by 32
-template <int BN>
-__device__ __forceinline__ int kslot(int k, int n) {
-    return k * BN + ((n + 32 * ((k >> 2) & 1)) & (BN - 1));
+// ---------------------------------------------------------------------------
+// fp32 operands on the bf16 matrix cores.  v = p0 + p1 + p2 with p0 = bf16(v),
+// p1 = bf16(v - p0), p2 = v - p0 - p1: 8 + 8 + 8 significand bits, so the sum
+// is exact for every v of 2^-110 and above (below it p2 reaches under the
+// smallest subnormal bf16).  a b is then the sum of the products p_i q_j; the
+// six with i + j <= 2 are taken, the other three are below 2^-25 |a b|.  Each
+// product of two bf16 is exact and the matrix core adds in fp32.
+// ---------------------------------------------------------------------------
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+constexpr int kPlanes = 3;
+
+// the planes of (a, b), a in the low half
+__device__ __forceinline__ void split2(float a, float b, uint32_t (&p)[kPlanes]) {
+#pragma unroll
+    for (int i = 0; i < kPlanes; ++i) {
+        const f32x2 v = {a, b};
+        p[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+        if (i + 1 < kPlanes) {
+            a = a - __uint_as_float(p[i] << 16);
+            b = b - __uint_as_float(p[i] & 0xffff0000u);
+        }
+    }
 }
 
-enum { kEpiNone = 0, kEpiBias = 1, kEpiGain = 2 };
+// LDS tiles hold rows of 32 k, 64 bytes (four 16-byte chunks) a plane, and
+// every access is 16 bytes a lane.  The order of a row's chunks depends on the
+// row (swz), so that the fragment reads, 16 consecutive rows at one chunk,
+// fall on 16 distinct 16-byte groups of the 64 banks (5.3 cycles a wave read
+// against 8 with chunks ordered by (row / 2) % 4), and so do the writes of
+// lanes along a row, 4 rows x 4 chunks.
+//   rowslot: the three planes of a row beside each other (the convolution's
+//     activations, read at any row offset);
+//   slot: a plane of its own, two rows to a 128-byte line, the halves of rows
+//     16 apart swapped for the transposing writes, 16 rows two apart (the
+//     weight gradient's tiles).
+__device__ __forceinline__ int swz(int row, int c) { return c ^ ((row >> 2) & 3); }
+constexpr int kRowSlots = 4 * kPlanes;  // uint4 per row of all planes
+__device__ __forceinline__ int rowslot(int row, int c) { return row * kRowSlots + swz(row, c); }
+constexpr int kRow4 = 4;  // uint4 per row of one plane
+__device__ __forceinline__ int slot(int row, int c) {
+    return (row >> 1) * 8 + ((row ^ (row >> 4)) & 1) * 4 + swz(row, c);
+}
+
+// the planes of 8 consecutive k
+__device__ __forceinline__ void split8(const float (&v)[8], uint4 (&p)[kPlanes]) {
+    uint32_t d[4][kPlanes];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) split2(v[2 * i], v[2 * i + 1], d[i]);
+#pragma unroll
+    for (int i = 0; i < kPlanes; ++i) p[i] = make_uint4(d[0][i], d[1][i], d[2][i], d[3][i]);
+}
+// ... written stride uint4 apart
+__device__ __forceinline__ void put8(uint4* t, int stride, const float (&v)[8]) {
+    uint4 p[kPlanes];
+    split8(v, p);
+#pragma unroll
+    for (int i = 0; i < kPlanes; ++i) t[i * stride] = p[i];
+}
+
+// a buffer resource at a uniform address: loads then take a scalar base and a
+// 32-bit lane offset instead of a 64-bit address in vector registers
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const float* p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, -1, 0x00020000);
+}
+
+__device__ __forceinline__ float keep(float v, bool ok) { return __uint_as_float(__float_as_uint(v) & (ok ? ~0u : 0u)); }
+
+// A wave's products over 16 k: T x U accumulators of 32 x 32 from the planes of
+// its row tiles' fragments (lane l: row l % 32, k 8 (l / 32) .. + 7).  The
+// matrix core cuts off what an addend has below the last place of the largest
+// one, towards minus infinity.  p0 q0 products lie on a coarse grid and lose
+// next to nothing; the five small products, added to the same accumulator,
+// would lose enough to shift every output by -6e-8 of its root mean square at
+// K = 1152, which sums over many outputs (a bias gradient, a norm's) show.  So
+// they have an accumulator of their own, `cor`, 2^-8 as large: error against
+// 64 bits 2.0e-7 (mean 2e-10) of the root mean square at K = 1152 with standard
+// normal operands, against 5.2e-7 (mean -6e-8) with one accumulator and 6.1e-7
+// with the fp32 MFMA.  Each product runs over all T x U accumulators, so
+// consecutive MFMAs rarely wait for each other's result.
+template <int T, int U>
+__device__ __forceinline__ void products(const uint4 (&a)[kPlanes][T], const uint4 (&b)[kPlanes][U],
+    f32x16 (&acc)[T][U], f32x16 (&cor)[T][U]) {
+    constexpr int PI[6] = {0, 2, 0, 1, 1, 0}, PJ[6] = {0, 0, 2, 1, 0, 1};
+#pragma unroll
+    for (int x = 0; x < 6; ++x)
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                f32x16& d = x ? cor[t][u] : acc[t][u];
+                d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[PI[x]][t]),
+                    __builtin_bit_cast(bf16x8, b[PJ[x]][u]), d, 0, 0, 0);
+            }
+}
+
+// The order of a step's instructions: after each MFMA up to six vector
+// instructions, and a load from LDS or memory where one is left.
+template <int MFMAS>
+__device__ __forceinline__ void sched() {
+#pragma unroll
+    for (int i = 0; i < MFMAS; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // VALU
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // memory read
+    }
+}
+
+// Whether a wave's results must be formed again from the unsplit operands: a
+// value that is not finite (an infinite or NaN operand, or one that rounds to
+// infinity in bf16, splits into NaN planes), or values all so small that an
+// operand may lie below the split's range.
+template <int T, int U>
+__device__ __forceinline__ bool split_failed(const f32x16 (&acc)[T][U]) {
+    bool bad = false;
+    float mx = 0.0f;
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float v = fabsf(acc[t][u][r]);
+                bad |= !(v <= 3.402823466e38f);
+                mx = fmaxf(mx, v);
+            }
+    if (__any(bad)) return true;
+    return !__any(mx >= 0x1p-80f) && __any(mx > 0.0f);
+}
+
 // Fused neighbours of the forward / input-gradient kernel (bit flags), with v
 // the output after bias or gain:
 //   kXeRes : y = wa * res[m, n] + wb * v            (launch_weighted_sum(y, res, v, wa, wb))
@@ -45,290 +172,401 @@ enum { kEpiNone = 0, kEpiBias = 1, kEpiGain = 2 };
 // those of the separate passes bit for bit.
 enum { kXeNone = 0, kXeRes = 1, kXeActG = 2, kXeMod = 4 };
 struct ConvEpi {
+    const float* bias;  // + bias[n], or null
+    const float* gain;  // * gain[0], or null
     const float* res;   // kXeRes: [M][C_out]
     const float* xa;    // kXeActG: [M][C_out]
     const float* cond;  // kXeMod: [B][C_out]
     float* y2;          // kXeMod: [M][C_out]
     float wa, wb;       // kXeRes weights
+    int mp;             // the activation is MP-SiLU (SiLU otherwise)
     FastDiv hw;         // kXeMod: output pixels per sample
 };
-// Source of operand B: the forward's weight Wt[k][n], or the input gradient's
-// flipped weight (sh is then the gradient's convolution: C_in = the layer's
-// C_out, C_out = the layer's C_in, so Wt is [K*K*sh.Cout][sh.Cin]).
-enum { kWFwd = 0, kWFlip = 1 };
 
-template <int EPI, int BN, int WSRC, int XE = kXeNone, int ACT = 0>
-__global__ __launch_bounds__(kTpb, 2) void igemm_fwd(float* __restrict__ Y, const float* __restrict__ X,
-    const float* __restrict__ Wt, const float* __restrict__ bias, const float* __restrict__ gain, ConvShape sh,
-    ConvEpi ep) {
-    constexpr int UT = BN / 64;  // 32-column accumulator tiles per wave
-    // weight float4 loaded per thread: a 4 x 4 block (forward) or BN / 32
-    // rows of one chunk (flipped)
-    constexpr int BQ = WSRC == kWFwd ? 4 : BN / 32;
-    constexpr int NQ = BN / 4;   // forward: n quads of the tile
-    __shared__ float4 As[2][kBM * 8];
-    __shared__ float4 Bs[2][BN * 8];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int wm = w >> 1, wn = w & 1;
-    const int m0 = blockIdx.x * kBM, n0 = blockIdx.y * BN;
-    // loader role: chunk ch of rows r0 + 32 q
-    const int ch = tid & 7, r0 = tid >> 3;
-    int pix[4], ihb[4], iwb[4];
-    bool rok[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int m = m0 + r0 + 32 * q;
-        rok[q] = m < sh.M;
-        const int mm = rok[q] ? m : 0;
-        uint32_t t, ow, b, oh;
-        sh.wo.divmod((uint32_t)mm, t, ow);
-        sh.ho.divmod(t, b, oh);
-        pix[q] = (int)b * sh.H * sh.W;
-        ihb[q] = (int)oh * sh.stride - sh.pad;
-        iwb[q] = (int)ow * sh.stride - sh.pad;
-    }
-    // forward weight roles: n quad n4, k rows 4 kq .. 4 kq + 3 of the slice
-    // (with BN = 64 the second half of the workgroup repeats the first's
-    // loads and stores nothing: every lane loads, see below)
-    const int n4 = tid % NQ, kq = (tid / NQ) % 8;
-    const bool bput = NQ * 8 >= kTpb || tid < NQ * 8;
-    const float* wq = Wt + (size_t)(4 * kq) * sh.Cout + n0 + 4 * n4;
-    // flipped weight: row n0 + r0 + 32 q of the tap's [C_in][C_out] block
-    const float* wrow = Wt + (size_t)(n0 + r0) * sh.Cin + ch * 4;
-    const int KK = sh.K * sh.K;
+// How the activations reach LDS:
+//   kHalo: the rows of all taps once per 32 channels (stride 1, output as large
+//     as the input: the input pixel of output pixel m and tap (kh, kw) is m +
+//     (kh - pad) W + kw - pad, so the pixels of 128 consecutive outputs lie in
+//     128 + 2 pad (W + 1) consecutive rows; taps outside the image read a row of
+//     zeros instead);
+//   kGather: 128 rows per tap and 32 channels, any geometry;
+//   kRagged: as kGather for channel counts that are no multiple of 8 or
+//     pointers that are not 16-byte aligned, loads of 4 bytes.
+enum { kHalo = 0, kGather = 1, kRagged = 2 };
 
-    // Every lane loads (a padding position reads channel ci of pixel 0 and is
-    // zeroed when stored): a branch around a load would make the compiler's
-    // later waits drain the whole vector-memory counter, i.e. wait for the
-    // next slice's loads before the current slice's MFMAs.
-    // Two register sets: the slice two ahead is loaded while the next one is
-    // written to LDS, so a load has two slices of MFMA work to arrive.
-    struct Regs {
-        float4 a[4], b[BQ];
-        bool ok[4];
-    };
-    Regs R0, R1;
-    auto load = [&](int kt, Regs& R) {
-        const int k0 = kt * kBK;
-        const int khw = k0 / sh.Cin, cs = k0 - khw * sh.Cin, ci = cs + ch * 4;
-        const int kh = khw / sh.K, kw = khw - kh * sh.K;
-        // flipped weight: the slice's channels cs.. of tap KK-1-khw, a
-        // uniform offset from each lane's row (held in a scalar register)
-        const int wfo = __builtin_amdgcn_readfirstlane((KK - 1 - khw) * sh.Cout * sh.Cin + cs);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int ih = ihb[q] + kh, iw = iwb[q] + kw;
-            R.ok[q] = rok[q] & ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
-            const int p = R.ok[q] ? pix[q] + ih * sh.W + iw : 0;
-            R.a[q] = ld4(X + (size_t)p * sh.Cin + ci);
-            if constexpr (WSRC == kWFwd) R.b[q] = ld4(wq + (size_t)(k0 + q) * sh.Cout);
-            else if (q < BQ) R.b[q] = ld4(wrow + wfo + 32 * q * sh.Cin);
-        }
-    };
-    // Padding is zeroed by masking the bits (a select of whole float4 values
-    // becomes a select of their addresses, which puts them in scratch memory).
-    auto store = [&](int buf, const Regs& R) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const unsigned mk = R.ok[q] ? 0xffffffffu : 0u;
-            const float4 a = R.a[q];
-            float4 v;
-            v.x = __uint_as_float(__float_as_uint(a.x) & mk);
-            v.y = __uint_as_float(__float_as_uint(a.y) & mk);
-            v.z = __uint_as_float(__float_as_uint(a.z) & mk);
-            v.w = __uint_as_float(__float_as_uint(a.w) & mk);
-            As[buf][slot(r0 + 32 * q, ch)] = v;
-            if constexpr (WSRC == kWFlip) {
-                if (q < BQ) Bs[buf][slot(r0 + 32 * q, ch)] = R.b[q];
-            }
-        }
-        // forward: k rows 4 kq + i, n 4 n4 .. 4 n4 + 3, as loaded
-        if constexpr (WSRC == kWFwd) {
-            if (bput) {
-                float* bs = reinterpret_cast<float*>(&Bs[buf][0]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    *reinterpret_cast<float4*>(bs + kslot<BN>(4 * kq + i, 4 * n4)) = R.b[i];
-            }
-        }
-    };
-
-    f32x16 acc[2][UT];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int u = 0; u < UT; ++u) acc[t][u] = (f32x16){};
-    const int nk = sh.KKC / kBK;
+// Y[m, n] = sum_k A[m, k] B[k, n] with the fused epilogue; FLIP: B is the input
+// gradient's flipped weight (sh is then the gradient's convolution: C_in = the
+// layer's C_out, C_out = the layer's C_in, so Wt is [K*K*sh.Cout][sh.Cin]).
+//
+// A workgroup computes 128 x BN outputs with four waves of 32 columns and 32 T
+// rows.  k runs over slices of 32 channels and, within one, over the taps.
+// Only the activations go through LDS, where the waves share them: they are
+// split into planes as they are stored.  A wave needs its weight columns
+// alone, so it loads them straight into the fragment's registers, a slice
+// ahead, and splits them there; no element of either is split twice per
+// workgroup and slice, and with kHalo none of the activations is per tap.
+// Two workgroups share a CU: one computes while the other stages.
+template <int BN, int MODE, bool FLIP, int XE>
+__global__ __launch_bounds__(kTpb, 2) void conv_x3(float* __restrict__ Y, const float* __restrict__ X,
+    const float* __restrict__ Wt, ConvShape sh, ConvEpi ep) {
+    constexpr int WN = BN / 32, T = WN;  // waves along n; row tiles per wave (4 / (4 / WN))
+    extern __shared__ uint4 As[];        // rowslot(): kHalo halo rows and a row of zeros, else 128 rows
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr = lane & 31, fh = lane >> 5;
-    // epilogue operands, loaded before the pipeline
-    float bn[UT], g = 1.0f;
+    const int nb = (sh.Cout + BN - 1) / BN;
+    const int tl = xcd_order((int)blockIdx.x, (int)gridDim.x);
+    const int m0 = tl / nb * kBM, n0 = tl % nb * BN;
+    const int wrow = w / WN * 32 * T;  // the wave's first row of the tile
+    const int n = n0 + 32 * (w % WN) + fr, nc = min(n, sh.Cout - 1);
+    const int nu = min(n0 + 32 * (w % WN), sh.Cout - 1);  // the wave's first column
+    const int KK = sh.K * sh.K, ncs = (sh.Cin + kBK - 1) / kBK;
+
+    // fragment rows: the lane's row of each row tile, as its LDS offset or
+    // (kHalo) its place among the halo rows of tap 0, with the taps that lie
+    // inside the image as bits
+    const char* as_bytes = reinterpret_cast<const char*>(As);
+    int arow[T];
+    uint32_t inside[T];
 #pragma unroll
-    for (int u = 0; u < UT; ++u) bn[u] = 0.0f;
-    if constexpr (EPI == kEpiBias) {
-#pragma unroll
-        for (int u = 0; u < UT; ++u) bn[u] = bias[n0 + wn * (BN / 2) + 32 * u + fr];
-    }
-    if constexpr (EPI == kEpiGain) g = gain[0];
-    // Fragments of a k quarter (8 k: one 128-bit read per row tile) and the
-    // 16 MFMAs on them.  The next quarter's reads are issued before the
-    // current quarter's MFMAs (two fragment register sets; the scheduling
-    // barriers keep the compiler from sinking the reads below the MFMAs, which
-    // would leave the matrix core idle for the LDS latency of every quarter).
-    auto frag = [&](int buf, int kq, float4 (&a)[2], float4 (&b)[UT]) {
-        const int c = 2 * kq + fh;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) a[t] = As[buf][slot(wm * 64 + 32 * t + fr, c)];
-        if constexpr (WSRC == kWFwd) {
-            // component j of b[u] = B[k = 4 c + j][n]: rows 8 kq + 4 fh + j
-            const float* bs = reinterpret_cast<const float*>(&Bs[buf][0]);
-#pragma unroll
-            for (int u = 0; u < UT; ++u) {
-                const int n = wn * (BN / 2) + 32 * u + fr;
-                b[u].x = bs[kslot<BN>(4 * c + 0, n)];
-                b[u].y = bs[kslot<BN>(4 * c + 1, n)];
-                b[u].z = bs[kslot<BN>(4 * c + 2, n)];
-                b[u].w = bs[kslot<BN>(4 * c + 3, n)];
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < UT; ++u) b[u] = Bs[buf][slot(wn * (BN / 2) + 32 * u + fr, c)];
+    for (int t = 0; t < T; ++t) {
+        const int r = wrow + 32 * t + fr;
+        arow[t] = MODE == kHalo ? r : 16 * rowslot(r, fh);
+        if constexpr (MODE == kHalo) {
+            const int m = m0 + r;
+            uint32_t q, ow, b, oh, cols = 0;
+            sh.wo.divmod((uint32_t)min(m, sh.M - 1), q, ow);
+            sh.ho.divmod(q, b, oh);
+            for (int kw = 0; kw < sh.K; ++kw) cols |= (uint32_t)((unsigned)((int)ow + kw - sh.pad) < (unsigned)sh.W) << kw;
+            inside[t] = 0;
+            for (int kh = 0; kh < sh.K; ++kh)
+                if ((unsigned)((int)oh + kh - sh.pad) < (unsigned)sh.H) inside[t] |= cols << (kh * sh.K);
+            if (m >= sh.M) inside[t] = 0;
         }
-    };
-    auto mfmas = [&](const float4 (&a)[2], const float4 (&b)[UT]) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int u = 0; u < UT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t].x, b[u].x, acc[t][u], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int u = 0; u < UT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t].y, b[u].y, acc[t][u], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int u = 0; u < UT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t].z, b[u].z, acc[t][u], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int u = 0; u < UT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t].w, b[u].w, acc[t][u], 0, 0, 0);
-    };
-    auto compute = [&](int buf) {
-        float4 a0[2], b0[UT], a1[2], b1[UT];
-        frag(buf, 0, a0, b0);
-        frag(buf, 1, a1, b1);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(a0, b0);
-        __builtin_amdgcn_sched_barrier(0);
-        frag(buf, 2, a0, b0);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(a1, b1);
-        __builtin_amdgcn_sched_barrier(0);
-        frag(buf, 3, a1, b1);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(a0, b0);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(a1, b1);
-    };
-    // Slices: prologue, a branch-free steady loop over pairs of slices (slice
-    // kt computes from LDS buffer kt % 2 while R[kt % 2] receives slice kt + 2
-    // and R[(kt + 1) % 2] goes to the other buffer; the second load of a pair
-    // is clamped to the last slice, a harmless reload), then the one or two
-    // slices left.
-    load(0, R0);
-    if (nk > 1) load(1, R1);
-    store(0, R0);
-    __syncthreads();
-    int kt = 0;
-    for (; kt + 2 < nk; kt += 2) {
-        load(kt + 2, R0);
-        compute(0);
-        store(1, R1);
-        __syncthreads();
-        load(min(kt + 3, nk - 1), R1);
-        compute(1);
-        store(0, R0);
-        __syncthreads();
-    }
-    // Fused epilogue operands: all of a lane's are loaded at the start of the
-    // epilogue, one round trip (the main loop's registers are free by then).
-    // A row past M reads row M - 1 (harmless) and stores nothing.  Offsets are
-    // 32-bit (the launcher bounds the tensors below 2^31 elements).
-    const int mrow = m0 + wm * 64 + 4 * fh, ncol = n0 + wn * (BN / 2) + fr;
-    const int rowlim = sh.M - 1 - mrow;
-    const uint32_t lofs = (uint32_t)(mrow * sh.Cout + ncol);
-    float e1[UT][2][16], e2[UT][2][16];
-    auto fetch = [&](int u) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int d = min(32 * t + 8 * (r >> 2) + (r & 3), rowlim);
-                const uint32_t off = lofs + (uint32_t)(d * sh.Cout + 32 * u);
-                if constexpr ((XE & kXeRes) != 0) e1[u][t][r] = ep.res[off];
-                if constexpr ((XE & kXeActG) != 0) e2[u][t][r] = ep.xa[off];
-                if constexpr ((XE & kXeMod) != 0) {
-                    uint32_t bb, q;
-                    ep.hw.divmod((uint32_t)(mrow + d), bb, q);
-                    e2[u][t][r] = ep.cond[bb * (uint32_t)sh.Cout + (uint32_t)(ncol + 32 * u)];
-                }
-            }
-    };
-    compute(0);
-    if (kt + 1 < nk) {
-        store(1, R1);
-        __syncthreads();
-        compute(1);
     }
 
-    // epilogue: lanes 0-31 and 32-63 each write 32 consecutive outputs of a
-    // row.  A full row tile stores with no per-row test (a branch per store
-    // would make every store wait for all earlier ones).
-    auto out = [&](int t, int u, int r) {
-        float v = acc[t][u][r];
-        if constexpr (EPI == kEpiBias) v = v + bn[u];
-        if constexpr (EPI == kEpiGain) v = v * g;
-        return v;
-    };
-    float* yb = Y + (size_t)(m0 + wm * 64 + 4 * fh) * sh.Cout + n0 + wn * (BN / 2) + fr;
-    if constexpr (XE != kXeNone) {
-#pragma unroll
-        for (int u = 0; u < UT; ++u) fetch(u);
-#pragma unroll
-        for (int u = 0; u < UT; ++u) {
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int dm = 32 * t + 8 * (r >> 2) + (r & 3);
-                    if (mrow + dm >= sh.M) continue;
-                    float v = out(t, u, r);
-                    if constexpr ((XE & kXeActG) != 0) v = v * act_grad<ACT, false>(e2[u][t][r]);
-                    if constexpr ((XE & kXeRes) != 0) v = ep.wa * e1[u][t][r] + ep.wb * v;
-                    yb[(size_t)dm * sh.Cout + 32 * u] = v;
-                    if constexpr ((XE & kXeMod) != 0)
-                        ep.y2[(size_t)(mrow + dm) * sh.Cout + ncol + 32 * u] =
-                            act_fwd<ACT, false>(v * (e2[u][t][r] + 1.0f));
-                }
-        }
-    } else if (m0 + kBM <= sh.M) {
-#pragma unroll
-        for (int u = 0; u < UT; ++u)
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    yb[(size_t)(32 * t + 8 * (r >> 2) + (r & 3)) * sh.Cout + 32 * u] = out(t, u, r);
+    // activation loader: chunk ch (8 channels) of rows r0, r0 + 64, ...
+    const int ch = tid & 3, r0 = tid >> 2;
+    float v0[8], v1[8];  // kGather: the rows r0, r0 + 64 of the next tap
+    bool ok0 = false, ok1 = false;
+    int pix[2], ihb[2], iwb[2];
+    const int halo = kBM + 2 * sh.pad * (sh.W + 1);
+    if constexpr (MODE == kHalo) {
+        if (tid < kRowSlots) As[halo * kRowSlots + tid] = make_uint4(0, 0, 0, 0);
     } else {
 #pragma unroll
-        for (int u = 0; u < UT; ++u)
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int dm = 32 * t + 8 * (r >> 2) + (r & 3);
-                    if (m0 + wm * 64 + 4 * fh + dm < sh.M) yb[(size_t)dm * sh.Cout + 32 * u] = out(t, u, r);
-                }
+        for (int q = 0; q < 2; ++q) {
+            const int m = m0 + r0 + 64 * q;
+            uint32_t t, ow, b, oh;
+            sh.wo.divmod((uint32_t)(m < sh.M ? m : 0), t, ow);  // a row past the end computes row 0, stores nothing
+            sh.ho.divmod(t, b, oh);
+            pix[q] = (int)b * sh.H * sh.W;
+            ihb[q] = (int)oh * sh.stride - sh.pad;
+            iwb[q] = (int)ow * sh.stride - sh.pad;
+        }
     }
+    // 8 channels from c on of pixel p; channels past the end are left to the
+    // caller to zero (they read valid ones)
+    auto pixel8 = [&](float (&v)[8], int p, int c) {
+        const float* x = X + (size_t)p * sh.Cin;
+        if constexpr (MODE == kRagged) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = x[min(c + i, sh.Cin - 1)];
+        } else {
+            const float4 u = ld4(x + min(c, sh.Cin - 8)), z = ld4(x + min(c, sh.Cin - 8) + 4);
+            v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w, v[4] = z.x, v[5] = z.y, v[6] = z.z, v[7] = z.w;
+        }
+    };
+    // zeroed by masking the bits (a select of values would become a select of
+    // their addresses); channels past C_in too
+    auto put_row = [&](int row, float (&v)[8], bool ok, int c) {
+        if constexpr (MODE == kRagged) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = keep(v[i], ok && c + i < sh.Cin);
+        } else if constexpr (MODE == kGather) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = keep(v[i], ok && c < sh.Cin);
+        } else if (!ok) {  // kHalo: ok is uniform but in the last slice
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = 0.0f;
+        }
+        put8(As + rowslot(row, ch), 4, v);
+    };
+    auto gather = [&](int cs, int kh, int kw) {
+        const int c = cs * kBK + 8 * ch;
+        ok0 = ((unsigned)(ihb[0] + kh) < (unsigned)sh.H) & ((unsigned)(iwb[0] + kw) < (unsigned)sh.W);
+        ok1 = ((unsigned)(ihb[1] + kh) < (unsigned)sh.H) & ((unsigned)(iwb[1] + kw) < (unsigned)sh.W);
+        pixel8(v0, ok0 ? pix[0] + (ihb[0] + kh) * sh.W + iwb[0] + kw : 0, c);
+        pixel8(v1, ok1 ? pix[1] + (ihb[1] + kh) * sh.W + iwb[1] + kw : 0, c);
+    };
+    auto stage_halo = [&](int cs) {
+        const int c = cs * kBK + 8 * ch, base = m0 - sh.pad * (sh.W + 1);
+        constexpr int NB = 2;  // rows in flight
+        for (int r = r0; r < halo; r += 64 * NB) {
+            float v[NB][8];
+#pragma unroll
+            for (int q = 0; q < NB; ++q) pixel8(v[q], min(max(base + r + 64 * q, 0), sh.M - 1), c);
+#pragma unroll
+            for (int q = 0; q < NB; ++q)
+                if (r + 64 * q < halo) put_row(r + 64 * q, v[q], c < sh.Cin, c);
+        }
+    };
+
+    // weight loader: the lane's 8 k (8 fh .. + 7) of 16 at column nc, for the
+    // 16 channels c0 .. of a tap.  Channels past the end read valid ones: the
+    // activations are zero there.
+    float wv[2][8];
+    auto weights = [&](float (&v)[8], int tap, int c0) {
+        if constexpr (MODE == kRagged) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int c = min(c0 + 8 * fh + i, sh.Cin - 1);
+                v[i] = FLIP ? Wt[((size_t)(KK - 1 - tap) * sh.Cout + nc) * sh.Cin + c]
+                            : Wt[(size_t)(tap * sh.Cin + c) * sh.Cout + nc];
+            }
+        } else {
+            const int cu = min(c0, sh.Cin - 8);  // c0 may lie past the end
+            const int lh = cu + 16 > sh.Cin ? 0 : fh;
+            // a uniform base in scalar registers and a 32-bit lane offset (at
+            // most 31 rows of C_in, or 16 of C_out)
+            if constexpr (FLIP) {
+                const auto q = buffer(Wt + ((size_t)(KK - 1 - tap) * sh.Cout + nu) * sh.Cin + cu);
+                const int lo = 4 * ((nc - nu) * sh.Cin + 8 * lh);
+                const f32x4 u = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(q, lo, 0, 0));
+                const f32x4 z = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(q, lo, 16, 0));
+                v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w, v[4] = z.x, v[5] = z.y, v[6] = z.z, v[7] = z.w;
+            } else {
+                const auto q = buffer(Wt + (size_t)(tap * sh.Cin + cu) * sh.Cout + nu);
+                const int lo = 4 * (8 * lh * sh.Cout + nc - nu);
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    v[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(q, lo, 4 * i * sh.Cout, 0));
+            }
+        }
+    };
+
+    f32x16 acc[T][1], cor[T][1];
+#pragma unroll
+    for (int t = 0; t < T; ++t) acc[t][0] = cor[t][0] = (f32x16){};
+
+    // Steps of 16 k: (slice, tap, half).  A step's MFMAs read fragments that are
+    // in registers when it begins; between them it reads the next step's
+    // activation fragments into the registers of planes that are done with,
+    // splits the next step's weights and loads those of the step after.  The
+    // pattern (sched) keeps the compiler from drawing those to one side of the
+    // MFMAs: a wave by itself then leaves the matrix core few gaps, where two
+    // waves that take their vector work and their MFMAs in turns fall into step
+    // and leave it idle together.
+    uint4 a[kPlanes][T], b[2][kPlanes][1];
+    auto split_w = [&](int h) {
+        uint4 q[kPlanes];
+        split8(wv[h], q);
+#pragma unroll
+        for (int p = 0; p < kPlanes; ++p) b[h][p][0] = q[p];
+    };
+    auto rows_of = [&](int tap, int shift, int (&as)[T]) {  // byte offsets of the lane's fragment rows
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            as[t] = arow[t];
+            if constexpr (MODE == kHalo) {
+                // the row's slot where the tap is inside, else the zeros: a bit
+                // select, which stays free of branches
+                const int row = arow[t] + shift, in = -(int)((inside[t] >> tap) & 1);
+                as[t] = ((__mul24(row, 16 * kRowSlots) + 16 * swz(row, fh)) & in) | (halo * kRowSlots * 16 & ~in);
+            }
+        }
+    };
+    auto frag = [&](int p, const int (&as)[T], int ks) {
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+            a[p][t] = *reinterpret_cast<const uint4*>(as_bytes + (as[t] ^ 32 * ks) + 64 * p);
+    };
+    auto mul = [&](int i, int j, int h, f32x16 (&d)[T][1]) {
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+            d[t][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[i][t]),
+                __builtin_bit_cast(bf16x8, b[h][j][0]), d[t][0], 0, 0, 0);
+    };
+    // One step: half h of a tap, whose rows are `as`; (nas, h ^ 1) the next
+    // step's rows and half; (ntap, nc0) the tap and channels of the weights two
+    // steps on.  Planes 1 and 2 of the activations are in registers when the
+    // step begins, plane 0 is read during the first three products.
+    auto step = [&](int h, const int (&as)[T], const int (&nas)[T], int ntap, int nc0) {
+        frag(0, as, h);
+        mul(2, 0, h, cor);
+        split_w(h ^ 1);
+        mul(1, 1, h, cor);
+        mul(1, 0, h, cor);
+        sched<3 * T>();
+        __builtin_amdgcn_sched_barrier(0);
+        frag(2, nas, h ^ 1);
+        frag(1, nas, h ^ 1);
+        weights(wv[h ^ 1], ntap, nc0);  // into the registers just split
+        mul(0, 2, h, cor);
+        mul(0, 1, h, cor);
+        mul(0, 0, h, acc);
+        sched<3 * T>();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    weights(wv[0], 0, 0);
+    weights(wv[1], 0, 16);
+    if constexpr (MODE != kHalo) gather(0, 0, 0);
+    split_w(0);
+    weights(wv[0], KK > 1 ? 1 : 0, KK > 1 ? 0 : min(kBK, sh.Cin - 1));
+    int as[T];
+    for (int cs = 0; cs < ncs; ++cs) {
+        if constexpr (MODE == kHalo) {
+            if (cs) __syncthreads();  // the slice before has been read
+            stage_halo(cs);
+            __syncthreads();
+            rows_of(0, 0, as);
+            frag(2, as, 0);
+            frag(1, as, 0);
+        }
+        int kh = 0, kw = 0;  // of the tap after this one
+        for (int tap = 0; tap < KK; ++tap) {
+            const bool last = tap + 1 == KK;
+            const int t1 = last ? 0 : tap + 1, s1 = last ? cs + 1 : cs;        // the next tap
+            const int t2 = t1 + 1 == KK ? 0 : t1 + 1, s2 = t1 + 1 == KK ? s1 + 1 : s1;  // and the one after
+            if (++kw == sh.K) kw = 0, ++kh;
+            if (last) kh = 0;
+            if constexpr (MODE != kHalo) {
+                if (cs | tap) __syncthreads();  // the tap before has been read
+                const int c = cs * kBK + 8 * ch;
+                put_row(r0, v0, ok0, c);
+                put_row(r0 + 64, v1, ok1, c);
+                gather(min(s1, ncs - 1), kh, kw);  // the last one: a harmless reload, and no branch
+                __syncthreads();
+                rows_of(0, 0, as);
+                frag(2, as, 0);
+                frag(1, as, 0);
+            }
+            step(0, as, as, t1, s1 * kBK + 16);
+            int nas[T];
+            rows_of(t1, kh * sh.W + kw, nas);  // after the last tap: tap 0, read again once staged
+            step(1, as, nas, t2, s2 * kBK);
+#pragma unroll
+            for (int t = 0; t < T; ++t) as[t] = nas[t];
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t) acc[t][0] += cor[t][0];
+    if (split_failed<T, 1>(acc)) {
+        // straight from memory in fp32, 2 k per MFMA; rare, so simple
+#pragma unroll
+        for (int t = 0; t < T; ++t) acc[t][0] = (f32x16){};
+        for (int tap = 0; tap < KK; ++tap) {
+            const int kh = tap / sh.K, kw = tap - kh * sh.K;
+            const float* xp[T];
+            bool ok[T];
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                const int m = m0 + wrow + 32 * t + fr;
+                uint32_t q, ow, b, oh;
+                sh.wo.divmod((uint32_t)min(m, sh.M - 1), q, ow);
+                sh.ho.divmod(q, b, oh);
+                const int ih = (int)oh * sh.stride - sh.pad + kh, iw = (int)ow * sh.stride - sh.pad + kw;
+                ok[t] = (m < sh.M) & ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
+                xp[t] = X + (size_t)(ok[t] ? ((int)b * sh.H + ih) * sh.W + iw : 0) * sh.Cin;
+            }
+            for (int c0 = 0; c0 < sh.Cin; c0 += 2) {
+                const int c = min(c0 + fh, sh.Cin - 1);
+                const bool in = c0 + fh < sh.Cin;
+                const float wgt = FLIP ? Wt[((size_t)(KK - 1 - tap) * sh.Cout + nc) * sh.Cin + c]
+                                       : Wt[(size_t)(tap * sh.Cin + c) * sh.Cout + nc];
+#pragma unroll
+                for (int t = 0; t < T; ++t) {
+                    const float x = xp[t][c];
+                    acc[t][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(in && ok[t] ? x : 0.0f, in ? wgt : 0.0f, acc[t][0], 0, 0, 0);
+                }
+            }
+        }
+    }
+    // Epilogue: lanes 0-31 and 32-63 each write 32 consecutive outputs of a row
+    // 8 (r / 4) + 4 fh + r % 4.  The fused operands of a row tile are loaded
+    // together; a row past M reads row M - 1 (harmless) and stores nothing.  Offsets are 32-bit
+    // (the launcher bounds the tensors below 2^31 elements).
+    const int mrow = m0 + wrow + 4 * fh;
+    const bool mp = ep.mp != 0;
+    const float bn = ep.bias ? ep.bias[nc] : 0.0f, g = ep.gain ? ep.gain[0] : 1.0f;
+    auto off = [&](int t, int r) {
+        return (uint32_t)(min(mrow + 32 * t + 8 * (r >> 2) + (r & 3), sh.M - 1) * sh.Cout + nc);
+    };
+    const bool full = m0 + kBM <= sh.M && n0 + BN <= sh.Cout;  // stores with no test per row
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        float e1[16], e2[16];
+        if constexpr (XE != kXeNone) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if constexpr ((XE & kXeRes) != 0) e1[r] = ep.res[off(t, r)];
+                if constexpr ((XE & kXeActG) != 0) e2[r] = ep.xa[off(t, r)];
+                if constexpr ((XE & kXeMod) != 0) {
+                    uint32_t bb, q;
+                    ep.hw.divmod((uint32_t)min(mrow + 32 * t + 8 * (r >> 2) + (r & 3), sh.M - 1), bb, q);
+                    e2[r] = ep.cond[bb * (uint32_t)sh.Cout + (uint32_t)nc];
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            if (!full && (mrow + 32 * t + 8 * (r >> 2) + (r & 3) >= sh.M || n >= sh.Cout)) continue;
+            float v = acc[t][0][r];
+            if (ep.bias) v = v + bn;
+            else if (ep.gain) v = v * g;
+            if constexpr ((XE & kXeActG) != 0) {
+                const float d = act_grad<ACT_SILU, false>(e2[r]);
+                v = v * (mp ? d * kMpSiluScale : d);
+            }
+            if constexpr ((XE & kXeRes) != 0) v = ep.wa * e1[r] + ep.wb * v;
+            Y[off(t, r)] = v;
+            if constexpr ((XE & kXeMod) != 0) {
+                const float z = act_fwd<ACT_SILU, false>(v * (e2[r] + 1.0f));
+                ep.y2[off(t, r)] = mp ? z * kMpSiluScale : z;
+            }
+        }
+    }
+}
+
+// Host side.  Columns per workgroup, how the activations are staged, and the
+// launch.
+inline int conv_bn(int N) { return N > 64 ? 128 : N > 32 ? 64 : 32; }
+
+// Halo rows that leave room for two workgroups on a CU (160 KB of LDS), with
+// the taps' bits in 32.
+inline int conv_mode(const ConvShape& sh, const float* X, const float* Wt, bool flip) {
+    const bool vec = sh.Cin % 8 == 0 && aligned16(X) && (!flip || aligned16(Wt));
+    if (!vec) return kRagged;
+    const int halo = kBM + 2 * sh.pad * (sh.W + 1);
+    return sh.stride == 1 && sh.Ho == sh.H && sh.Wo == sh.W && sh.K <= 5 && (halo + 1) * kRowSlots * 16 <= 80000 ? kHalo
+                                                                                                             : kGather;
+}
+
+template <bool FLIP, int XE>
+void conv_launch(float* Y, const float* X, const float* Wt, const ConvShape& sh, const ConvEpi& ep, hipStream_t s) {
+    const int BN = conv_bn(sh.Cout), mode = conv_mode(sh, X, Wt, FLIP);
+    const unsigned grid = (unsigned)((sh.M + kBM - 1) / kBM) * (unsigned)((sh.Cout + BN - 1) / BN);
+    const int rows = mode == kHalo ? kBM + 2 * sh.pad * (sh.W + 1) + 1 : kBM;
+    const size_t lds = (size_t)rows * kRowSlots * sizeof(uint4);
+#define NNK_CONV(BN_, MODE_)                                                                                      \
+    do {                                                                                                          \
+        if (MODE_ == kHalo) {                                                                                     \
+            static const hipError_t once = hipFuncSetAttribute((const void*)conv_x3<BN_, MODE_, FLIP, XE>,         \
+                hipFuncAttributeMaxDynamicSharedMemorySize, 81920);                                               \
+            (void)once;                                                                                           \
+        }                                                                                                         \
+        conv_x3<BN_, MODE_, FLIP, XE><<<grid, kTpb, lds, s>>>(Y, X, Wt, sh, ep);                                  \
+    } while (0)
+#define NNK_CONV_MODE(MODE_)                 \
+    do {                                     \
+        if (BN == 128) NNK_CONV(128, MODE_); \
+        else if (BN == 64) NNK_CONV(64, MODE_); \
+        else NNK_CONV(32, MODE_);            \
+    } while (0)
+    if (mode == kHalo) NNK_CONV_MODE(kHalo);
+    else if (mode == kGather) NNK_CONV_MODE(kGather);
+    else if constexpr (XE == kXeNone) NNK_CONV_MODE(kRagged);
+#undef NNK_CONV_MODE
+#undef NNK_CONV
 }
 
 // ---------------------------------------------------------------------------
@@ -339,46 +577,21 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_fwd(float* __restrict__ Y, cons
 // tile to part[z], and a second launch adds the S partials in split order.
 //
 // Per stage a workgroup stages 32 pixel rows m of A (its 128 k columns) and
-// of dY (its BN n columns) in LDS transposed: per column, 8 float4 chunks of
-// 4 consecutive m (tslot).  A lane's MFMA operands then run along the pixel
-// reduction in one 128-bit read: in quad Q of the stage, lane l reads pixels
-// 8 Q + 4 (l / 32) .. + 3 of its column (k, or n, = l % 32 of a 32-column
-// block), and component c feeds the c-th MFMA, which pairs pixels 8 Q + c and
-// 8 Q + 4 + c of the two half-waves (any pairing gives the same sum, as long
-// as A and dY use the same one; this one is fixed).  Each loader thread
-// gathers 4 consecutive pixel rows of one 4-column chunk (one pixel decode,
-// then steps along the output row) and transposes them in registers into 4
-// chunk writes.
+// of dY (its BN n columns) in LDS transposed and split: per plane and column,
+// 32 consecutive m, so that a lane's MFMA operands run along the pixel
+// reduction (slice_mfma).  Each loader thread gathers 8 consecutive pixel rows
+// of 2 columns, and its registers hold them transposed.  The pixels of a wave
+// are the same in all lanes, so they are decoded in scalar registers.
 // ---------------------------------------------------------------------------
 constexpr int kWgM = 32;  // m rows per stage
-
-// float4 slot of (column, chunk of 4 m) in a [columns][8] transposed tile.
-// The xor with (col ^ col / 8) mod 8 puts the 16 columns that a 16-lane group
-// reads (consecutive columns, one chunk) on 16 distinct bank quads, and the
-// columns 4 ch + i that a loader instruction writes (ch = 16 consecutive
-// lanes) on at most two lanes per quad.
-__device__ __forceinline__ int tslot(int col, int mc) { return col * 8 + (mc ^ ((col ^ (col >> 3)) & 7)); }
-
-// XCD-aware tile order.  Workgroups are dispatched round-robin over the
-// device's 8 XCDs (workgroup L on XCD L % 8), each with its own L2.  Tile
-// L' = xcd_order(L) gives XCD x a contiguous range of tiles, so the k tiles
-// of one m split, which read the same X and dY rows, run in the same L2
-// instead of on different XCDs.  A bijection of [0, total) for any total.
-constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_order(int L, int total) {
-    const int x = L % kXcds, j = L / kXcds, q = total / kXcds, r = total % kXcds;
-    return x * q + min(x, r) + j;
-}
 
 template <int BN>
 __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part, const float* __restrict__ X,
     const float* __restrict__ dY, ConvShape sh, int rows_per_split) {
     constexpr int UT = BN / 64;               // 32-column accumulator tiles per wave
-    constexpr int DCH = BN / 4;               // float4 chunks per dY row
-    constexpr int DTHR = DCH * (kWgM / 4);    // dY loader threads: (n chunk, group of 4 rows)
-    static_assert(kWgM == 32 && DTHR <= kTpb && kTpb == 32 * (kWgM / 4), "loader roles");
-    __shared__ float4 As[2][128 * 8];
-    __shared__ float4 Ds[2][BN * 8];
+    constexpr int PA = 128 * kRow4, PD = BN * kRow4;  // uint4 per plane
+    __shared__ uint4 As[kPlanes * PA];
+    __shared__ uint4 Ds[kPlanes * PD];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int wk = w >> 1, wn = w & 1;
     // tile (k tile, n tile, split z), k tile fastest, in XCD-aware order
@@ -387,162 +600,128 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
     const int k0 = (tl % KT) * 128, n0 = ((tl / KT) % NT) * BN, z = tl / (KT * NT);
     const int mbeg = z * rows_per_split;
     const int mend = min(sh.M, mbeg + rows_per_split);
-    // loader roles: A chunk ch (k = k0 + 4 ch .. + 3) of the stage's pixel rows
-    // 4 g .. 4 g + 3; dY chunk dch (n = n0 + 4 dch .. + 3) of rows 4 dg .. + 3
-    const int ch = tid & 31, g = tid >> 5;
-    const int dch = tid % DCH, dg = tid / DCH;
-    const bool dld = tid < DTHR;
-    const int kc = k0 + 4 * ch;
-    const bool kok = kc < sh.KKC;
-    const int tap = kok ? kc / sh.Cin : 0, ci = kok ? kc - tap * sh.Cin : 0;
+    // loader roles: A columns k0 + 2 pc, + 1 of the stage's pixel rows 8 ws ..
+    // + 7 (ws the wave); dY columns n0 + 2 pn, + 1 of rows 8 dg .. + 7 (with
+    // BN = 64 the upper two waves store no dY)
+    const int ws = __builtin_amdgcn_readfirstlane(w);
+    const int pn = tid % (BN / 2), dg = (tid / (BN / 2)) & 3;
+    const bool dput = BN == 128 || tid < 2 * BN;
+    const int kcol = k0 + 2 * lane;
+    const int tap = kcol < sh.KKC ? kcol / sh.Cin : 0, ci = kcol < sh.KKC ? kcol - tap * sh.Cin : 0;
     const int kh = tap / sh.K, kw = tap - kh * sh.K;
-    const float* dcol = dY + n0 + 4 * dch;
-    const uint32_t Wo = (uint32_t)sh.Wo, Ho = (uint32_t)sh.Ho;
+    const float* xc = X + ci;
+    const float* dc = dY + n0 + 2 * pn;
 
-    // Two register sets: the stage two ahead is loaded while the next one is
-    // written to LDS, so a load has two stages of MFMA work to arrive.  Every
-    // lane loads (rows past the end, padding and the idle dY loaders of a
-    // 64-column tile read a valid address and are zeroed when stored): a
-    // branch around a load would make the compiler's later waits drain the
-    // whole vector-memory counter.
-    struct Regs {
-        float4 a[4], d[4];
-        bool aok[4], dok[4];
-    };
-    Regs R0, R1;
-    auto load = [&](int ms, Regs& R) {
-        // decode the first of the 4 rows once, then step along the output row
-        const int m0 = ms + 4 * g;
+    // Every lane loads (rows past the end, padding and columns past K*K*C_in
+    // read a valid address): a branch around a load would make the compiler's
+    // later waits drain the whole vector-memory counter.  A's rows past the end
+    // and padding are zeroed when stored.  The next stage's loads are issued
+    // before the current stage's MFMAs and split after them.
+    float2 va[8], vd[8];
+    bool aok[8];
+    auto load = [&](int ms) {
+        // decode the first of the 8 rows, then step along the output row
+        const int mf = ms + 8 * ws;
         uint32_t t, ow, b, oh;
-        sh.wo.divmod((uint32_t)(m0 < sh.M ? m0 : 0), t, ow);
+        sh.wo.divmod((uint32_t)(mf < sh.M ? mf : 0), t, ow);
         sh.ho.divmod(t, b, oh);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < 8; ++q) {
             const int ih = (int)oh * sh.stride - sh.pad + kh, iw = (int)ow * sh.stride - sh.pad + kw;
-            R.aok[q] = (m0 + q < mend) & kok & ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
-            const int p = R.aok[q] ? ((int)b * sh.H + ih) * sh.W + iw : 0;
-            // 32-bit element offsets (the host bounds x and dy below 2^31
-            // elements): same-box A/B 346.5 -> 343.7 us at cfg3 against 64-bit
-            // products; the forward's loader measured slower with the same change
-            R.a[q] = ld4(X + (uint32_t)(p * sh.Cin + ci));
-            if (++ow == Wo) {
+            aok[q] = (mf + q < mend) & ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
+            const int p = aok[q] ? ((int)b * sh.H + ih) * sh.W + iw : 0;
+            // 32-bit element offsets (the host bounds x and dy below 2^31 elements)
+            va[q] = *reinterpret_cast<const float2*>(xc + (uint32_t)(p * sh.Cin));
+            if (++ow == (uint32_t)sh.Wo) {
                 ow = 0;
-                if (++oh == Ho) {
+                if (++oh == (uint32_t)sh.Ho) {
                     oh = 0;
                     ++b;
                 }
             }
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int m = ms + 4 * dg + q;
-            R.dok[q] = dld & (m < mend);
-            R.d[q] = ld4(dcol + (uint32_t)((R.dok[q] ? m : 0) * sh.Cout));
-        }
+        for (int q = 0; q < 8; ++q)
+            vd[q] = *reinterpret_cast<const float2*>(dc + (uint32_t)(min(ms + 8 * dg + q, mend - 1) * sh.Cout));
     };
-    auto mask4 = [](float4 v, bool ok) {
-        const unsigned mk = ok ? 0xffffffffu : 0u;
-        v.x = __uint_as_float(__float_as_uint(v.x) & mk);
-        v.y = __uint_as_float(__float_as_uint(v.y) & mk);
-        v.z = __uint_as_float(__float_as_uint(v.z) & mk);
-        v.w = __uint_as_float(__float_as_uint(v.w) & mk);
-        return v;
-    };
-    // 4 rows x 4 columns in registers -> 4 column chunks (rows 4 gg .. + 3)
-    auto put = [&](float4* tile, int col0, int gg, const float4 (&v)[4], const bool (&ok)[4]) {
-        const float4 r0 = mask4(v[0], ok[0]), r1 = mask4(v[1], ok[1]), r2 = mask4(v[2], ok[2]),
-                     r3 = mask4(v[3], ok[3]);
-        tile[tslot(col0 + 0, gg)] = make_float4(r0.x, r1.x, r2.x, r3.x);
-        tile[tslot(col0 + 1, gg)] = make_float4(r0.y, r1.y, r2.y, r3.y);
-        tile[tslot(col0 + 2, gg)] = make_float4(r0.z, r1.z, r2.z, r3.z);
-        tile[tslot(col0 + 3, gg)] = make_float4(r0.w, r1.w, r2.w, r3.w);
-    };
-    auto store = [&](int buf, const Regs& R) {
-        put(As[buf], 4 * ch, g, R.a, R.aok);
-        if (dld) put(Ds[buf], 4 * dch, dg, R.d, R.dok);
-    };
-    f32x16 acc[2][UT];
+    f32x16 acc[2][UT], cor[2][UT];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int u = 0; u < UT; ++u) acc[t][u] = (f32x16){};
+        for (int u = 0; u < UT; ++u) acc[t][u] = cor[t][u] = (f32x16){};
     const int fr = lane & 31, fh = lane >> 5;
-    // Operands of quad Q (pixels 8 Q .. 8 Q + 7) and their MFMAs.  Two operand
-    // register sets: the reads of quad Q + 2 are issued right after the MFMAs
-    // of quad Q (the scheduling barriers keep them there), so each quad's
-    // reads have the next quad's 4 x 2 x UT MFMAs to arrive.
-    auto qfrag = [&](int buf, int Q, float4 (&a)[2], float4 (&d)[UT]) {
-        const int mc = 2 * Q + fh;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) a[t] = As[buf][tslot(wk * 64 + 32 * t + fr, mc)];
-#pragma unroll
-        for (int u = 0; u < UT; ++u) d[u] = Ds[buf][tslot(wn * (BN / 2) + 32 * u + fr, mc)];
-    };
-    // component-major: the 2 x UT accumulators in turn, so consecutive MFMAs
-    // never wait for each other's result
-    auto qmfma = [&](const float4 (&a)[2], const float4 (&d)[UT]) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int u = 0; u < UT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t].x, d[u].x, acc[t][u], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int u = 0; u < UT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t].y, d[u].y, acc[t][u], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int u = 0; u < UT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t].z, d[u].z, acc[t][u], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int u = 0; u < UT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t].w, d[u].w, acc[t][u], 0, 0, 0);
-    };
-    auto compute = [&](int buf) {
-        float4 a0[2], d0[UT], a1[2], d1[UT];
-        qfrag(buf, 0, a0, d0);
-        qfrag(buf, 1, a1, d1);
-        __builtin_amdgcn_sched_barrier(0);
-        qmfma(a0, d0);
-        __builtin_amdgcn_sched_barrier(0);
-        qfrag(buf, 2, a0, d0);
-        __builtin_amdgcn_sched_barrier(0);
-        qmfma(a1, d1);
-        __builtin_amdgcn_sched_barrier(0);
-        qfrag(buf, 3, a1, d1);
-        __builtin_amdgcn_sched_barrier(0);
-        qmfma(a0, d0);
-        __builtin_amdgcn_sched_barrier(0);
-        qmfma(a1, d1);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    // Stages: prologue, a branch-free steady loop over pairs of stages (stage
-    // st computes from LDS buffer st % 2 while R[st % 2] receives stage st + 2
-    // and R[(st + 1) % 2] goes to the other buffer; the second load of a pair
-    // is clamped to the last stage, a harmless reload), then the one or two
-    // stages left.
     const int nst = (mend - mbeg + kWgM - 1) / kWgM;
-    if (nst > 0) {
-        load(mbeg, R0);
-        if (nst > 1) load(mbeg + kWgM, R1);
-        store(0, R0);
-        __syncthreads();
-        int st = 0;
-        for (; st + 2 < nst; st += 2) {
-            load(mbeg + (st + 2) * kWgM, R0);
-            compute(0);
-            store(1, R1);
-            __syncthreads();
-            load(mbeg + min(st + 3, nst - 1) * kWgM, R1);
-            compute(1);
-            store(0, R0);
-            __syncthreads();
+    const int sa = slot(wk * 64 + fr, fh), sd = slot(wn * (BN / 2) + fr, fh);
+    if (nst > 0) load(mbeg);
+    for (int st = 0; st < nst; ++st) {
+        if (st) __syncthreads();  // the stage before has been read
+        put8(As + slot(2 * lane, ws), PA, {keep(va[0].x, aok[0]), keep(va[1].x, aok[1]), keep(va[2].x, aok[2]),
+                                       keep(va[3].x, aok[3]), keep(va[4].x, aok[4]), keep(va[5].x, aok[5]),
+                                       keep(va[6].x, aok[6]), keep(va[7].x, aok[7])});
+        put8(As + slot(2 * lane + 1, ws), PA, {keep(va[0].y, aok[0]), keep(va[1].y, aok[1]), keep(va[2].y, aok[2]),
+                                           keep(va[3].y, aok[3]), keep(va[4].y, aok[4]), keep(va[5].y, aok[5]),
+                                           keep(va[6].y, aok[6]), keep(va[7].y, aok[7])});
+        if (dput) {
+            put8(Ds + slot(2 * pn, dg), PD, {vd[0].x, vd[1].x, vd[2].x, vd[3].x, vd[4].x, vd[5].x, vd[6].x, vd[7].x});
+            put8(Ds + slot(2 * pn + 1, dg), PD, {vd[0].y, vd[1].y, vd[2].y, vd[3].y, vd[4].y, vd[5].y, vd[6].y, vd[7].y});
         }
-        compute(0);
-        if (st + 1 < nst) {
-            store(1, R1);
-            __syncthreads();
-            compute(1);
+        load(mbeg + min(st + 1, nst - 1) * kWgM);  // the last one again: harmless, and no branch
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            uint4 a[kPlanes][2], d[kPlanes][UT];
+#pragma unroll
+            for (int p = 0; p < kPlanes; ++p) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) a[p][t] = As[p * PA + 32 * t * kRow4 + (sa ^ 2 * ks)];
+#pragma unroll
+                for (int u = 0; u < UT; ++u) d[p][u] = Ds[p * PD + 32 * u * kRow4 + (sd ^ 2 * ks)];
+            }
+            products<2, UT>(a, d, acc, cor);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int u = 0; u < UT; ++u) acc[t][u] += cor[t][u];
+    if (split_failed<2, UT>(acc)) {
+        // straight from memory in fp32, 2 pixels per MFMA; rare, so simple
+        int tp[2], cc[2];
+        bool ck[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int k = k0 + wk * 64 + 32 * t + fr;
+            ck[t] = k < sh.KKC;
+            tp[t] = ck[t] ? k / sh.Cin : 0;
+            cc[t] = ck[t] ? k - tp[t] * sh.Cin : 0;
+#pragma unroll
+            for (int u = 0; u < UT; ++u) acc[t][u] = (f32x16){};
+        }
+        for (int ms = mbeg; ms < mend; ms += 2) {
+            const int m = ms + fh;
+            const bool in = m < mend;
+            uint32_t q, ow, b, oh;
+            sh.wo.divmod((uint32_t)(in ? m : mbeg), q, ow);
+            sh.ho.divmod(q, b, oh);
+            float av[2], dv[UT];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int th = tp[t] / sh.K, tw = tp[t] - th * sh.K;
+                const int ih = (int)oh * sh.stride - sh.pad + th, iw = (int)ow * sh.stride - sh.pad + tw;
+                const bool ok = in & ck[t] & ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
+                const float v = X[(size_t)(ok ? ((int)b * sh.H + ih) * sh.W + iw : 0) * sh.Cin + cc[t]];
+                av[t] = ok ? v : 0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < UT; ++u) {
+                const float v = dY[(size_t)(in ? m : mbeg) * sh.Cout + n0 + wn * (BN / 2) + 32 * u + fr];
+                dv[u] = in ? v : 0.0f;
+            }
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int u = 0; u < UT; ++u)
+                    acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[t], dv[u], acc[t][u], 0, 0, 0);
         }
     }
     // partial tile: D[k][n], rows k = k0 + wk 64 + 32 t + 8 (r / 4) + 4 h + r % 4

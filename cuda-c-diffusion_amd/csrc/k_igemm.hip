@@ -1,45 +1,41 @@
-// k_igemm.hip -- NHWC convolution forward as an implicit GEMM on the fp32
-// matrix cores (v_mfma_f32_32x32x2f32), replacing im2col + GEMM + bias/gain
-// pass of the reference's conv2d forward (src/conv2d.c:17-34: launch_im2col,
-// gemm_forward, launch_add_bias or launch_scale_by_scalar), and the stride-1
-// input gradient as the same kernel over dy with the kernel flipped
-// (replacing gemm_dX + col2im, src/conv2d.c:48-65).
+// k_igemm.hip -- NHWC convolution forward as an implicit GEMM on the matrix
+// cores, replacing im2col + GEMM + bias/gain pass of the reference's conv2d
+// forward (src/conv2d.c:17-34: launch_im2col, gemm_forward, launch_add_bias or
+// launch_scale_by_scalar), the stride-1 input gradient as the same kernel over
+// dy with the kernel flipped (replacing gemm_dX + col2im, src/conv2d.c:48-65),
+// and the weight gradient (src/conv2d.c:44-47).
 //
 //   Y[m, n] = sum_k A[m, k] Wt[k, n]  (+ bias[n] | * gain[0])
 //   m = (b, oh, ow), k = (kh, kw, ci), A[m, k] = X[b, oh s + kh - p, ow s + kw - p, ci]
 //   (0 outside the image), Wt = the reference's [K*K*C_in, C_out] weight.
 //
-// The im2col matrix is never written: each workgroup gathers its A tile from X
-// directly (a k-slice of 32 channels of one (kh, kw) is 128 contiguous bytes
-// of one input pixel).  The weight is read in the reference's layout too, with
-// no transposed or flipped copy: the forward stages its [32 k][BN n] slice as
-// it lies in Wt and reads the B operand 32 bits at a time; the input
-// gradient's operand B[ci][(kh, kw, co)] = Wt[((K-1-kh) K + (K-1-kw)) C_in +
-// ci][co] is k-contiguous and is staged like A.
+// The im2col matrix is never written and the weight is read in the reference's
+// layout, with no transposed, flipped or converted copy in memory.
 //
-// Workgroup tile 128 (m) x BN (n, 128 or 64), k in slices of 32; 4 waves of
-// 64 x BN/2, each a 2 x BN/64 grid of 32 x 32 MFMA accumulators.  Per slice a
-// thread loads 4 float4 of A and up to 4 of the weight into registers, the
-// slice before it computes from LDS, then the registers go to the other LDS
-// buffer (two buffers of 2 x 16 KB; two workgroups fit a CU).  A tiles (and
-// the input gradient's B) are [128 rows][8 float4 chunks of 4 k] with the
-// chunk index xor-swizzled by the row (slot()), so the 128-bit fragment reads
-// of a wave (32 rows, one chunk per half-wave) and the tile writes are free of
-// bank conflicts.  The forward's B tile is [32 k][BN n], each row rotated by
-// 32 n on alternate groups of 4 rows (kslot()), so the two half-waves of a
-// 32-bit fragment read (rows k and k + 4, 32 consecutive n each) use
-// disjoint banks.
+// fp32 products on the bf16 matrix cores.  v_mfma_f32_32x32x2f32 holds 134
+// TFLOP/s here, v_mfma_f32_32x32x16_bf16 1780 (register-only loops, 512
+// workgroups): 13 times.  Each fp32 operand is split exactly into three bf16
+// planes and six of the nine plane products are formed (igemm.h), 297 TFLOP/s
+// of fp32 products at most.  With data from memory a large bf16 product of the
+// vendor library holds 1250 TFLOP/s, because the clock falls to 1.7 GHz under
+// that load, so 208 is what to expect.  Measured: cfg3 forward (3x3, 128 -> 128,
+// [128, 32, 32]) 320 -> 191 us (202 TFLOP/s), 256 -> 256 at [16, 64, 64] 627 ->
+// 351 us (220), their input gradients 317 -> 193 and 620 -> 359 us; the matrix
+// cores are busy 0.69 of the time at 1.67 GHz.  On the way: the fp32 kernel's
+// staging (both operands through LDS per tap, a split of each) 230-260 us;
+// activations staged once per 32 channels for all taps, weights split in
+// registers by the one wave that needs them 205-214; the next step's loads and
+// splits between the MFMAs 191.  Error against 64 bits: below the fp32 MFMA's
+// at every size measured (igemm.h).
 //
-// Lane layout of v_mfma_f32_32x32x2f32 (checked on the device): lane l supplies
-// A[l % 32][l / 32] and B[l / 32][l % 32]; accumulator register r of lane l
-// holds D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].  A 128-bit fragment read
-// gives a lane 4 consecutive k of its row; component c feeds the c-th MFMA,
-// which pairs k = 4h + c of the two half-waves h: any pairing of k is the same
-// sum, as long as A and B use the same one.
+// Lane layout of v_mfma_f32_32x32x16_bf16 (checked on the device): lane l
+// supplies A[l % 32][8 (l / 32) .. + 7] and B[8 (l / 32) .. + 7][l % 32];
+// accumulator register r of lane l holds D[8 (r / 4) + 4 (l / 32) + r % 4][l %
+// 32].
 //
-// Summation order: each output is a fixed-order fp32 sum (per slice, pairs of
-// k in MFMA order, slices in k order); it differs from a library GEMM's order
-// by rounding only, and is the same on every run.
+// Summation order: each output is a fixed-order sum (slices of 32 channels,
+// taps, halves of 16), the same on every run and in both staging forms; it
+// differs from a library GEMM's order by rounding only.
 #include "igemm.h"
 
 extern "C" {
@@ -55,18 +51,10 @@ void launch_conv2d_forward_implicit(float* Y, const float* X, const float* Wt, c
     ConvShape sh;
     if (fwd_setup(what, Y, X, Wt, bias, gain, batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, sh) <= 0)
         return;
-    const int BN = tile_n(C_out);
-    const dim3 grid((unsigned)((sh.M + kBM - 1) / kBM), (unsigned)(C_out / BN));
-#define NNK_IGEMM_FWD(BN_)                                                                               \
-    if (bias) igemm_fwd<kEpiBias, BN_, kWFwd><<<grid, kTpb, 0, s>>>(Y, X, Wt, bias, nullptr, sh, ConvEpi{});       \
-    else if (gain) igemm_fwd<kEpiGain, BN_, kWFwd><<<grid, kTpb, 0, s>>>(Y, X, Wt, nullptr, gain, sh, ConvEpi{});  \
-    else igemm_fwd<kEpiNone, BN_, kWFwd><<<grid, kTpb, 0, s>>>(Y, X, Wt, nullptr, nullptr, sh, ConvEpi{});
-    if (BN == 128) {
-        NNK_IGEMM_FWD(128)
-    } else {
-        NNK_IGEMM_FWD(64)
-    }
-#undef NNK_IGEMM_FWD
+    ConvEpi ep{};
+    ep.bias = bias;
+    ep.gain = gain;
+    conv_launch<false, kXeNone>(Y, X, Wt, sh, ep, s);
     nnk_after_launch(what, s);
 }
 
@@ -79,17 +67,9 @@ void launch_conv2d_input_grad_implicit(float* dX, const float* dY, const float* 
     const char* what = "launch_conv2d_input_grad_implicit";
     ConvShape sh;
     if (dgrad_setup(what, dX, dY, Wt, batch, H, W, C_in, C_out, K, pad, sh) <= 0) return;
-    const int BN = tile_n(C_in);
-    const dim3 grid((unsigned)((sh.M + kBM - 1) / kBM), (unsigned)(C_in / BN));
-#define NNK_IGEMM_DGRAD(BN_)                                                                                  \
-    if (gain) igemm_fwd<kEpiGain, BN_, kWFlip><<<grid, kTpb, 0, s>>>(dX, dY, Wt, nullptr, gain, sh, ConvEpi{});           \
-    else igemm_fwd<kEpiNone, BN_, kWFlip><<<grid, kTpb, 0, s>>>(dX, dY, Wt, nullptr, nullptr, sh, ConvEpi{});
-    if (BN == 128) {
-        NNK_IGEMM_DGRAD(128)
-    } else {
-        NNK_IGEMM_DGRAD(64)
-    }
-#undef NNK_IGEMM_DGRAD
+    ConvEpi ep{};
+    ep.gain = gain;
+    conv_launch<true, kXeNone>(dX, dY, Wt, sh, ep, s);
     nnk_after_launch(what, s);
 }
 

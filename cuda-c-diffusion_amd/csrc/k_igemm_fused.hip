@@ -44,24 +44,11 @@ void launch_conv2d_forward_implicit_fused(float* Y, const float* X, const float*
     ep.cond = f->cond;
     ep.y2 = f->y2;
     ep.hw = FastDiv((uint32_t)(H_out * W_out));
-    const int BN = tile_n(C_out);
-    const dim3 grid((unsigned)((sh.M + kBM - 1) / kBM), (unsigned)(C_out / BN));
-#define NNK_FWD_EPI(XE_, ACT_, BN_)                                                                             \
-    do {                                                                                                        \
-        if (bias) igemm_fwd<kEpiBias, BN_, kWFwd, XE_, ACT_><<<grid, kTpb, 0, s>>>(Y, X, Wt, bias, nullptr, sh, ep); \
-        else if (gain) igemm_fwd<kEpiGain, BN_, kWFwd, XE_, ACT_><<<grid, kTpb, 0, s>>>(Y, X, Wt, nullptr, gain, sh, ep); \
-        else igemm_fwd<kEpiNone, BN_, kWFwd, XE_, ACT_><<<grid, kTpb, 0, s>>>(Y, X, Wt, nullptr, nullptr, sh, ep); \
-    } while (0)
-#define NNK_FWD_BN(XE_, ACT_)                 \
-    do {                                      \
-        if (BN == 128) NNK_FWD_EPI(XE_, ACT_, 128); \
-        else NNK_FWD_EPI(XE_, ACT_, 64);      \
-    } while (0)
-    if (f->res) NNK_FWD_BN(kXeRes, 0);
-    else if (f->act == ACT_SILU) NNK_FWD_BN(kXeMod, ACT_SILU);
-    else NNK_FWD_BN(kXeMod, ACT_MP_SILU);
-#undef NNK_FWD_BN
-#undef NNK_FWD_EPI
+    ep.bias = bias;
+    ep.gain = gain;
+    ep.mp = f->act == ACT_MP_SILU;
+    if (f->res) conv_launch<false, kXeRes>(Y, X, Wt, sh, ep, s);
+    else conv_launch<false, kXeMod>(Y, X, Wt, sh, ep, s);
     nnk_after_launch(what, s);
 }
 
@@ -80,22 +67,9 @@ void launch_conv2d_input_grad_implicit_fused(float* dX, const float* dY, const f
     ep.xa = f->act_in;
     ep.wa = f->res_w;
     ep.wb = f->out_w;
-    const int BN = tile_n(C_in);
-    const dim3 grid((unsigned)((sh.M + kBM - 1) / kBM), (unsigned)(C_in / BN));
-#define NNK_DGRAD_EPI(ACT_, BN_)                                                                                 \
-    do {                                                                                                         \
-        if (gain) igemm_fwd<kEpiGain, BN_, kWFlip, kXeActG | kXeRes, ACT_><<<grid, kTpb, 0, s>>>(dX, dY, Wt, nullptr, gain, sh, ep); \
-        else igemm_fwd<kEpiNone, BN_, kWFlip, kXeActG | kXeRes, ACT_><<<grid, kTpb, 0, s>>>(dX, dY, Wt, nullptr, nullptr, sh, ep); \
-    } while (0)
-#define NNK_DGRAD_BN(ACT_)                 \
-    do {                                   \
-        if (BN == 128) NNK_DGRAD_EPI(ACT_, 128); \
-        else NNK_DGRAD_EPI(ACT_, 64);      \
-    } while (0)
-    if (f->act == ACT_SILU) NNK_DGRAD_BN(ACT_SILU);
-    else NNK_DGRAD_BN(ACT_MP_SILU);
-#undef NNK_DGRAD_BN
-#undef NNK_DGRAD_EPI
+    ep.gain = gain;
+    ep.mp = f->act == ACT_MP_SILU;
+    conv_launch<true, kXeActG | kXeRes>(dX, dY, Wt, sh, ep, s);
     nnk_after_launch(what, s);
 }
 

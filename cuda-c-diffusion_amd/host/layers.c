@@ -365,18 +365,18 @@ static int conv_implicit_forced(void)
 
 /* Whether the implicit-GEMM kernel (igemm_fwd: the forward, and the stride-1
    input gradient) beats im2col + rocBLAS for an M x N x K product, by a cost
-   model fitted on MI355X.  A 128 x BN output tile takes ~2.25 us per 32-deep k
+   model fitted on MI355X.  A 128 x BN output tile takes ~1.33 us per 32-deep k
    slice with one workgroup per CU (cfg3's forward: 36 slices, 1024 tiles,
-   four tiles per CU: 320 us), so few tiles leave the device idle: at the
+   four tiles per CU: 191 us), so few tiles leave the device idle: at the
    reference DDPM's 7 x 7 x 128 level (M = 392 at batch 8, 4 tiles) the kernel
-   takes ~83 us where the GEMM path takes ~10.  The GEMM path: ~10 us of fixed
+   takes ~48 us where the GEMM path takes ~20.  The GEMM path: ~10 us of fixed
    cost, the GEMM at ~70 TFLOP/s (rocBLAS fp32, measured at cfg3) and the
    im2col matrix written and read at ~6 TB/s. */
 static int conv_implicit_wins(long long M, int N, int K)
 {
     const int bn = N % 128 == 0 ? 128 : 64;
     const double tiles = (double)((M + 127) / 128) * ((N + bn - 1) / bn);
-    const double t_impl = (K / 32.0) * 2.25 * ceil(tiles / 256.0);
+    const double t_impl = (K / 32.0) * 1.33 * ceil(tiles / 256.0);
     const double t_gemm = 10.0 + 2.0 * (double)M * N * K / 70e6 + 8.0 * (double)M * K / 6e6;
     return t_impl <= t_gemm;
 }
