@@ -243,3 +243,11 @@ bool nnk_gn_fwd_reg_dispatch(int cfg, int v4pp, int act, float* y, float* mu, fl
 bool nnk_gn_bwd_reg_dispatch(int cfg, int v4pp, int act, float* dx, float* part_g, float* part_b,
     const float* dy, const float* x, const float* gamma, const float* beta,
     const float* mu, const float* rstd, int B, int G, int HW, int C, hipStream_t s);
+
+// Any cpg up to 1024 and any alignment (k_gn_slab.hip); the partials as above.
+bool nnk_gn_slab_takes(int HW, int C, int G);
+void nnk_gn_fwd_slab(int act, float* y, float* mu, float* rstd, const float* x, const float* gamma, const float* beta,
+    int B, int G, int HW, int C, float eps, hipStream_t s);
+void nnk_gn_bwd_slab(int act, float* dx, float* part_g, float* part_b, const float* dy, const float* x,
+    const float* gamma, const float* beta, const float* mu, const float* rstd, int B, int G, int HW, int C,
+    hipStream_t s);
