@@ -3,12 +3,18 @@
 // Reference maths: src/kernels.cu:255-297 with launchers 330-344.
 //
 // W is [in, out] row-major and every output column j is normalised over its
-// `in` rows.  One 1024-thread workgroup owns kCols = 16 whole columns: a wave
-// instruction covers 4 rows x 16 columns (64-byte row segments), lane (r, c)
-// walks rows 4 w + r, + 64, ... of column 16 b + c with eight rows' loads in
-// flight; its partial, the 4 row lanes of the wave and then the 16 waves are
-// added in a fixed order.  Each column total therefore has a fixed order and
-// needs no scratch or second pass; a [1152, 128] weight spreads over 8 CUs.
+// `in` rows.  One 1024-thread workgroup owns COLS whole columns: a wave
+// instruction covers 64 / COLS rows, lane (r, c) walks rows of column COLS b + c
+// and keeps up to kKeep of them in registers, all loaded at once; its partial,
+// the row lanes of the wave and then the 16 waves are added in a fixed order.
+// Each column total therefore has a fixed order and needs no scratch or second
+// pass.  The work is one round trip of loads and one of stores, so what counts
+// is how many CUs share it and that no round follows another: COLS = 4 puts
+// [1152, 128] on 32 CUs with 5 rows a lane and [4032, 448] on 112 with 16 (rows
+// longer than kKeep steps are read again from cache, in batches).  Neighbouring
+// blocks share 128-byte lines, so they run on one XCD.  Against 16 columns a
+// workgroup and 8 rows at a time: forward 20.1 -> 12.2 us and backward 37.0 ->
+// 19.6 at [4032, 448], 6.7 -> 5.2 and 11.3 -> 8.4 at [1152, 128].
 //   forward : column sum of squares, then W *= rsqrt(sum + eps)    (one launch;
 //             the second read of W comes from cache)
 //   backward: dot_j = <Wn_j, gW_j>, then gW = gain * (gW - dot_j Wn) (one
@@ -24,37 +30,31 @@ using namespace nnk;
 
 constexpr int kTpb = 1024;
 constexpr int kNw = kTpb / kWave;
-constexpr int kCols = 16;              // columns per workgroup
+constexpr int kCols = 4;               // columns per workgroup
 constexpr int kRowsPerWave = kWave / kCols;
 constexpr int kRowStep = kNw * kRowsPerWave;
-constexpr int kBatch = 8;
+constexpr int kKeep = 16;              // rows a lane keeps in registers
+constexpr int kMore = 8;               // rows in flight beyond those
 
-// Total of A .* B over all rows of this lane's column (identical on the
-// kRowsPerWave lanes of the column in every wave).  `l` is [kNw][kCols].
-__device__ __forceinline__ float column_dot(const float* __restrict__ A, const float* __restrict__ B,
-    int in, int out, float (*l)[kCols]) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wid = threadIdx.x / kWave;
-    const int c = lane % kCols, r = lane / kCols;
-    const int j = blockIdx.x * kCols + c;
-    float s = 0.0f;
-    if (j < out) {
-        int i = wid * kRowsPerWave + r;
-        for (; i + (kBatch - 1) * kRowStep < in; i += kBatch * kRowStep) {
-            float a[kBatch], b[kBatch];
+// Rows i0 + u kRowStep of this lane's column, 0 past the end.
+template <int N>
+__device__ __forceinline__ void column_rows(float (&v)[N], const float* __restrict__ A, int i0, int in, int out,
+    int j) {
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                a[u] = A[(size_t)(i + u * kRowStep) * out + j];
-                b[u] = B[(size_t)(i + u * kRowStep) * out + j];
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) s += a[u] * b[u];
-        }
-        for (; i < in; i += kRowStep) s += A[(size_t)i * out + j] * B[(size_t)i * out + j];
+    for (int u = 0; u < N; ++u) {
+        const int i = i0 + u * kRowStep;
+        v[u] = i < in ? A[(size_t)i * out + j] : 0.0f;
     }
+}
+
+// Total of the lanes' s over the column (identical on all its lanes, in every
+// wave).  `l` is [kNw][kCols].
+__device__ __forceinline__ float column_total(float s, float (*l)[kCols]) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int c = lane % kCols;
 #pragma unroll
     for (int o = kCols; o < kWave; o <<= 1) s += __shfl_xor(s, o, kWave);
-    if (r == 0) l[wid][c] = s;
+    if (lane < kCols) l[threadIdx.x / kWave][c] = s;
     __syncthreads();
     float t = l[0][c];
 #pragma unroll
@@ -64,15 +64,31 @@ __device__ __forceinline__ float column_dot(const float* __restrict__ A, const f
 
 __global__ __launch_bounds__(kTpb) void wn_forward(float* __restrict__ W, int in, int out, float eps) {
     __shared__ float l[kNw][kCols];
+    const int bid = xcd_swizzle(blockIdx.x, gridDim.x);
     const int lane = threadIdx.x & (kWave - 1);
-    const int wid = threadIdx.x / kWave;
-    const int j = blockIdx.x * kCols + lane % kCols;
-    const float inv = rsqrtf(column_dot(W, W, in, out, l) + eps);
+    const int i0 = threadIdx.x / kWave * kRowsPerWave + lane / kCols;
+    const int j = bid * kCols + lane % kCols, jc = min(j, out - 1);
+    float v[kKeep], s = 0.0f;
+    column_rows(v, W, i0, in, out, jc);
+#pragma unroll
+    for (int u = 0; u < kKeep; ++u) s += v[u] * v[u];
+    for (int i = i0 + kKeep * kRowStep; i < in; i += kMore * kRowStep) {
+        float x[kMore];
+        column_rows(x, W, i, in, out, jc);
+#pragma unroll
+        for (int u = 0; u < kMore; ++u) s += x[u] * x[u];
+    }
+    const float inv = rsqrtf(column_total(s, l) + eps);
     if (j >= out) return;
-    for (int i = wid * kRowsPerWave + lane / kCols; i < in; i += kRowStep) W[(size_t)i * out + j] *= inv;
+#pragma unroll
+    for (int u = 0; u < kKeep; ++u) {
+        const int i = i0 + u * kRowStep;
+        if (i < in) W[(size_t)i * out + j] = v[u] * inv;
+    }
+    for (int i = i0 + kKeep * kRowStep; i < in; i += kRowStep) W[(size_t)i * out + j] *= inv;
 }
 
-// gW = gain * (gW - dot_j * Wn); part[blockIdx.x] = sum of this block's dot_j.
+// gW = gain * (gW - dot_j * Wn); part[b] = sum of block b's dot_j.
 // LAST: the last workgroup to arrive (counter) adds part[0..gridDim.x) to
 // *g_gain in index order and re-arms the counter.
 template <bool LAST>
@@ -81,14 +97,29 @@ __global__ __launch_bounds__(kTpb) void wn_backward(float* __restrict__ gW, cons
     float* __restrict__ g_gain, int in, int out) {
     __shared__ float l[kNw][kCols];
     __shared__ int last;
+    const int bid = xcd_swizzle(blockIdx.x, gridDim.x);
     const int lane = threadIdx.x & (kWave - 1);
     const int wid = threadIdx.x / kWave;
-    const int j = blockIdx.x * kCols + lane % kCols;
-    const float dot = column_dot(Wn, gW, in, out, l);  // its barrier orders every read of gW before the writes below
+    const int i0 = wid * kRowsPerWave + lane / kCols;
+    const int j = bid * kCols + lane % kCols, jc = min(j, out - 1);
+    float a[kKeep], b[kKeep], s = 0.0f;
+    column_rows(a, gW, i0, in, out, jc);
+    column_rows(b, Wn, i0, in, out, jc);
+    const float g = gain[0];
+#pragma unroll
+    for (int u = 0; u < kKeep; ++u) s += b[u] * a[u];
+    for (int i = i0 + kKeep * kRowStep; i < in; i += kMore * kRowStep) {
+        float x[kMore], y[kMore];
+        column_rows(x, gW, i, in, out, jc);
+        column_rows(y, Wn, i, in, out, jc);
+#pragma unroll
+        for (int u = 0; u < kMore; ++u) s += y[u] * x[u];
+    }
+    const float dot = column_total(s, l);  // its barrier orders every read of gW before the writes below
     if (wid == 0) {
-        // lanes 0..kCols-1 hold the block's column totals (r == 0 lanes)
+        // lanes 0..kCols-1 hold the block's column totals
         const float t = wave_sum(lane < kCols && j < out ? dot : 0.0f);
-        if (lane == 0) part[blockIdx.x] = t;
+        if (lane == 0) part[bid] = t;
     }
     if constexpr (LAST) {
         __syncthreads();
@@ -108,11 +139,16 @@ __global__ __launch_bounds__(kTpb) void wn_backward(float* __restrict__ gW, cons
             }
         }
     }
-    if (j >= out) return;
-    const float g = gain[0];
-    for (int i = wid * kRowsPerWave + lane / kCols; i < in; i += kRowStep) {
-        const size_t o = (size_t)i * out + j;
-        gW[o] = g * (gW[o] - dot * Wn[o]);
+    if (j < out) {
+#pragma unroll
+        for (int u = 0; u < kKeep; ++u) {
+            const int i = i0 + u * kRowStep;
+            if (i < in) gW[(size_t)i * out + j] = g * (a[u] - dot * b[u]);
+        }
+        for (int i = i0 + kKeep * kRowStep; i < in; i += kRowStep) {
+            const size_t o = (size_t)i * out + j;
+            gW[o] = g * (gW[o] - dot * Wn[o]);
+        }
     }
 }
 
