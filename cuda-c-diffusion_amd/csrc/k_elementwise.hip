@@ -210,37 +210,51 @@ __global__ __launch_bounds__(kTpb) void add_bias_vec_kernel(float* __restrict__ 
 }
 
 // ---------------- bias_grad: gb[n] = sum_r g[r,n] ----------------
-// Stage 1: grid (ceil(N/64), chunks); lanes walk 64 consecutive columns
-// (coalesced), 4 waves split the chunk's rows.  part[chunk*N + n].
-constexpr int kBgRows = 256;
-__global__ __launch_bounds__(kTpb) void bias_grad_partial(float* __restrict__ part,
-    const float* __restrict__ g, int rows, int N) {
-    __shared__ float l[4][kWave];
+// 64 columns a workgroup (coalesced rows of 256 bytes), 16 waves; a wave sums
+// every 16th row with eight rows' loads in flight, the waves' sums are added in
+// order.  Grid (ceil(N / 64), chunks of rows): the sum of a chunk goes to
+// out[chunk * N + n], and the same kernel adds the chunks, whose sums are rows
+// themselves.  Up to kBgDirect rows one launch does all: more rows in one
+// workgroup take longer than the second launch.  At [65536, 256] 22 us against
+// 77 with chunks of 256 rows whose sums one thread a column added one by one,
+// at [128, 256] 3 against 6 us in two launches.
+constexpr int kBgTpb = 1024;
+constexpr int kBgWaves = kBgTpb / kWave;
+constexpr int kBgBatch = 8;
+constexpr int kBgDirect = 4 * kBgWaves * kBgBatch;
+constexpr int kBgBlocks = 512;  // two workgroups a CU
+__global__ __launch_bounds__(kBgTpb) void column_sum(float* __restrict__ out, const float* __restrict__ g, int rows,
+    int N, int chunk) {
+    __shared__ float l[kBgWaves][kWave];
     const int lane = threadIdx.x & (kWave - 1);
     const int wid = threadIdx.x / kWave;
     const int n = blockIdx.x * kWave + lane;
-    const int r0 = blockIdx.y * kBgRows;
-    const int r1 = min(rows, r0 + kBgRows);
+    const int r0 = blockIdx.y * chunk, r1 = min(rows, r0 + chunk);
     float s = 0.0f;
-    if (n < N)
-        for (int r = r0 + wid; r < r1; r += 4) s += g[(size_t)r * N + n];
+    if (n < N) {
+        int r = r0 + wid;
+        for (; r + (kBgBatch - 1) * kBgWaves < r1; r += kBgBatch * kBgWaves) {
+            float v[kBgBatch];
+#pragma unroll
+            for (int u = 0; u < kBgBatch; ++u) v[u] = g[(size_t)(r + u * kBgWaves) * N + n];
+#pragma unroll
+            for (int u = 0; u < kBgBatch; ++u) s += v[u];
+        }
+        for (; r < r1; r += kBgWaves) s += g[(size_t)r * N + n];
+    }
     l[wid][lane] = s;
     __syncthreads();
-    if (wid == 0 && n < N) part[(size_t)blockIdx.y * N + n] = ((l[0][lane] + l[1][lane]) + l[2][lane]) + l[3][lane];
+    if (wid == 0 && n < N) {
+        float t = l[0][lane];
+#pragma unroll
+        for (int w = 1; w < kBgWaves; ++w) t += l[w][lane];
+        out[(size_t)blockIdx.y * N + n] = t;
+    }
 }
 
 __global__ __launch_bounds__(kTpb) void fill_kernel(float* __restrict__ p, float v, int n) {
     const int i = blockIdx.x * kTpb + threadIdx.x;
     if (i < n) p[i] = v;
-}
-
-__global__ __launch_bounds__(kTpb) void bias_grad_final(float* __restrict__ gb,
-    const float* __restrict__ part, int chunks, int N) {
-    const int n = blockIdx.x * kTpb + threadIdx.x;
-    if (n >= N) return;
-    float s = 0.0f;
-    for (int c = 0; c < chunks; ++c) s += part[(size_t)c * N + n];
-    gb[n] = s;
 }
 
 // ---------------- mp_cat / mp channel cat: 8 B/out-elem ----------------
@@ -477,18 +491,30 @@ void launch_add_bias(float* Y, const float* b, int M, int N, hipStream_t s) {
 void launch_bias_grad(float* gb, const float* grad_out, int batch, int N, hipStream_t s) {
     NNK_REQUIRE(batch >= 0 && N > 0, "bias_grad", "launch_bias_grad: bad shape batch=%d N=%d", batch, N);
     NNK_REQUIRE(gb, "bias_grad", "launch_bias_grad: null pointer");
-    const int chunks = batch > 0 ? (batch + kBgRows - 1) / kBgRows : 0;
-    if (chunks == 0) {
+    if (batch == 0) {
         // an empty sum is 0, as the reference's loop leaves it
         fill_kernel<<<dim3((unsigned)((N + kTpb - 1) / kTpb)), kTpb, 0, s>>>(gb, 0.0f, N);
         nnk_after_launch("launch_bias_grad", s);
         return;
     }
     NNK_REQUIRE(grad_out, "bias_grad", "launch_bias_grad: null pointer");
+    const int cols = (N + kWave - 1) / kWave;
+    const int per = kBgWaves * kBgBatch;  // rows a workgroup sums per round of loads
+    int chunk = batch;
+    if (batch > kBgDirect) {
+        const int most = cols < kBgBlocks / 2 ? kBgBlocks / cols : 2;
+        chunk = ((batch + most - 1) / most + per - 1) / per * per;
+    }
+    const int chunks = (batch + chunk - 1) / chunk;
+    // taken in every case, so that a capture is refused or not whatever the rows
     float* part = nnk_scratch_acquire((size_t)chunks * N, s, "launch_bias_grad");
     if (!part) return;
-    bias_grad_partial<<<dim3((unsigned)((N + kWave - 1) / kWave), (unsigned)chunks), kTpb, 0, s>>>(part, grad_out, batch, N);
-    bias_grad_final<<<dim3((unsigned)((N + kTpb - 1) / kTpb)), kTpb, 0, s>>>(gb, part, chunks, N);
+    if (chunks == 1) {
+        column_sum<<<dim3((unsigned)cols), kBgTpb, 0, s>>>(gb, grad_out, batch, N, chunk);
+    } else {
+        column_sum<<<dim3((unsigned)cols, (unsigned)chunks), kBgTpb, 0, s>>>(part, grad_out, batch, N, chunk);
+        column_sum<<<dim3((unsigned)cols), kBgTpb, 0, s>>>(gb, part, chunks, N, chunks);
+    }
     nnk_scratch_release(part, s);
     nnk_after_launch("launch_bias_grad", s);
 }
