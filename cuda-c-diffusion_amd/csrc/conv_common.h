@@ -1,0 +1,168 @@
+// conv_common.h -- what the matrix-core convolution kernels share: the shape and
+// epilogue descriptions, the split of fp32 operands into bf16 planes and the
+// products of planes.  Design notes and the MFMA lane layout: k_igemm.hip.
+#pragma once
+#include "nn_hip_rt.h"
+#include "nnk_common.h"
+
+namespace nnk {
+namespace conv {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+struct ConvShape {
+    int B, H, W, Cin, Cout, K, stride, pad, Ho, Wo;
+    int M;    // B * Ho * Wo
+    int KKC;  // K * K * Cin
+    FastDiv wo, ho;  // output pixel decode m -> (b, oh, ow)
+};
+
+// XCD-aware tile order.  Workgroups are dispatched round-robin over the
+// device's 8 XCDs (workgroup L on XCD L % 8), each with its own L2.  Tile
+// L' = xcd_order(L) gives XCD x a contiguous range of tiles, so tiles that
+// read the same activations run in the same L2 instead of on different XCDs.  A bijection of [0, total) for any total.
+constexpr int kXcds = 8;
+__device__ __forceinline__ int xcd_order(int L, int total) {
+    const int x = L % kXcds, j = L / kXcds, q = total / kXcds, r = total % kXcds;
+    return x * q + min(x, r) + j;
+}
+
+// ---------------------------------------------------------------------------
+// fp32 operands on the bf16 matrix cores.  v = p0 + p1 + p2 with p0 = bf16(v),
+// p1 = bf16(v - p0), p2 = v - p0 - p1: 8 + 8 + 8 significand bits, so the sum
+// is exact for every v of 2^-110 and above (below it p2 reaches under the
+// smallest subnormal bf16).  a b is then the sum of the products p_i q_j; the
+// six with i + j <= 2 are taken, the other three are below 2^-25 |a b|.  Each
+// product of two bf16 is exact and the matrix core adds in fp32.
+// ---------------------------------------------------------------------------
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+constexpr int kPlanes = 3;
+
+// the planes of (a, b), a in the low half
+__device__ __forceinline__ void split2(float a, float b, uint32_t (&p)[kPlanes]) {
+#pragma unroll
+    for (int i = 0; i < kPlanes; ++i) {
+        const f32x2 v = {a, b};
+        p[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+        if (i + 1 < kPlanes) {
+            a = a - __uint_as_float(p[i] << 16);
+            b = b - __uint_as_float(p[i] & 0xffff0000u);
+        }
+    }
+}
+
+// the planes of 8 consecutive k
+__device__ __forceinline__ void split8(const float (&v)[8], uint4 (&p)[kPlanes]) {
+    uint32_t d[4][kPlanes];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) split2(v[2 * i], v[2 * i + 1], d[i]);
+#pragma unroll
+    for (int i = 0; i < kPlanes; ++i) p[i] = make_uint4(d[0][i], d[1][i], d[2][i], d[3][i]);
+}
+__device__ __forceinline__ float keep(float v, bool ok) { return __uint_as_float(__float_as_uint(v) & (ok ? ~0u : 0u)); }
+
+// A wave's products over 16 k: T x U accumulators of 32 x 32 from the planes of
+// its row tiles' fragments (lane l: row l % 32, k 8 (l / 32) .. + 7).  The
+// matrix core cuts off what an addend has below the last place of the largest
+// one, towards minus infinity.  p0 q0 products lie on a coarse grid and lose
+// next to nothing; the five small products, added to the same accumulator,
+// would lose enough to shift every output by -6e-8 of its root mean square at
+// K = 1152, which sums over many outputs (a bias gradient, a norm's) show.  So
+// they have an accumulator of their own, `cor`, 2^-8 as large: error against
+// 64 bits 2.0e-7 (mean 2e-10) of the root mean square at K = 1152 with standard
+// normal operands, against 5.2e-7 (mean -6e-8) with one accumulator and 6.1e-7
+// with the fp32 MFMA.  Each product runs over all T x U accumulators, so
+// consecutive MFMAs rarely wait for each other's result.
+template <int T, int U>
+__device__ __forceinline__ void products(const uint4 (&a)[kPlanes][T], const uint4 (&b)[kPlanes][U],
+    f32x16 (&acc)[T][U], f32x16 (&cor)[T][U]) {
+    constexpr int PI[6] = {0, 2, 0, 1, 1, 0}, PJ[6] = {0, 0, 2, 1, 0, 1};
+#pragma unroll
+    for (int x = 0; x < 6; ++x)
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                f32x16& d = x ? cor[t][u] : acc[t][u];
+                d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[PI[x]][t]),
+                    __builtin_bit_cast(bf16x8, b[PJ[x]][u]), d, 0, 0, 0);
+            }
+}
+
+// Whether a wave's results must be formed again from the unsplit operands: a
+// value that is not finite (an infinite or NaN operand, or one that rounds to
+// infinity in bf16, splits into NaN planes), or values all so small that an
+// operand may lie below the split's range.
+template <int T, int U>
+__device__ __forceinline__ bool split_failed(const f32x16 (&acc)[T][U]) {
+    bool bad = false;
+    float mx = 0.0f;
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float v = fabsf(acc[t][u][r]);
+                bad |= !(v <= 3.402823466e38f);
+                mx = fmaxf(mx, v);
+            }
+    if (__any(bad)) return true;
+    return !__any(mx >= 0x1p-80f) && __any(mx > 0.0f);
+}
+
+// Fused neighbours of the forward / input-gradient kernel (bit flags), with v
+// the output after bias or gain:
+//   kXeRes : y = wa * res[m, n] + wb * v            (launch_weighted_sum(y, res, v, wa, wb))
+//   kXeActG: v = v * act'(xa[m, n]) first            (launch_activation_backward)
+//   kXeMod : y = v and y2 = act(v * (cond[b, n] + 1)) (launch_spatial_modulate_act_forward)
+// each with the operation order of the pass it replaces, so the results are
+// those of the separate passes bit for bit.
+enum { kXeNone = 0, kXeRes = 1, kXeActG = 2, kXeMod = 4 };
+struct ConvEpi {
+    const float* bias;  // + bias[n], or null
+    const float* gain;  // * gain[0], or null
+    const float* res;   // kXeRes: [M][C_out]
+    const float* xa;    // kXeActG: [M][C_out]
+    const float* cond;  // kXeMod: [B][C_out]
+    float* y2;          // kXeMod: [M][C_out]
+    float wa, wb;       // kXeRes weights
+    int mp;             // the activation is MP-SiLU (SiLU otherwise)
+    FastDiv hw;         // kXeMod: output pixels per sample
+};
+
+// v with bias or gain, then the fused neighbours in xe, at output (m, n)
+// (offset o).  The act' operand and the residual are read here.
+__device__ __forceinline__ void epilogue_store(float* __restrict__ Y, float v, int xe, uint32_t o, uint32_t co,
+    const ConvEpi& ep, float bias, float gain) {
+    if (ep.bias) v = v + bias;
+    else if (ep.gain) v = v * gain;
+    if (xe & kXeActG) {
+        const float d = act_grad<ACT_SILU, false>(ep.xa[o]);
+        v = v * (ep.mp ? d * kMpSiluScale : d);
+    }
+    if (xe & kXeRes) v = ep.wa * ep.res[o] + ep.wb * v;
+    Y[o] = v;
+    if (xe & kXeMod) {
+        const float z = act_fwd<ACT_SILU, false>(v * (ep.cond[co] + 1.0f));
+        ep.y2[o] = ep.mp ? z * kMpSiluScale : z;
+    }
+}
+
+}  // namespace conv
+}  // namespace nnk
+
+// Few output tiles: 32 x 32 outputs a workgroup, the k range split over its
+// waves (k_conv_small.hip).  `flip`, `xe`: as conv_x3's parameters.
+void nnk_conv_small(bool flip, int xe, float* Y, const float* X, const float* Wt, const nnk::conv::ConvShape& sh,
+    const nnk::conv::ConvEpi& ep, hipStream_t s);
+// gW (overwritten), and with gb non-null the column sums of dY, in one launch.
+void nnk_wgrad_small(float* gW, float* gb, const float* X, const float* dY, const nnk::conv::ConvShape& sh,
+    hipStream_t s);
+// The tiled kernels with a neighbour folded in, of checked shapes (k_igemm_fused.hip).
+void nnk_conv_forward_fused(float* Y, const float* X, const float* Wt, const nnk::conv::ConvShape& sh,
+    nnk::conv::ConvEpi ep, const NnConvFusion& f, hipStream_t s);
+void nnk_conv_input_grad_fused(float* dX, const float* dY, const float* Wt, const nnk::conv::ConvShape& sh,
+    nnk::conv::ConvEpi ep, const NnConvFusion& f, hipStream_t s);

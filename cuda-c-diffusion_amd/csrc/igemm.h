@@ -1,61 +1,19 @@
-// igemm.h -- the implicit-GEMM convolution kernels on the matrix cores, shared
-// by k_igemm.hip (the plain launchers) and k_igemm_fused.hip (the launchers
-// with a neighbouring pass folded into a kernel's operand loads or epilogue).
-// Design notes, the operand split and the MFMA lane layout: k_igemm.hip.
+// igemm.h -- the tiled implicit-GEMM convolution kernels on the matrix cores,
+// shared by k_igemm.hip (the plain launchers) and k_igemm_fused.hip (the
+// launchers with a neighbouring pass folded into a kernel's operand loads or
+// epilogue).  Design notes: k_igemm.hip.
 #pragma once
-#include "nn_hip_rt.h"
-#include "nnk_common.h"
+#include <math.h>
+
+#include "conv_common.h"
 
 namespace {
 
 using namespace nnk;
+using namespace nnk::conv;
 
 constexpr int kBM = 128, kBK = 32, kTpb = 256;
 constexpr int kBNmin = 64;  // output-channel tiles of 128 or 64
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-struct ConvShape {
-    int B, H, W, Cin, Cout, K, stride, pad, Ho, Wo;
-    int M;    // B * Ho * Wo
-    int KKC;  // K * K * Cin
-    FastDiv wo, ho;  // output pixel decode m -> (b, oh, ow)
-};
-
-// XCD-aware tile order.  Workgroups are dispatched round-robin over the
-// device's 8 XCDs (workgroup L on XCD L % 8), each with its own L2.  Tile
-// L' = xcd_order(L) gives XCD x a contiguous range of tiles, so tiles that
-// read the same activations run in the same L2 instead of on different XCDs.  A bijection of [0, total) for any total.
-constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_order(int L, int total) {
-    const int x = L % kXcds, j = L / kXcds, q = total / kXcds, r = total % kXcds;
-    return x * q + min(x, r) + j;
-}
-
-// ---------------------------------------------------------------------------
-// fp32 operands on the bf16 matrix cores.  v = p0 + p1 + p2 with p0 = bf16(v),
-// p1 = bf16(v - p0), p2 = v - p0 - p1: 8 + 8 + 8 significand bits, so the sum
-// is exact for every v of 2^-110 and above (below it p2 reaches under the
-// smallest subnormal bf16).  a b is then the sum of the products p_i q_j; the
-// six with i + j <= 2 are taken, the other three are below 2^-25 |a b|.  Each
-// product of two bf16 is exact and the matrix core adds in fp32.
-// ---------------------------------------------------------------------------
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-constexpr int kPlanes = 3;
-
-// the planes of (a, b), a in the low half
-__device__ __forceinline__ void split2(float a, float b, uint32_t (&p)[kPlanes]) {
-#pragma unroll
-    for (int i = 0; i < kPlanes; ++i) {
-        const f32x2 v = {a, b};
-        p[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-        if (i + 1 < kPlanes) {
-            a = a - __uint_as_float(p[i] << 16);
-            b = b - __uint_as_float(p[i] & 0xffff0000u);
-        }
-    }
-}
 
 // LDS tiles hold rows of 32 k, 64 bytes (four 16-byte chunks) a plane, and
 // every access is 16 bytes a lane.  The order of a row's chunks depends on the
@@ -76,14 +34,6 @@ __device__ __forceinline__ int slot(int row, int c) {
     return (row >> 1) * 8 + ((row ^ (row >> 4)) & 1) * 4 + swz(row, c);
 }
 
-// the planes of 8 consecutive k
-__device__ __forceinline__ void split8(const float (&v)[8], uint4 (&p)[kPlanes]) {
-    uint32_t d[4][kPlanes];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) split2(v[2 * i], v[2 * i + 1], d[i]);
-#pragma unroll
-    for (int i = 0; i < kPlanes; ++i) p[i] = make_uint4(d[0][i], d[1][i], d[2][i], d[3][i]);
-}
 // ... written stride uint4 apart
 __device__ __forceinline__ void put8(uint4* t, int stride, const float (&v)[8]) {
     uint4 p[kPlanes];
@@ -98,36 +48,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const float* p) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, -1, 0x00020000);
 }
 
-__device__ __forceinline__ float keep(float v, bool ok) { return __uint_as_float(__float_as_uint(v) & (ok ? ~0u : 0u)); }
-
-// A wave's products over 16 k: T x U accumulators of 32 x 32 from the planes of
-// its row tiles' fragments (lane l: row l % 32, k 8 (l / 32) .. + 7).  The
-// matrix core cuts off what an addend has below the last place of the largest
-// one, towards minus infinity.  p0 q0 products lie on a coarse grid and lose
-// next to nothing; the five small products, added to the same accumulator,
-// would lose enough to shift every output by -6e-8 of its root mean square at
-// K = 1152, which sums over many outputs (a bias gradient, a norm's) show.  So
-// they have an accumulator of their own, `cor`, 2^-8 as large: error against
-// 64 bits 2.0e-7 (mean 2e-10) of the root mean square at K = 1152 with standard
-// normal operands, against 5.2e-7 (mean -6e-8) with one accumulator and 6.1e-7
-// with the fp32 MFMA.  Each product runs over all T x U accumulators, so
-// consecutive MFMAs rarely wait for each other's result.
-template <int T, int U>
-__device__ __forceinline__ void products(const uint4 (&a)[kPlanes][T], const uint4 (&b)[kPlanes][U],
-    f32x16 (&acc)[T][U], f32x16 (&cor)[T][U]) {
-    constexpr int PI[6] = {0, 2, 0, 1, 1, 0}, PJ[6] = {0, 0, 2, 1, 0, 1};
-#pragma unroll
-    for (int x = 0; x < 6; ++x)
-#pragma unroll
-        for (int t = 0; t < T; ++t)
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                f32x16& d = x ? cor[t][u] : acc[t][u];
-                d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[PI[x]][t]),
-                    __builtin_bit_cast(bf16x8, b[PJ[x]][u]), d, 0, 0, 0);
-            }
-}
-
 // The order of a step's instructions: after each MFMA up to six vector
 // instructions, and a load from LDS or memory where one is left.
 template <int MFMAS>
@@ -140,48 +60,6 @@ __device__ __forceinline__ void sched() {
         __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // memory read
     }
 }
-
-// Whether a wave's results must be formed again from the unsplit operands: a
-// value that is not finite (an infinite or NaN operand, or one that rounds to
-// infinity in bf16, splits into NaN planes), or values all so small that an
-// operand may lie below the split's range.
-template <int T, int U>
-__device__ __forceinline__ bool split_failed(const f32x16 (&acc)[T][U]) {
-    bool bad = false;
-    float mx = 0.0f;
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float v = fabsf(acc[t][u][r]);
-                bad |= !(v <= 3.402823466e38f);
-                mx = fmaxf(mx, v);
-            }
-    if (__any(bad)) return true;
-    return !__any(mx >= 0x1p-80f) && __any(mx > 0.0f);
-}
-
-// Fused neighbours of the forward / input-gradient kernel (bit flags), with v
-// the output after bias or gain:
-//   kXeRes : y = wa * res[m, n] + wb * v            (launch_weighted_sum(y, res, v, wa, wb))
-//   kXeActG: v = v * act'(xa[m, n]) first            (launch_activation_backward)
-//   kXeMod : y = v and y2 = act(v * (cond[b, n] + 1)) (launch_spatial_modulate_act_forward)
-// each with the operation order of the pass it replaces, so the results are
-// those of the separate passes bit for bit.
-enum { kXeNone = 0, kXeRes = 1, kXeActG = 2, kXeMod = 4 };
-struct ConvEpi {
-    const float* bias;  // + bias[n], or null
-    const float* gain;  // * gain[0], or null
-    const float* res;   // kXeRes: [M][C_out]
-    const float* xa;    // kXeActG: [M][C_out]
-    const float* cond;  // kXeMod: [B][C_out]
-    float* y2;          // kXeMod: [M][C_out]
-    float wa, wb;       // kXeRes weights
-    int mp;             // the activation is MP-SiLU (SiLU otherwise)
-    FastDiv hw;         // kXeMod: output pixels per sample
-};
 
 // How the activations reach LDS:
 //   kHalo: the rows of all taps once per 32 channels (stride 1, output as large
@@ -527,9 +405,7 @@ __global__ __launch_bounds__(kTpb, 2) void conv_x3(float* __restrict__ Y, const 
     }
 }
 
-// Host side.  Columns per workgroup, how the activations are staged, and the
-// launch.
-inline int conv_bn(int N) { return N > 64 ? 128 : N > 32 ? 64 : 32; }
+// Host side: how the activations are staged, the tile, and the launch.
 
 // Halo rows that leave room for two workgroups on a CU (160 KB of LDS), with
 // the taps' bits in 32.
@@ -541,9 +417,44 @@ inline int conv_mode(const ConvShape& sh, const float* X, const float* Wt, bool 
                                                                                                              : kGather;
 }
 
+// Columns per workgroup of the tiled kernels, or 0 for the small tiles: the
+// least of the times, in us, that fit a sweep of 23 shapes (1x1 to 5x5, 3 to
+// 1024 channels, 3 to 131072 rows).  A tiled workgroup by itself takes `lone` us
+// per slice of 32 channels and tap, and the device `full` us per slice and tile;
+// the small tiles are bound by a wave's round trips of loads or by their vector
+// work (which a flipped weight's scattered rows lengthen).  For example, forward
+// at [8, 7 x 7, 128 -> 128]: small 9.3, 32 / 64 / 128 columns 25 / 33 / 46; [64, 8
+// x 8, 448 -> 448]: 180, 117 / 107 / 138; [20, 40 x 40, 80 -> 200]: 177, 88 / 81 /
+// 74; [4, 16 x 16, 256 -> 256]: 15, 45 / 59 / 80; [16, 16 x 16, 256 -> 256]: 56,
+// 46 / 59 / 80.
+inline int conv_tile(const ConvShape& sh, bool flip) {
+    struct Tile {
+        int bn;
+        double lone, full;
+    };
+    constexpr Tile kTiles[] = {{128, 1.15, 0.0050}, {64, 0.82, 0.0027}, {32, 0.62, 0.0017}};
+    const double KK = (double)sh.K * sh.K;
+    const double steps = KK * ((sh.Cin + 15) / 16), slices = KK * ((sh.Cin + 31) / 32);
+    const double cells = (double)((sh.M + 31) / 32) * ((sh.Cout + 31) / 32);
+    const double waves = steps <= 8 ? 4 : steps <= 24 ? 8 : 16;
+    const double trips = 1.15 * ceil(steps / waves), work = (flip ? 0.00050 : 0.00041) * cells * steps;
+    double best = 3.5 + (trips > work ? trips : work);
+    int bn = 0;
+    for (const Tile& t : kTiles) {
+        const double tiles = (double)((sh.M + kBM - 1) / kBM) * ((sh.Cout + t.bn - 1) / t.bn);
+        const double us = 5.0 + slices * (t.lone > t.full * tiles ? t.lone : t.full * tiles);
+        if (us < best) best = us, bn = t.bn;
+    }
+    return bn;
+}
+
 template <bool FLIP, int XE>
 void conv_launch(float* Y, const float* X, const float* Wt, const ConvShape& sh, const ConvEpi& ep, hipStream_t s) {
-    const int BN = conv_bn(sh.Cout), mode = conv_mode(sh, X, Wt, FLIP);
+    const int BN = conv_tile(sh, FLIP), mode = conv_mode(sh, X, Wt, FLIP);
+    if (BN == 0) {
+        nnk_conv_small(FLIP, XE, Y, X, Wt, sh, ep, s);
+        return;
+    }
     const unsigned grid = (unsigned)((sh.M + kBM - 1) / kBM) * (unsigned)((sh.Cout + BN - 1) / BN);
     const int rows = mode == kHalo ? kBM + 2 * sh.pad * (sh.W + 1) + 1 : kBM;
     const size_t lds = (size_t)rows * kRowSlots * sizeof(uint4);
@@ -565,6 +476,7 @@ void conv_launch(float* Y, const float* X, const float* Wt, const ConvShape& sh,
     if (mode == kHalo) NNK_CONV_MODE(kHalo);
     else if (mode == kGather) NNK_CONV_MODE(kGather);
     else if constexpr (XE == kXeNone) NNK_CONV_MODE(kRagged);
+    else nnk_conv_small(FLIP, XE, Y, X, Wt, sh, ep, s);  // the ragged form has no fused epilogues
 #undef NNK_CONV_MODE
 #undef NNK_CONV
 }
@@ -585,7 +497,9 @@ void conv_launch(float* Y, const float* X, const float* Wt, const ConvShape& sh,
 // ---------------------------------------------------------------------------
 constexpr int kWgM = 32;  // m rows per stage
 
-template <int BN>
+// RAGGED: any channel counts and alignments, columns loaded one by one; else
+// both counts are even and the pointers 8-byte aligned, columns in pairs.
+template <int BN, bool RAGGED>
 __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part, const float* __restrict__ X,
     const float* __restrict__ dY, ConvShape sh, int rows_per_split) {
     constexpr int UT = BN / 64;               // 32-column accumulator tiles per wave
@@ -595,7 +509,7 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int wk = w >> 1, wn = w & 1;
     // tile (k tile, n tile, split z), k tile fastest, in XCD-aware order
-    const int KT = (sh.KKC + 127) / 128, NT = sh.Cout / BN;
+    const int KT = (sh.KKC + 127) / 128, NT = (sh.Cout + BN - 1) / BN;
     const int tl = xcd_order((int)blockIdx.x, (int)gridDim.x);
     const int k0 = (tl % KT) * 128, n0 = ((tl / KT) % NT) * BN, z = tl / (KT * NT);
     const int mbeg = z * rows_per_split;
@@ -606,11 +520,18 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
     const int ws = __builtin_amdgcn_readfirstlane(w);
     const int pn = tid % (BN / 2), dg = (tid / (BN / 2)) & 3;
     const bool dput = BN == 128 || tid < 2 * BN;
-    const int kcol = k0 + 2 * lane;
-    const int tap = kcol < sh.KKC ? kcol / sh.Cin : 0, ci = kcol < sh.KKC ? kcol - tap * sh.Cin : 0;
-    const int kh = tap / sh.K, kw = tap - kh * sh.K;
-    const float* xc = X + ci;
-    const float* dc = dY + n0 + 2 * pn;
+    constexpr int NC = RAGGED ? 2 : 1;  // column addresses of a pair
+    int kh[NC], kw[NC];
+    const float *xc[NC], *dc[NC];
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+        // columns past the end compute the last ones, stored nowhere
+        const int kcol = min(k0 + 2 * lane + j, sh.KKC - (RAGGED ? 1 : 2)), tap = kcol / sh.Cin;
+        kh[j] = tap / sh.K;
+        kw[j] = tap - kh[j] * sh.K;
+        xc[j] = X + (kcol - tap * sh.Cin);
+        dc[j] = dY + min(n0 + 2 * pn + j, sh.Cout - (RAGGED ? 1 : 2));
+    }
 
     // Every lane loads (rows past the end, padding and columns past K*K*C_in
     // read a valid address): a branch around a load would make the compiler's
@@ -618,7 +539,7 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
     // and padding are zeroed when stored.  The next stage's loads are issued
     // before the current stage's MFMAs and split after them.
     float2 va[8], vd[8];
-    bool aok[8];
+    bool aok[NC][8];
     auto load = [&](int ms) {
         // decode the first of the 8 rows, then step along the output row
         const int mf = ms + 8 * ws;
@@ -627,11 +548,17 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
         sh.ho.divmod(t, b, oh);
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            const int ih = (int)oh * sh.stride - sh.pad + kh, iw = (int)ow * sh.stride - sh.pad + kw;
-            aok[q] = (mf + q < mend) & ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
-            const int p = aok[q] ? ((int)b * sh.H + ih) * sh.W + iw : 0;
-            // 32-bit element offsets (the host bounds x and dy below 2^31 elements)
-            va[q] = *reinterpret_cast<const float2*>(xc + (uint32_t)(p * sh.Cin));
+            float v[NC + 1];
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                const int ih = (int)oh * sh.stride - sh.pad + kh[j], iw = (int)ow * sh.stride - sh.pad + kw[j];
+                aok[j][q] = (mf + q < mend) & ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
+                const int p = aok[j][q] ? ((int)b * sh.H + ih) * sh.W + iw : 0;
+                // 32-bit element offsets (the host bounds x and dy below 2^31 elements)
+                if constexpr (RAGGED) v[j] = xc[j][(uint32_t)(p * sh.Cin)];
+                else va[q] = *reinterpret_cast<const float2*>(xc[j] + (uint32_t)(p * sh.Cin));
+            }
+            if constexpr (RAGGED) va[q] = make_float2(v[0], v[1]);
             if (++ow == (uint32_t)sh.Wo) {
                 ow = 0;
                 if (++oh == (uint32_t)sh.Ho) {
@@ -641,8 +568,11 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
             }
         }
 #pragma unroll
-        for (int q = 0; q < 8; ++q)
-            vd[q] = *reinterpret_cast<const float2*>(dc + (uint32_t)(min(ms + 8 * dg + q, mend - 1) * sh.Cout));
+        for (int q = 0; q < 8; ++q) {
+            const uint32_t o = (uint32_t)(min(ms + 8 * dg + q, mend - 1) * sh.Cout);
+            if constexpr (RAGGED) vd[q] = make_float2(dc[0][o], dc[NC - 1][o]);
+            else vd[q] = *reinterpret_cast<const float2*>(dc[0] + o);
+        }
     };
     f32x16 acc[2][UT], cor[2][UT];
 #pragma unroll
@@ -655,12 +585,12 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
     if (nst > 0) load(mbeg);
     for (int st = 0; st < nst; ++st) {
         if (st) __syncthreads();  // the stage before has been read
-        put8(As + slot(2 * lane, ws), PA, {keep(va[0].x, aok[0]), keep(va[1].x, aok[1]), keep(va[2].x, aok[2]),
-                                       keep(va[3].x, aok[3]), keep(va[4].x, aok[4]), keep(va[5].x, aok[5]),
-                                       keep(va[6].x, aok[6]), keep(va[7].x, aok[7])});
-        put8(As + slot(2 * lane + 1, ws), PA, {keep(va[0].y, aok[0]), keep(va[1].y, aok[1]), keep(va[2].y, aok[2]),
-                                           keep(va[3].y, aok[3]), keep(va[4].y, aok[4]), keep(va[5].y, aok[5]),
-                                           keep(va[6].y, aok[6]), keep(va[7].y, aok[7])});
+        put8(As + slot(2 * lane, ws), PA, {keep(va[0].x, aok[0][0]), keep(va[1].x, aok[0][1]), keep(va[2].x, aok[0][2]),
+                                       keep(va[3].x, aok[0][3]), keep(va[4].x, aok[0][4]), keep(va[5].x, aok[0][5]),
+                                       keep(va[6].x, aok[0][6]), keep(va[7].x, aok[0][7])});
+        put8(As + slot(2 * lane + 1, ws), PA, {keep(va[0].y, aok[NC - 1][0]), keep(va[1].y, aok[NC - 1][1]), keep(va[2].y, aok[NC - 1][2]),
+                                           keep(va[3].y, aok[NC - 1][3]), keep(va[4].y, aok[NC - 1][4]), keep(va[5].y, aok[NC - 1][5]),
+                                           keep(va[6].y, aok[NC - 1][6]), keep(va[7].y, aok[NC - 1][7])});
         if (dput) {
             put8(Ds + slot(2 * pn, dg), PD, {vd[0].x, vd[1].x, vd[2].x, vd[3].x, vd[4].x, vd[5].x, vd[6].x, vd[7].x});
             put8(Ds + slot(2 * pn + 1, dg), PD, {vd[0].y, vd[1].y, vd[2].y, vd[3].y, vd[4].y, vd[5].y, vd[6].y, vd[7].y});
@@ -714,7 +644,7 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
             }
 #pragma unroll
             for (int u = 0; u < UT; ++u) {
-                const float v = dY[(size_t)(in ? m : mbeg) * sh.Cout + n0 + wn * (BN / 2) + 32 * u + fr];
+                const float v = dY[(size_t)(in ? m : mbeg) * sh.Cout + min(n0 + wn * (BN / 2) + 32 * u + fr, sh.Cout - 1)];
                 dv[u] = in ? v : 0.0f;
             }
 #pragma unroll
@@ -724,7 +654,7 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
                     acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[t], dv[u], acc[t][u], 0, 0, 0);
         }
     }
-    // partial tile: D[k][n], rows k = k0 + wk 64 + 32 t + 8 (r / 4) + 4 h + r % 4
+    // partial tile (columns past the end are not stored): D[k][n], rows k = k0 + wk 64 + 32 t + 8 (r / 4) + 4 h + r % 4
     float* pb = part + (size_t)z * sh.KKC * sh.Cout + (size_t)(k0 + wk * 64 + 4 * fh) * sh.Cout + n0 + wn * (BN / 2) + fr;
 #pragma unroll
     for (int u = 0; u < UT; ++u)
@@ -733,7 +663,8 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int dk = 32 * t + 8 * (r >> 2) + (r & 3);
-                if (k0 + wk * 64 + 4 * fh + dk < sh.KKC) pb[(size_t)dk * sh.Cout + 32 * u] = acc[t][u][r];
+                if (k0 + wk * 64 + 4 * fh + dk < sh.KKC && n0 + wn * (BN / 2) + 32 * u + fr < sh.Cout)
+                    pb[(size_t)dk * sh.Cout + 32 * u] = acc[t][u][r];
             }
 }
 
@@ -757,14 +688,46 @@ __global__ __launch_bounds__(256) void wgrad_reduce(float* __restrict__ gW, cons
     gW[i] = t;
 }
 
+// The same for many slices of few elements (S beyond kTallS): 16 waves share
+// the slices of 64 elements, eight in flight each, and add their sums in order.
+constexpr int kTallS = 24;
+__global__ __launch_bounds__(1024) void wgrad_reduce_tall(float* __restrict__ gW, const float* __restrict__ part, int S,
+    long long n) {
+    __shared__ float l[16][kWave];
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    const long long i = (long long)blockIdx.x * kWave + lane;
+    float t = 0.0f;
+    if (i < n) {
+        constexpr int kB = 8;
+        int z = wid;
+        for (; z + (kB - 1) * 16 < S; z += kB * 16) {
+            float v[kB];
+#pragma unroll
+            for (int u = 0; u < kB; ++u) v[u] = part[(size_t)(z + 16 * u) * n + i];
+#pragma unroll
+            for (int u = 0; u < kB; ++u) t += v[u];
+        }
+        for (; z < S; z += 16) t += part[(size_t)z * n + i];
+    }
+    l[wid][lane] = t;
+    __syncthreads();
+    if (wid == 0 && i < n) {
+        float a = l[0][lane];
+#pragma unroll
+        for (int w = 1; w < 16; ++w) a += l[w][lane];
+        gW[i] = a;
+    }
+}
+
 struct WgradPlan {
     int S, rows;
 };
 
-int tile_n(int Cout) { return Cout % 128 == 0 ? 128 : 64; }
+// 128 columns a workgroup above 64: a tile of 64 takes more than half as long.
+inline int tile_n(int Cout) { return Cout > 64 ? 128 : 64; }
 
-WgradPlan wgrad_plan(int M, int KKC, int Cout) {
-    const int tiles = ((KKC + 127) / 128) * (Cout / tile_n(Cout));
+inline WgradPlan wgrad_plan(int M, int KKC, int Cout) {
+    const int tiles = ((KKC + 127) / 128) * ((Cout + tile_n(Cout) - 1) / tile_n(Cout));
     // one round of resident workgroups (two per CU on 256 CUs)
     int S = tiles >= 512 ? 1 : 512 / tiles;
     const int smax = (M + kWgM - 1) / kWgM;
@@ -778,6 +741,21 @@ WgradPlan wgrad_plan(int M, int KKC, int Cout) {
     return p;
 }
 
+// Whether the small tiles beat the tiled kernel, by times in us that fit the
+// sweep of conv_tile: the small tiles are bound by round trips or by their
+// vector work, the tiled kernel takes a stage's time for the stages of a split,
+// then the sum of the splits (and the column sums a launch of their own).  For
+// example [8, 7 x 7, 128 -> 128]: small 8.1, tiled 16.5 us; dense [128, 512 ->
+// 512]: 6.0, 13.3; [8, 28 x 28, 32 -> 32]: 61, 19; [16, 16 x 16, 256 -> 256]: 118,
+// 53.
+inline bool wgrad_small_wins(const ConvShape& sh) {
+    const double steps = (sh.M + 15) / 16, cells = (double)((sh.KKC + 31) / 32) * ((sh.Cout + 31) / 32);
+    const double waves = steps <= 8 ? 4 : steps <= 24 ? 8 : 16;
+    const double trips = 2.3 * ceil(steps / waves), work = 0.00078 * cells * steps;
+    const WgradPlan p = wgrad_plan(sh.M, sh.KKC, sh.Cout);
+    const double stage = tile_n(sh.Cout) == 128 ? 3.3 : 2.0;
+    return 4.0 + (trips > work ? trips : work) < 12.0 + stage * (p.rows / kWgM);
+}
 
 // Checks shared by the forward launchers (plain and fused): -1 after
 // recording an error, 0 when there is nothing to do (batch 0), 1 with `sh`
@@ -826,7 +804,37 @@ inline int dgrad_setup(const char* what, const float* dX, const float* dY, const
     return 1;
 }
 
-void wgrad_launch(const char* what, float* gW, const float* X, const float* dY, int batch, int H, int W, int C_in,
+// The tiled weight gradient of a checked, non-empty shape.
+inline void wgrad_run(const char* what, float* gW, const float* X, const float* dY, const ConvShape& sh,
+    float* workspace, hipStream_t s) {
+    const WgradPlan p = wgrad_plan(sh.M, sh.KKC, sh.Cout);
+    float* part = gW;
+    bool pooled = false;
+    if (p.S > 1) {
+        if (workspace) {
+            part = workspace;
+        } else {
+            part = nnk_scratch_acquire((size_t)p.S * sh.KKC * sh.Cout, s, what);
+            if (!part) return;
+            pooled = true;
+        }
+    }
+    const int BN = tile_n(sh.Cout);
+    const dim3 grid((unsigned)((sh.KKC + 127) / 128) * (unsigned)((sh.Cout + BN - 1) / BN) * (unsigned)p.S);
+    const bool pairs = sh.Cin % 2 == 0 && sh.Cout % 2 == 0 && (uintptr_t)X % 8 == 0 && (uintptr_t)dY % 8 == 0;
+    if (BN == 128 && pairs) igemm_wgrad<128, false><<<grid, kTpb, 0, s>>>(part, X, dY, sh, p.rows);
+    else if (BN == 128) igemm_wgrad<128, true><<<grid, kTpb, 0, s>>>(part, X, dY, sh, p.rows);
+    else if (pairs) igemm_wgrad<64, false><<<grid, kTpb, 0, s>>>(part, X, dY, sh, p.rows);
+    else igemm_wgrad<64, true><<<grid, kTpb, 0, s>>>(part, X, dY, sh, p.rows);
+    if (p.S > 1) {
+        const long long n = (long long)sh.KKC * sh.Cout;
+        if (p.S > kTallS) wgrad_reduce_tall<<<(unsigned)((n + kWave - 1) / kWave), 1024, 0, s>>>(gW, part, p.S, n);
+        else wgrad_reduce<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(gW, part, p.S, n);
+    }
+    if (pooled) nnk_scratch_release(part, s);
+}
+
+inline void wgrad_launch(const char* what, float* gW, const float* X, const float* dY, int batch, int H, int W, int C_in,
     int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace, hipStream_t s) {
     NNK_REQUIRE(batch >= 0 && H > 0 && W > 0 && K > 0 && stride > 0 && pad >= 0, what, "%s: bad geometry", what);
     NNK_REQUIRE(nnhip_conv2d_wgrad_implicit_supported(C_in, C_out), what,
@@ -845,27 +853,8 @@ void wgrad_launch(const char* what, float* gW, const float* X, const float* dY, 
     NNK_REQUIRE(aligned16(X) && aligned16(dY), what, "%s: X and dY must be 16-byte aligned", what);
     ConvShape sh{batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, batch * H_out * W_out, KKC,
         FastDiv((uint32_t)W_out), FastDiv((uint32_t)H_out)};
-    const WgradPlan p = wgrad_plan(sh.M, KKC, C_out);
-    float* part = gW;
-    bool pooled = false;
-    if (p.S > 1) {
-        if (workspace) {
-            part = workspace;
-        } else {
-            part = nnk_scratch_acquire((size_t)p.S * KKC * C_out, s, what);
-            if (!part) return;
-            pooled = true;
-        }
-    }
-    const int BN = tile_n(C_out);
-    const dim3 grid((unsigned)((KKC + 127) / 128) * (unsigned)(C_out / BN) * (unsigned)p.S);
-    if (BN == 128) igemm_wgrad<128><<<grid, kTpb, 0, s>>>(part, X, dY, sh, p.rows);
-    else igemm_wgrad<64><<<grid, kTpb, 0, s>>>(part, X, dY, sh, p.rows);
-    if (p.S > 1) {
-        const long long n = (long long)KKC * C_out;
-        wgrad_reduce<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(gW, part, p.S, n);
-    }
-    if (pooled) nnk_scratch_release(part, s);
+    if (wgrad_small_wins(sh)) nnk_wgrad_small(gW, nullptr, X, dY, sh, s);
+    else wgrad_run(what, gW, X, dY, sh, workspace, s);
     nnk_after_launch(what, s);
 }
 

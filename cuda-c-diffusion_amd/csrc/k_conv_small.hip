@@ -1,0 +1,294 @@
+// k_conv_small.hip -- convolutions and dense layers (a convolution of one pixel)
+// with few output tiles: 32 x 32 outputs a workgroup, whose waves share the k
+// range, so that a few hundred rows still spread over the device.  The tiled
+// kernels (igemm.h) put the reference DDPM's 7 x 7 x 128 level (392 rows) on
+// four workgroups.
+//
+// A wave loads the fragments of its steps of 16 k straight from memory (lane l:
+// row or column l % 32, k 8 (l / 32) .. + 7), a step ahead, splits both operands
+// in registers and adds up its part of the tile; the parts are added in wave
+// order through LDS and go through the epilogue, so one launch does all and
+// nothing is kept in memory between.  Both operands are split per 32 x 32 tile,
+// four times as often as in the tiled kernels: ~90 vector instructions beside 6
+// MFMAs a step bound it, at about half the tiled kernels' full rate, but from
+// the first workgroup on.  The rules between the two are conv_tile and
+// wgrad_small_wins (igemm.h).
+// Against im2col, rocBLAS and the bias pass at [8, 7 x 7, 128 -> 128]: forward 17 ->
+// 9.3 us, input gradient 12 -> 11.6, weight gradient with the bias gradient 30 ->
+// 8.1; dense [128, 512 -> 512] with bias 8 -> 6.2, its weight and bias gradients 11
+// -> 6.0.
+#include "conv_common.h"
+
+namespace {
+
+using namespace nnk;
+using namespace nnk::conv;
+
+constexpr int kT = 32;     // tile edge
+// Steps whose operands are on their way.  Two measured 5-20 % slower: the vector
+// work of the four waves on a SIMD, not the loads, bounds a step.
+constexpr int kAhead = 1;
+
+// Parts in LDS, [wave][row][column]; accumulator register r of lane l holds row
+// 8 (r / 4) + 4 (l / 32) + r % 4 of column l % 32.
+__device__ __forceinline__ void put_part(float* lds, int w, int fr, int fh, const f32x16& v) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) lds[w * kT * kT + (8 * (r >> 2) + 4 * fh + (r & 3)) * kT + fr] = v[r];
+}
+
+// the sum of the waves' parts of element i, in wave order
+template <int WAVES>
+__device__ __forceinline__ float sum_parts(const float* lds, int i) {
+    float v = lds[i];
+#pragma unroll
+    for (int q = 1; q < WAVES; ++q) v += lds[q * kT * kT + i];
+    return v;
+}
+
+// VEC: channel counts are multiples of 8 and the pointers 16-byte aligned, so
+// that 8 k of a pixel (and of a flipped weight's row) are two 16-byte loads.
+template <int WAVES, bool FLIP, bool VEC>
+__global__ __launch_bounds__(64 * WAVES) void conv_small(float* __restrict__ Y, const float* __restrict__ X,
+    const float* __restrict__ Wt, ConvShape sh, ConvEpi ep, int xe) {
+    __shared__ float lds[WAVES * kT * kT];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 31, fh = lane >> 5;
+    const int nt = (sh.Cout + kT - 1) / kT;
+    const int tl = xcd_order((int)blockIdx.x, (int)gridDim.x);
+    const int m0 = tl / nt * kT, n0 = tl % nt * kT;
+    const int nc = min(n0 + fr, sh.Cout - 1);
+    const int KK = sh.K * sh.K, nk = (sh.Cin + 15) / 16, steps = KK * nk;
+    const int per = (steps + WAVES - 1) / WAVES, s0 = w * per, s1 = min(steps, s0 + per);
+    uint32_t q, ow, b, oh;
+    sh.wo.divmod((uint32_t)min(m0 + fr, sh.M - 1), q, ow);  // a row past the end computes the last, stores nothing
+    sh.ho.divmod(q, b, oh);
+    const int ih0 = (int)oh * sh.stride - sh.pad, iw0 = (int)ow * sh.stride - sh.pad;
+    const float* xb = X + (size_t)b * sh.H * sh.W * sh.Cin;
+
+    // the operands of the next kAhead steps; channels past C_in are zeroed in
+    // the activations (both read valid ones)
+    struct Ops {
+        float va[8], vw[8];
+        bool ok;
+        int c;
+    };
+    Ops o[kAhead];
+    int tap = s0 / nk, c16 = s0 - tap * nk;
+    auto load = [&](Ops& r) {
+        const int kh = tap / sh.K, kw = tap - kh * sh.K, ih = ih0 + kh, iw = iw0 + kw;
+        r.ok = ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
+        const float* x = xb + (size_t)(r.ok ? ih * sh.W + iw : 0) * sh.Cin;
+        r.c = 16 * c16 + 8 * fh;
+        const size_t wt = FLIP ? ((size_t)(KK - 1 - tap) * sh.Cout + nc) * sh.Cin : (size_t)tap * sh.Cin * sh.Cout + nc;
+        if constexpr (VEC) {
+            const int cc = min(r.c, sh.Cin - 8);
+            const float4 u = ld4(x + cc), z = ld4(x + cc + 4);
+            r.va[0] = u.x, r.va[1] = u.y, r.va[2] = u.z, r.va[3] = u.w;
+            r.va[4] = z.x, r.va[5] = z.y, r.va[6] = z.z, r.va[7] = z.w;
+            if constexpr (FLIP) {
+                const float4 g = ld4(Wt + wt + cc), h = ld4(Wt + wt + cc + 4);
+                r.vw[0] = g.x, r.vw[1] = g.y, r.vw[2] = g.z, r.vw[3] = g.w;
+                r.vw[4] = h.x, r.vw[5] = h.y, r.vw[6] = h.z, r.vw[7] = h.w;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) r.vw[i] = Wt[wt + (size_t)(cc + i) * sh.Cout];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int cc = min(r.c + i, sh.Cin - 1);
+                r.va[i] = x[cc];
+                r.vw[i] = Wt[FLIP ? wt + cc : wt + (size_t)cc * sh.Cout];
+            }
+        }
+        if (++c16 == nk) c16 = 0, tap = min(tap + 1, KK - 1);  // past the last step: a harmless reload
+    };
+    f32x16 acc[1][1], cor[1][1];
+    acc[0][0] = cor[0][0] = (f32x16){};
+    if (s0 < s1) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) load(o[u]);
+    }
+    for (int s = s0; s < s1; s += kAhead) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            uint4 pa[kPlanes], pw[kPlanes], a[kPlanes][1], bb[kPlanes][1];
+            const bool in = o[u].ok && s + u < s1;  // a step past the wave's last adds zeros
+#pragma unroll
+            for (int i = 0; i < 8; ++i) o[u].va[i] = keep(o[u].va[i], in && (VEC ? o[u].c : o[u].c + i) < sh.Cin);
+            split8(o[u].va, pa);
+            split8(o[u].vw, pw);
+            load(o[u]);
+#pragma unroll
+            for (int p = 0; p < kPlanes; ++p) a[p][0] = pa[p], bb[p][0] = pw[p];
+            products<1, 1>(a, bb, acc, cor);
+        }
+    }
+    acc[0][0] += cor[0][0];
+    if (split_failed<1, 1>(acc)) {
+        // straight from memory in fp32, 2 k per MFMA; rare, so simple
+        acc[0][0] = (f32x16){};
+        for (int s = s0; s < s1; ++s) {
+            const int t = s / nk, kh = t / sh.K, kw = t - kh * sh.K, ih = ih0 + kh, iw = iw0 + kw;
+            const bool in = ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
+            for (int i = 0; i < 16; i += 2) {
+                const int ci = 16 * (s - t * nk) + i + fh, cc = min(ci, sh.Cin - 1);
+                const float x = xb[(size_t)(in ? ih * sh.W + iw : 0) * sh.Cin + cc];
+                const float y = FLIP ? Wt[((size_t)(KK - 1 - t) * sh.Cout + nc) * sh.Cin + cc]
+                                     : Wt[((size_t)t * sh.Cin + cc) * sh.Cout + nc];
+                acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(in && ci < sh.Cin ? x : 0.0f, ci < sh.Cin ? y : 0.0f,
+                    acc[0][0], 0, 0, 0);
+            }
+        }
+    }
+    put_part(lds, w, fr, fh, acc[0][0]);
+    __syncthreads();
+    const float gain = ep.gain ? ep.gain[0] : 1.0f;
+    for (int i = tid; i < kT * kT; i += 64 * WAVES) {
+        const int m = m0 + i / kT, n = n0 + i % kT;
+        if (m >= sh.M || n >= sh.Cout) continue;
+        uint32_t co = 0;
+        if (xe & kXeMod) {
+            uint32_t bb, r;
+            ep.hw.divmod((uint32_t)m, bb, r);
+            co = bb * (uint32_t)sh.Cout + (uint32_t)n;
+        }
+        epilogue_store(Y, sum_parts<WAVES>(lds, i), xe, (uint32_t)m * (uint32_t)sh.Cout + (uint32_t)n, co, ep,
+            ep.bias ? ep.bias[n] : 0.0f, gain);
+    }
+}
+
+// gW[k, n] = sum_m A[m, k] dY[m, n], A gathered from X; gb[n] = sum_m dY[m, n]
+// from the workgroups of the first k tile.  A step is 16 rows m; all loads are
+// 4 bytes a lane along k and n, so any channel counts and alignments do.
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void wgrad_small(float* __restrict__ gW, float* __restrict__ gb,
+    const float* __restrict__ X, const float* __restrict__ dY, ConvShape sh) {
+    __shared__ float lds[WAVES * kT * kT];
+    __shared__ float bl[WAVES][64];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 31, fh = lane >> 5;
+    const int nt = (sh.Cout + kT - 1) / kT;
+    const int tl = xcd_order((int)blockIdx.x, (int)gridDim.x);
+    const int k0 = tl / nt * kT, n0 = tl % nt * kT;
+    const bool sums = gb != nullptr && k0 == 0;
+    const int nc = min(n0 + fr, sh.Cout - 1), k = min(k0 + fr, sh.KKC - 1);
+    const int tap = k / sh.Cin, ci = k - tap * sh.Cin, kh = tap / sh.K - sh.pad, kw = tap % sh.K - sh.pad;
+    const int steps = (sh.M + 15) / 16, per = (steps + WAVES - 1) / WAVES;
+    const int s0 = w * per, s1 = min(steps, s0 + per);
+
+    struct Ops {
+        float va[8], vd[8];
+        bool in[8];
+    };
+    Ops o[kAhead];
+    auto load = [&](Ops& r, int s) {
+        int m = 16 * s + 8 * fh;
+        uint32_t q, ow, b, oh;
+        sh.wo.divmod((uint32_t)min(m, sh.M - 1), q, ow);
+        sh.ho.divmod(q, b, oh);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int ih = (int)oh * sh.stride + kh, iw = (int)ow * sh.stride + kw;
+            r.in[i] = (m + i < sh.M) & ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
+            r.va[i] = X[(uint32_t)((r.in[i] ? ((int)b * sh.H + ih) * sh.W + iw : 0) * sh.Cin + ci)];
+            r.vd[i] = dY[(uint32_t)(min(m + i, sh.M - 1) * sh.Cout + nc)];
+            if (++ow == (uint32_t)sh.Wo) {
+                ow = 0;
+                if (++oh == (uint32_t)sh.Ho) oh = 0, ++b;
+            }
+        }
+    };
+    f32x16 acc[1][1], cor[1][1];
+    acc[0][0] = cor[0][0] = (f32x16){};
+    float bs = 0.0f;
+    if (s0 < s1) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) load(o[u], min(s0 + u, s1 - 1));
+    }
+    for (int s = s0; s < s1; s += kAhead) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            uint4 pa[kPlanes], pd[kPlanes], a[kPlanes][1], d[kPlanes][1];
+            const bool mine = s + u < s1;  // a step past the wave's last adds zeros
+            if (sums) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) bs += mine && 16 * (s + u) + 8 * fh + i < sh.M ? o[u].vd[i] : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) o[u].va[i] = keep(o[u].va[i], mine && o[u].in[i]);
+            split8(o[u].va, pa);
+            split8(o[u].vd, pd);
+            load(o[u], min(s + u + kAhead, s1 - 1));  // the last one again: harmless, and no branch
+#pragma unroll
+            for (int p = 0; p < kPlanes; ++p) a[p][0] = pa[p], d[p][0] = pd[p];
+            products<1, 1>(a, d, acc, cor);
+        }
+    }
+    acc[0][0] += cor[0][0];
+    if (split_failed<1, 1>(acc)) {
+        // straight from memory in fp32, 2 rows per MFMA; rare, so simple
+        acc[0][0] = (f32x16){};
+        for (int m2 = 16 * s0; m2 < min(16 * s1, sh.M); m2 += 2) {
+            const int m = m2 + fh;
+            uint32_t q, ow, b, oh;
+            sh.wo.divmod((uint32_t)min(m, sh.M - 1), q, ow);
+            sh.ho.divmod(q, b, oh);
+            const int ih = (int)oh * sh.stride + kh, iw = (int)ow * sh.stride + kw;
+            const bool inside = (m < sh.M) & ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
+            const float x = X[(size_t)(inside ? ((int)b * sh.H + ih) * sh.W + iw : 0) * sh.Cin + ci];
+            const float y = dY[(size_t)min(m, sh.M - 1) * sh.Cout + nc];
+            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(inside ? x : 0.0f, m < sh.M ? y : 0.0f, acc[0][0], 0, 0, 0);
+        }
+    }
+    put_part(lds, w, fr, fh, acc[0][0]);
+    if (sums) bl[w][lane] = bs;
+    __syncthreads();
+    for (int i = tid; i < kT * kT; i += 64 * WAVES) {
+        const int kk = k0 + i / kT, n = n0 + i % kT;
+        if (kk < sh.KKC && n < sh.Cout) gW[(size_t)kk * sh.Cout + n] = sum_parts<WAVES>(lds, i);
+    }
+    if (sums && tid < kT && n0 + tid < sh.Cout) {
+        float t = 0.0f;
+#pragma unroll
+        for (int q = 0; q < WAVES; ++q) t += bl[q][tid] + bl[q][tid + 32];
+        gb[n0 + tid] = t;
+    }
+}
+
+// Waves by the steps of a tile: about two steps each, while loads of more waves
+// in flight shorten a tile's time.
+int waves_for(int steps) { return steps <= 8 ? 4 : steps <= 24 ? 8 : 16; }
+
+}  // namespace
+
+void nnk_conv_small(bool flip, int xe, float* Y, const float* X, const float* Wt, const ConvShape& sh,
+    const ConvEpi& ep, hipStream_t s) {
+    const unsigned grid = (unsigned)((sh.M + kT - 1) / kT) * (unsigned)((sh.Cout + kT - 1) / kT);
+    const int waves = waves_for(sh.K * sh.K * ((sh.Cin + 15) / 16));
+    const bool vec = sh.Cin % 8 == 0 && aligned16(X) && (!flip || aligned16(Wt));
+#define NNK_SMALL(W_, F_, V_) conv_small<W_, F_, V_><<<grid, 64 * W_, 0, s>>>(Y, X, Wt, sh, ep, xe)
+#define NNK_SMALL_W(F_, V_)                    \
+    do {                                       \
+        if (waves == 4) NNK_SMALL(4, F_, V_);  \
+        else if (waves == 8) NNK_SMALL(8, F_, V_); \
+        else NNK_SMALL(16, F_, V_);            \
+    } while (0)
+    if (flip) {
+        if (vec) NNK_SMALL_W(true, true);
+        else NNK_SMALL_W(true, false);
+    } else {
+        if (vec) NNK_SMALL_W(false, true);
+        else NNK_SMALL_W(false, false);
+    }
+#undef NNK_SMALL_W
+#undef NNK_SMALL
+}
+
+void nnk_wgrad_small(float* gW, float* gb, const float* X, const float* dY, const ConvShape& sh, hipStream_t s) {
+    const unsigned grid = (unsigned)((sh.KKC + kT - 1) / kT) * (unsigned)((sh.Cout + kT - 1) / kT);
+    const int waves = waves_for((sh.M + 15) / 16);
+    if (waves == 4) wgrad_small<4><<<grid, 256, 0, s>>>(gW, gb, X, dY, sh);
+    else if (waves == 8) wgrad_small<8><<<grid, 512, 0, s>>>(gW, gb, X, dY, sh);
+    else wgrad_small<16><<<grid, 1024, 0, s>>>(gW, gb, X, dY, sh);
+}

@@ -38,6 +38,8 @@
 // differs from a library GEMM's order by rounding only.
 #include "igemm.h"
 
+#include "conv_api.h"
+
 extern "C" {
 
 int nnhip_conv2d_implicit_supported(int C_in, int C_out) {
@@ -89,6 +91,74 @@ void launch_conv2d_weight_grad_implicit(float* gW, const float* X, const float* 
     int C_in, int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace, hipStream_t s) {
     wgrad_launch("launch_conv2d_weight_grad_implicit", gW, X, dY, batch, H, W, C_in, C_out, K, stride, pad, H_out,
         W_out, workspace, s);
+}
+
+// ---- the host modules' products (conv_api.h) ----
+
+int nnk_conv_fits(int batch, int H, int W, int C_in, int C_out, int K, int H_out, int W_out) {
+    const long long most = 1LL << 31;
+    return (long long)batch * H * W * C_in < most && (long long)batch * H_out * W_out * C_out < most &&
+           (long long)K * K * C_in * C_out < most;
+}
+
+void nnk_conv_forward(float* y, const float* x, const float* w, const float* bias, const float* gain, int batch,
+    int H, int W, int C_in, int C_out, int K, int stride, int pad, int H_out, int W_out, const NnConvFusion* f,
+    hipStream_t s) {
+    const char* what = "conv2d forward";
+    NNK_REQUIRE(nnk_conv_fits(batch, H, W, C_in, C_out, K, H_out, W_out), what, "%s: tensor exceeds the 32-bit index range", what);
+    if (batch <= 0) return;
+    const ConvShape sh{batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, batch * H_out * W_out, K * K * C_in,
+        FastDiv((uint32_t)W_out), FastDiv((uint32_t)H_out)};
+    ConvEpi ep{};
+    ep.bias = bias;
+    ep.gain = gain;
+    if (f) nnk_conv_forward_fused(y, x, w, sh, ep, *f, s);
+    else conv_launch<false, kXeNone>(y, x, w, sh, ep, s);
+    nnk_after_launch(what, s);
+}
+
+void nnk_conv_input_grad(float* dx, const float* dy, const float* w, const float* gain, int batch, int H, int W,
+    int C_in, int C_out, int K, int pad, const NnConvFusion* f, hipStream_t s) {
+    const char* what = "conv2d input gradient";
+    NNK_REQUIRE(nnk_conv_fits(batch, H, W, C_in, C_out, K, H + 2 * pad - K + 1, W + 2 * pad - K + 1), what, "%s: tensor exceeds the 32-bit index range", what);
+    if (batch <= 0) return;
+    const ConvShape sh{batch, H + 2 * pad - K + 1, W + 2 * pad - K + 1, C_out, C_in, K, 1, K - 1 - pad, H, W,
+        batch * H * W, K * K * C_out, FastDiv((uint32_t)W), FastDiv((uint32_t)H)};
+    ConvEpi ep{};
+    ep.gain = gain;
+    if (f) nnk_conv_input_grad_fused(dx, dy, w, sh, ep, *f, s);
+    else conv_launch<true, kXeNone>(dx, dy, w, sh, ep, s);
+    nnk_after_launch(what, s);
+}
+
+size_t nnk_conv_weight_grad_workspace(int batch, int C_in, int C_out, int K, int H_out, int W_out) {
+    const long long M = (long long)batch * H_out * W_out;
+    if (M <= 0 || M >= (1LL << 31)) return 0;
+    const WgradPlan p = wgrad_plan((int)M, K * K * C_in, C_out);
+    return p.S > 1 ? (size_t)p.S * K * K * C_in * C_out : 0;
+}
+
+void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy, int batch, int H, int W, int C_in,
+    int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace, hipStream_t s) {
+    const char* what = "conv2d weight gradient";
+    NNK_REQUIRE(nnk_conv_fits(batch, H, W, C_in, C_out, K, H_out, W_out), what, "%s: tensor exceeds the 32-bit index range", what);
+    const int KKC = K * K * C_in;
+    if (batch <= 0) {
+        nnhip_fill_f32(gw, 0.0f, (size_t)KKC * C_out, s);
+        if (gb) nnhip_fill_f32(gb, 0.0f, (size_t)C_out, s);
+        return;
+    }
+    const ConvShape sh{batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, batch * H_out * W_out, KKC,
+        FastDiv((uint32_t)W_out), FastDiv((uint32_t)H_out)};
+    // a capture may not need scratch that the stream does not have: without a
+    // workspace it takes the small tiles, which need none
+    if (wgrad_small_wins(sh) || (!workspace && nnk_capturing(s))) {
+        nnk_wgrad_small(gw, gb, x, dy, sh, s);
+    } else {
+        wgrad_run(what, gw, x, dy, sh, workspace, s);
+        if (gb) launch_bias_grad(gb, dy, sh.M, C_out, s);
+    }
+    nnk_after_launch(what, s);
 }
 
 }  // extern "C"

@@ -19,6 +19,29 @@ bool act_fusable(int act) { return act == ACT_SILU || act == ACT_MP_SILU; }
 
 }  // namespace
 
+void nnk_conv_forward_fused(float* Y, const float* X, const float* Wt, const ConvShape& sh, ConvEpi ep,
+    const NnConvFusion& f, hipStream_t s) {
+    ep.res = f.res;
+    ep.wa = f.res_w;
+    ep.wb = f.out_w;
+    ep.cond = f.cond;
+    ep.y2 = f.y2;
+    ep.hw = FastDiv((uint32_t)(sh.Ho * sh.Wo));
+    ep.mp = f.act == ACT_MP_SILU;
+    if (f.res) conv_launch<false, kXeRes>(Y, X, Wt, sh, ep, s);
+    else conv_launch<false, kXeMod>(Y, X, Wt, sh, ep, s);
+}
+
+void nnk_conv_input_grad_fused(float* dX, const float* dY, const float* Wt, const ConvShape& sh, ConvEpi ep,
+    const NnConvFusion& f, hipStream_t s) {
+    ep.res = f.res;
+    ep.xa = f.act_in;
+    ep.wa = f.res_w;
+    ep.wb = f.out_w;
+    ep.mp = f.act == ACT_MP_SILU;
+    conv_launch<true, kXeActG | kXeRes>(dX, dY, Wt, sh, ep, s);
+}
+
 extern "C" {
 
 void launch_conv2d_forward_implicit_fused(float* Y, const float* X, const float* Wt, const float* bias,
@@ -38,17 +61,9 @@ void launch_conv2d_forward_implicit_fused(float* Y, const float* X, const float*
         return;
     NNK_REQUIRE(!f->cond || f->y2, what, "%s: null y2", what);
     ConvEpi ep{};
-    ep.res = f->res;
-    ep.wa = f->res_w;
-    ep.wb = f->out_w;
-    ep.cond = f->cond;
-    ep.y2 = f->y2;
-    ep.hw = FastDiv((uint32_t)(H_out * W_out));
     ep.bias = bias;
     ep.gain = gain;
-    ep.mp = f->act == ACT_MP_SILU;
-    if (f->res) conv_launch<false, kXeRes>(Y, X, Wt, sh, ep, s);
-    else conv_launch<false, kXeMod>(Y, X, Wt, sh, ep, s);
+    nnk_conv_forward_fused(Y, X, Wt, sh, ep, *f, s);
     nnk_after_launch(what, s);
 }
 
@@ -63,13 +78,8 @@ void launch_conv2d_input_grad_implicit_fused(float* dX, const float* dY, const f
     ConvShape sh;
     if (dgrad_setup(what, dX, dY, Wt, batch, H, W, C_in, C_out, K, pad, sh) <= 0) return;
     ConvEpi ep{};
-    ep.res = f->res;
-    ep.xa = f->act_in;
-    ep.wa = f->res_w;
-    ep.wb = f->out_w;
     ep.gain = gain;
-    ep.mp = f->act == ACT_MP_SILU;
-    conv_launch<true, kXeActG | kXeRes>(dX, dY, Wt, sh, ep, s);
+    nnk_conv_input_grad_fused(dX, dY, Wt, sh, ep, *f, s);
     nnk_after_launch(what, s);
 }
 

@@ -1,0 +1,39 @@
+/* conv_api.h -- the products inside the conv2d, linear and mp_linear modules,
+ * on the matrix-core kernels (csrc/igemm.h, csrc/k_conv_small.hip).  Unlike the
+ * launchers of nn_hip.h they take any channel counts and 4-byte alignment, and
+ * pick the tiled or the small-tile kernels by the work's size.  A dense layer
+ * is a convolution with H = W = K = 1.  Tensors below 2^31 elements
+ * (nnk_conv_fits); errors go to the launch layer's record.
+ */
+#ifndef NN_CONV_API_H
+#define NN_CONV_API_H
+
+#include "nn_hip.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* Whether every tensor of the convolution is within the index range. */
+int nnk_conv_fits(int batch, int H, int W, int C_in, int C_out, int K, int H_out, int W_out);
+
+/* y = conv(x) + bias | * gain[0], then the neighbour in f (may be NULL) as in
+   launch_conv2d_forward_implicit_fused. */
+void nnk_conv_forward(float* y, const float* x, const float* w, const float* bias, const float* gain, int batch,
+    int H, int W, int C_in, int C_out, int K, int stride, int pad, int H_out, int W_out, const NnConvFusion* f,
+    hipStream_t s);
+/* dx of a stride-1 convolution with pad <= K - 1, * gain[0]; f (may be NULL) as
+   in launch_conv2d_input_grad_implicit_fused. */
+void nnk_conv_input_grad(float* dx, const float* dy, const float* w, const float* gain, int batch, int H, int W,
+    int C_in, int C_out, int K, int pad, const NnConvFusion* f, hipStream_t s);
+/* gw, and with gb non-NULL the column sums of dy.  workspace:
+   nnk_conv_weight_grad_workspace floats, enough for every smaller batch. */
+void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy, int batch, int H, int W, int C_in,
+    int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace, hipStream_t s);
+size_t nnk_conv_weight_grad_workspace(int batch, int C_in, int C_out, int K, int H_out, int W_out);
+
+#ifdef __cplusplus
+}
+#endif
+
+#endif /* NN_CONV_API_H */

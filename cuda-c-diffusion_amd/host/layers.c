@@ -19,12 +19,13 @@
  *       (src/sinusoidal.c:47)
  *   launch sequences (the maths)              each kind below cites its own
  * Everything else -- one arena per module, lent workspaces so that no call
- * allocates, the fused GroupNorm+activation kind, the implicit-GEMM
+ * allocates, the fused GroupNorm+activation kind, the matrix-core
  * convolution paths -- is this library's.
  */
 #include <math.h>
 #include <string.h>
 
+#include "conv_api.h"
 #include "layer.h"
 #include "nn_gemm.h"
 
@@ -202,54 +203,87 @@ void groupnorm_shift_backward(Module* gn, const float* x, const float* shift, co
 }
 
 /* ------------------------------------------------------------------------
- * dense layers around a rocBLAS GEMM (the GEMM is outside the fused path):
+ * dense layers, each product a 1 x 1 convolution of one pixel (conv_api.h) with
+ * bias or gain in its epilogue:
  *   mp_linear (src/mp_linear.c:12-39): W normalised in place every forward,
  *     Y = X W * gain; backward gW = X^T dY, g_gain zeroed then accumulated,
  *     gW projected and scaled, dX = dY W^T * gain;
  *   linear (src/linear.c:12-30): Y = X W + b; gW = X^T dY, gb = column sums,
  *     dX = dY W^T.
+ * A product outside the kernels' index range is rocBLAS and a pass of its own.
  * ------------------------------------------------------------------------ */
 
 enum { DB_W, DB_GW, DB_AUX, DB_GAUX, DB_WNWS };
 enum { DD_IN, DD_OUT };
 
-static void mpl_fwd(Layer* L, const float* in, float* out, int batch, Context* ctx)
+/* Y = X W + bias | * gain[0] */
+static void dense_fwd(const Layer* L, const float* in, float* out, const float* bias, const float* gain, int batch,
+    Context* ctx)
 {
     const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
-    launch_weight_normalize(L->buf[DB_W], ni, no, L->k[0], ctx->stream);
+    if (nnk_conv_fits(batch, 1, 1, ni, no, 1, 1, 1)) {
+        nnk_conv_forward(out, in, L->buf[DB_W], bias, gain, batch, 1, 1, ni, no, 1, 1, 0, 1, 1, NULL, ctx->stream);
+        return;
+    }
     nn_gemm_forward(ctx->blas, 1.0f, in, L->buf[DB_W], out, batch, ni, no);
-    launch_scale_by_scalar(out, L->buf[DB_AUX], batch * no, ctx->stream);
+    if (bias) launch_add_bias(out, bias, batch, no, ctx->stream);
+    if (gain) launch_scale_by_scalar(out, gain, batch * no, ctx->stream);
+}
+
+/* gW = X^T dY and, with gb, the column sums of dY */
+static void dense_wgrad(const Layer* L, const float* in, const float* grad_out, float* gb, int batch, Context* ctx)
+{
+    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
+    /* no workspace is lent: the library's scratch where the rows are split */
+    if (nnk_conv_fits(batch, 1, 1, ni, no, 1, 1, 1)) {
+        nnk_conv_weight_grad(L->buf[DB_GW], gb, in, grad_out, batch, 1, 1, ni, no, 1, 1, 0, 1, 1, NULL, ctx->stream);
+        return;
+    }
+    nn_gemm_dW(ctx->blas, 1.0f, in, grad_out, L->buf[DB_GW], batch, ni, no);
+    if (gb) launch_bias_grad(gb, grad_out, batch, no, ctx->stream);
+}
+
+/* dX = dY W^T * gain[0] */
+static void dense_dgrad(const Layer* L, const float* grad_out, float* grad_in, const float* gain, int batch,
+    Context* ctx)
+{
+    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
+    if (nnk_conv_fits(batch, 1, 1, ni, no, 1, 1, 1)) {
+        nnk_conv_input_grad(grad_in, grad_out, L->buf[DB_W], gain, batch, 1, 1, ni, no, 1, 0, NULL, ctx->stream);
+        return;
+    }
+    nn_gemm_dX(ctx->blas, 1.0f, L->buf[DB_W], grad_out, grad_in, batch, ni, no);
+    if (gain) launch_scale_by_scalar(grad_in, gain, batch * ni, ctx->stream);
+}
+
+static void mpl_fwd(Layer* L, const float* in, float* out, int batch, Context* ctx)
+{
+    launch_weight_normalize(L->buf[DB_W], L->dim[DD_IN], L->dim[DD_OUT], L->k[0], ctx->stream);
+    dense_fwd(L, in, out, NULL, L->buf[DB_AUX], batch, ctx);
 }
 
 static void mpl_bwd(Layer* L, const float* in, const float* out, const float* grad_out, float* grad_in, int batch,
     Context* ctx)
 {
     (void)out;
-    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
-    nn_gemm_dW(ctx->blas, 1.0f, in, grad_out, L->buf[DB_GW], batch, ni, no);
+    dense_wgrad(L, in, grad_out, NULL, batch, ctx);
     nnhip_fill_f32(L->buf[DB_GAUX], 0.0f, 1, ctx->stream);
-    launch_weight_normalize_backward_ws(L->buf[DB_GW], L->buf[DB_W], L->buf[DB_AUX], L->buf[DB_GAUX], ni, no,
-        L->buf[DB_WNWS], ctx->stream);
-    if (!grad_in) return;
-    nn_gemm_dX(ctx->blas, 1.0f, L->buf[DB_W], grad_out, grad_in, batch, ni, no);
-    launch_scale_by_scalar(grad_in, L->buf[DB_AUX], batch * ni, ctx->stream);
+    launch_weight_normalize_backward_ws(L->buf[DB_GW], L->buf[DB_W], L->buf[DB_AUX], L->buf[DB_GAUX], L->dim[DD_IN],
+        L->dim[DD_OUT], L->buf[DB_WNWS], ctx->stream);
+    if (grad_in) dense_dgrad(L, grad_out, grad_in, L->buf[DB_AUX], batch, ctx);
 }
 
 static void lin_fwd(Layer* L, const float* in, float* out, int batch, Context* ctx)
 {
-    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
-    nn_gemm_forward(ctx->blas, 1.0f, in, L->buf[DB_W], out, batch, ni, no);
-    launch_add_bias(out, L->buf[DB_AUX], batch, no, ctx->stream);
+    dense_fwd(L, in, out, L->buf[DB_AUX], NULL, batch, ctx);
 }
 
 static void lin_bwd(Layer* L, const float* in, const float* out, const float* grad_out, float* grad_in, int batch,
     Context* ctx)
 {
     (void)out;
-    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
-    nn_gemm_dW(ctx->blas, 1.0f, in, grad_out, L->buf[DB_GW], batch, ni, no);
-    launch_bias_grad(L->buf[DB_GAUX], grad_out, batch, no, ctx->stream);
-    if (grad_in) nn_gemm_dX(ctx->blas, 1.0f, L->buf[DB_W], grad_out, grad_in, batch, ni, no);
+    dense_wgrad(L, in, grad_out, L->buf[DB_GAUX], batch, ctx);
+    if (grad_in) dense_dgrad(L, grad_out, grad_in, NULL, batch, ctx);
 }
 
 static const LayerKind kMpLinear = {"mp_linear", mpl_fwd, mpl_bwd};
@@ -334,18 +368,15 @@ Module* sinusoidal_create(int num_channels, float max_period)
 /* ------------------------------------------------------------------------
  * conv2d, NHWC, plain (bias) or magnitude-preserving (forced weight norm and
  * gain), weights [K*K*C_in, C_out] row-major (src/conv2d.c:17-66).
- * Forward: the implicit-GEMM kernel on the matrix cores when the channel
- * counts allow it (C_in % 32 == 0, C_out % 64 == 0), bias or gain in its
- * epilogue; otherwise im2col + rocBLAS + the bias/gain pass, as the
- * reference.  Backward: the weight gradient as an implicit GEMM (C_in % 4,
- * C_out % 64), the stride-1 input gradient as the implicit convolution of
- * grad_out with the flipped kernel (C_out % 32, C_in % 64); otherwise
- * im2col + rocBLAS and the gather col2im, which needs no memset of grad_in.
- * The implicit kernels read the weight in its own layout.
- * NNHIP_CONV_PATH=gemm forces the reference's sequence.  Its im2col matrix
- * (max_batch * H_out * W_out * K*K*C_in floats, 604 MB at cfg3) is allocated
- * only for a path the implicit kernels do not take, or when the variable is
- * set as the module is created; forcing the sequence later is refused.
+ * The matrix-core kernels (conv_api.h) take every forward and weight gradient
+ * and the input gradient of stride 1 with pad <= K - 1, at any channel counts,
+ * bias or gain in the epilogue, the weight in its own layout.  The input
+ * gradient of other strides is rocBLAS and the gather col2im, which needs no
+ * memset of grad_in.  NNHIP_CONV_PATH=gemm forces the reference's sequence of
+ * im2col, GEMM and bias/gain pass.  Its im2col matrix (max_batch * H_out * W_out
+ * * K*K*C_in floats, 604 MB at cfg3) is allocated only for a path the kernels do
+ * not take, or when the variable is set as the module is created; forcing the
+ * sequence later is refused.
  * ------------------------------------------------------------------------ */
 
 enum { CB_W, CB_GW, CB_AUX, CB_GAUX, CB_COL, CB_WGWS, CB_WNWS };
@@ -357,30 +388,6 @@ static int conv_gemm_forced(void)
     return e && strcmp(e, "gemm") == 0;
 }
 
-static int conv_implicit_forced(void)
-{
-    const char* e = getenv("NNHIP_CONV_PATH");
-    return e && strcmp(e, "implicit") == 0;
-}
-
-/* Whether the implicit-GEMM kernel (igemm_fwd: the forward, and the stride-1
-   input gradient) beats im2col + rocBLAS for an M x N x K product, by a cost
-   model fitted on MI355X.  A 128 x BN output tile takes ~1.33 us per 32-deep k
-   slice with one workgroup per CU (cfg3's forward: 36 slices, 1024 tiles,
-   four tiles per CU: 191 us), so few tiles leave the device idle: at the
-   reference DDPM's 7 x 7 x 128 level (M = 392 at batch 8, 4 tiles) the kernel
-   takes ~48 us where the GEMM path takes ~20.  The GEMM path: ~10 us of fixed
-   cost, the GEMM at ~70 TFLOP/s (rocBLAS fp32, measured at cfg3) and the
-   im2col matrix written and read at ~6 TB/s. */
-static int conv_implicit_wins(long long M, int N, int K)
-{
-    const int bn = N % 128 == 0 ? 128 : 64;
-    const double tiles = (double)((M + 127) / 128) * ((N + bn - 1) / bn);
-    const double t_impl = (K / 32.0) * 1.33 * ceil(tiles / 256.0);
-    const double t_gemm = 10.0 + 2.0 * (double)M * N * K / 70e6 + 8.0 * (double)M * K / 6e6;
-    return t_impl <= t_gemm;
-}
-
 /* the reference's sequence asked for at this call (needs the im2col buffer) */
 static int conv_gemm_path(const Layer* L)
 {
@@ -390,18 +397,6 @@ static int conv_gemm_path(const Layer* L)
     return 1;
 }
 
-/* The implicit-GEMM kernels take 128-bit loads of the activations they
-   gather; a misaligned tensor would make them refuse and leave the output
-   unwritten, so the module stops with a message instead. */
-static void conv_require_aligned(const float* p, const char* what)
-{
-    if (((uintptr_t)p & 15u) != 0) {
-        fprintf(stderr, "conv2d: %s at %p is not 16-byte aligned (the implicit-GEMM path needs it)\n", what,
-            (const void*)p);
-        exit(1);
-    }
-}
-
 static void conv_fwd(Layer* L, const float* in, float* out, int batch, Context* ctx)
 {
     const int* d = L->dim;
@@ -409,9 +404,8 @@ static void conv_fwd(Layer* L, const float* in, float* out, int batch, Context* 
     float *w = L->buf[CB_W], *aux = L->buf[CB_AUX];
     if (d[CD_MP]) launch_weight_normalize(w, kg, d[CD_COUT], L->k[0], ctx->stream);
     if (d[CD_FWD] && !conv_gemm_path(L)) {
-        conv_require_aligned(in, "the forward input");
-        launch_conv2d_forward_implicit(out, in, w, d[CD_MP] ? NULL : aux, d[CD_MP] ? aux : NULL, batch,
-            d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_S], d[CD_P], d[CD_HO], d[CD_WO], ctx->stream);
+        nnk_conv_forward(out, in, w, d[CD_MP] ? NULL : aux, d[CD_MP] ? aux : NULL, batch, d[CD_HI], d[CD_WI],
+            d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_S], d[CD_P], d[CD_HO], d[CD_WO], NULL, ctx->stream);
         return;
     }
     launch_im2col(L->buf[CB_COL], in, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_K], d[CD_S], d[CD_P], d[CD_HO],
@@ -429,30 +423,27 @@ static void conv_bwd(Layer* L, const float* in, const float* out, const float* g
     const int kg = d[CD_K] * d[CD_K] * d[CD_CIN], rows = batch * d[CD_HO] * d[CD_WO];
     const int forced = conv_gemm_path(L);
     float *w = L->buf[CB_W], *gw = L->buf[CB_GW], *col = L->buf[CB_COL];
+    float* gb = d[CD_MP] ? NULL : L->buf[CB_GAUX];
     if (d[CD_WGRAD] && !forced) {
-        conv_require_aligned(in, "the forward input");
-        conv_require_aligned(grad_out, "the output gradient");
-        launch_conv2d_weight_grad_implicit(gw, in, grad_out, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT],
-            d[CD_K], d[CD_S], d[CD_P], d[CD_HO], d[CD_WO], L->buf[CB_WGWS], ctx->stream);
+        nnk_conv_weight_grad(gw, gb, in, grad_out, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K],
+            d[CD_S], d[CD_P], d[CD_HO], d[CD_WO], L->buf[CB_WGWS], ctx->stream);
     } else {
         launch_im2col(col, in, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_K], d[CD_S], d[CD_P], d[CD_HO], d[CD_WO],
             ctx->stream);
         nn_gemm_dW(ctx->blas, 1.0f, col, grad_out, gw, rows, kg, d[CD_COUT]);
+        if (gb) launch_bias_grad(gb, grad_out, rows, d[CD_COUT], ctx->stream);
     }
     if (d[CD_MP]) {
         nnhip_fill_f32(L->buf[CB_GAUX], 0.0f, 1, ctx->stream);
         launch_weight_normalize_backward_ws(gw, w, L->buf[CB_AUX], L->buf[CB_GAUX], kg, d[CD_COUT],
             L->buf[CB_WNWS], ctx->stream);
-    } else {
-        launch_bias_grad(L->buf[CB_GAUX], grad_out, rows, d[CD_COUT], ctx->stream);
     }
     if (!grad_in) return;
     const float* gain = d[CD_MP] ? L->buf[CB_AUX] : NULL;
     if (d[CD_DGRAD] && !forced) {
         /* stride 1: dx = conv(dy, flipped kernel, pad K-1-pad), times the gain in mp mode */
-        conv_require_aligned(grad_out, "the output gradient");
-        launch_conv2d_input_grad_implicit(grad_in, grad_out, w, gain, batch, d[CD_HI], d[CD_WI], d[CD_CIN],
-            d[CD_COUT], d[CD_K], d[CD_P], ctx->stream);
+        nnk_conv_input_grad(grad_in, grad_out, w, gain, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K],
+            d[CD_P], NULL, ctx->stream);
         return;
     }
     nn_gemm_dX(ctx->blas, 1.0f, w, grad_out, col, rows, kg, d[CD_COUT]);
@@ -464,23 +455,25 @@ static void conv_bwd(Layer* L, const float* in, const float* out, const float* g
 static const LayerKind kConv2d = {"conv2d", conv_fwd, conv_bwd};
 
 /* The convolution with a neighbouring pass of the diffusion blocks folded into
-   its implicit-GEMM kernels (launch_conv2d_*_implicit_fused), so that the
-   tensor between the two never goes through HBM.  Where the implicit kernels
-   do not take the convolution (channel counts, NNHIP_CONV_PATH=gemm), the
+   its kernels, so that the tensor between the two never goes through HBM.
+   Where they do not take it (channel counts that are no multiple of 8, which
+   the kernels' epilogues do not serve at full speed, NNHIP_CONV_PATH=gemm), the
    module's own forward/backward runs and the pass follows as a launch of its
    own, the reference's sequence.  The results are the same either way. */
 
-static int conv_fused_fwd(const Layer* L) { return L->dim[CD_FWD] && !conv_gemm_path(L); }
-static int conv_fused_bwd(const Layer* L) { return L->dim[CD_WGRAD] && L->dim[CD_DGRAD] && !conv_gemm_path(L); }
+static int conv_fused_fwd(const Layer* L) { return L->dim[CD_FWD] && L->dim[CD_CIN] % 8 == 0 && !conv_gemm_path(L); }
+static int conv_fused_bwd(const Layer* L)
+{
+    return L->dim[CD_WGRAD] && L->dim[CD_DGRAD] && L->dim[CD_COUT] % 8 == 0 && !conv_gemm_path(L);
+}
 
 static void conv_fused_forward(Layer* L, const float* in, float* out, int batch, const NnConvFusion* f, Context* ctx)
 {
     const int* d = L->dim;
     float *w = L->buf[CB_W], *aux = L->buf[CB_AUX];
     if (d[CD_MP]) launch_weight_normalize(w, d[CD_K] * d[CD_K] * d[CD_CIN], d[CD_COUT], L->k[0], ctx->stream);
-    conv_require_aligned(in, "the forward input");
-    launch_conv2d_forward_implicit_fused(out, in, w, d[CD_MP] ? NULL : aux, d[CD_MP] ? aux : NULL, batch, d[CD_HI],
-        d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_S], d[CD_P], d[CD_HO], d[CD_WO], f, ctx->stream);
+    nnk_conv_forward(out, in, w, d[CD_MP] ? NULL : aux, d[CD_MP] ? aux : NULL, batch, d[CD_HI], d[CD_WI],
+        d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_S], d[CD_P], d[CD_HO], d[CD_WO], f, ctx->stream);
 }
 
 void conv2d_forward_residual(Module* m, const float* in, float* out, const float* res, float res_w, float out_w,
@@ -541,9 +534,8 @@ void conv2d_backward_act_residual(Module* m, const float* in, const float* grad_
     f.res = res;
     f.res_w = res_w;
     f.out_w = 1.0f;
-    conv_require_aligned(grad_out, "the output gradient");
-    launch_conv2d_input_grad_implicit_fused(grad_in, grad_out, L->buf[CB_W], d[CD_MP] ? L->buf[CB_AUX] : NULL, batch,
-        d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_P], &f, ctx->stream);
+    nnk_conv_input_grad(grad_in, grad_out, L->buf[CB_W], d[CD_MP] ? L->buf[CB_AUX] : NULL, batch, d[CD_HI],
+        d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_P], &f, ctx->stream);
 }
 
 Module* conv2d_create(Context* ctx, int C_in, int C_out, int K, int stride, int pad, int H, int W, int max_batch,
@@ -564,25 +556,20 @@ Module* conv2d_create(Context* ctx, int C_in, int C_out, int K, int stride, int 
     d[CD_HO] = Ho;
     d[CD_WO] = Wo;
     d[CD_MP] = mp_mode != 0;
-    /* the implicit kernels where the channel counts allow them and, for the
-       forward and input gradient, where they beat the GEMM path at max_batch
-       (NNHIP_CONV_PATH=implicit at creation: wherever allowed) */
-    const int forced = conv_implicit_forced();
-    d[CD_FWD] = nnhip_conv2d_implicit_supported(C_in, C_out) &&
-                (forced || conv_implicit_wins((long long)max_batch * Ho * Wo, C_out, kg));
-    d[CD_WGRAD] = nnhip_conv2d_wgrad_implicit_supported(C_in, C_out);
-    d[CD_DGRAD] = nnhip_conv2d_input_grad_implicit_supported(C_in, C_out, K, stride, pad) &&
-                  (forced || conv_implicit_wins((long long)max_batch * H * W, C_in, K * K * C_out));
+    const int fits = nnk_conv_fits(max_batch, H, W, C_in, C_out, K, Ho, Wo);
+    d[CD_FWD] = fits;
+    d[CD_WGRAD] = fits;
+    d[CD_DGRAD] = fits && stride == 1 && pad <= K - 1;
     L->k[0] = 1e-4f;
     const int aux_n = mp_mode ? 1 : C_out;
     layer_buf(L, nw, 0);
     layer_buf(L, nw, 0);
     layer_buf(L, (size_t)aux_n, 1);
     layer_buf(L, (size_t)aux_n, 0);
-    /* the im2col matrix, for the paths the implicit kernels do not take */
+    /* the im2col matrix, for the paths the matrix-core kernels do not take */
     const int need_col = !d[CD_FWD] || !d[CD_WGRAD] || !d[CD_DGRAD] || conv_gemm_forced();
     layer_buf(L, need_col ? (size_t)max_batch * Ho * Wo * kg : 0, 0);
-    layer_buf(L, d[CD_WGRAD] ? nnhip_conv2d_wgrad_workspace(max_batch, C_in, C_out, K, Ho, Wo) : 0, 0);
+    layer_buf(L, d[CD_WGRAD] ? nnk_conv_weight_grad_workspace(max_batch, C_in, C_out, K, Ho, Wo) : 0, 0);
     layer_buf(L, mp_mode ? nnhip_weight_normalize_backward_workspace(C_out) : 0, 1);
     layer_param(L, CB_W, CB_GW, (int)nw);
     layer_param(L, CB_AUX, CB_GAUX, aux_n);

@@ -1,0 +1,135 @@
+"""The products of the conv2d, linear and mp_linear modules (host/conv_api.h) at
+any channel counts and alignment, at the edges of the small tiles (32 x 32
+outputs, 16 k a step, 4 / 8 / 16 waves) and of the tiled kernels' ragged forms,
+against double; bar as in test_gpu_conv_implicit.py.  Geometries past each rule
+of the choice between them: few tiles (small), many (128, 64 or 32 columns)."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from helpers import TOL, assert_bits_equal
+from test_gpu_conv_split import _conv64
+
+pytestmark = pytest.mark.gpu
+
+P, I = C.c_void_p, C.c_int
+
+GEOMS = [
+    # B, H, W, C_in, C_out, K, stride, pad, offset of every tensor in floats
+    (1, 1, 1, 1, 1, 1, 1, 0, 0),        # one product
+    (33, 1, 1, 17, 31, 1, 1, 0, 0),     # dense, ragged, two row tiles
+    (128, 1, 1, 512, 512, 1, 1, 0, 0),  # dense
+    (5, 1, 1, 64, 96, 1, 1, 0, 1),      # dense, misaligned
+    (8, 7, 7, 128, 128, 3, 1, 1, 0),    # small tiles, 72 steps
+    (2, 6, 5, 40, 33, 3, 1, 1, 0),      # C_in no multiple of 16
+    (64, 32, 32, 3, 64, 3, 1, 1, 0),    # an image in: ragged rows, tiled
+    (64, 32, 32, 64, 3, 3, 1, 1, 0),    # an image out
+    (3, 65, 64, 20, 70, 3, 1, 1, 0),    # ragged, 128 columns of which 70 are
+    (40, 32, 32, 24, 48, 3, 1, 1, 0),   # halo rows with a partial slice, 64 columns
+    (40, 32, 32, 48, 96, 3, 1, 1, 1),   # misaligned: 4-byte loads
+    (16, 33, 31, 10, 130, 5, 2, 2, 0),  # strided, even channels in pairs
+    (90, 16, 16, 5, 7, 3, 2, 1, 0),
+    (700, 7, 7, 6, 34, 1, 1, 0, 0),     # weight gradient of many splits and few elements
+]
+
+
+def _api(L):
+    d = L.dll
+    d.nnk_conv_forward.argtypes = [P] * 5 + [I] * 10 + [P, P]
+    d.nnk_conv_input_grad.argtypes = [P] * 4 + [I] * 7 + [P, P]
+    d.nnk_conv_weight_grad.argtypes = [P] * 4 + [I] * 10 + [P, P]
+    d.nnk_conv_weight_grad_workspace.argtypes = [I] * 6
+    d.nnk_conv_weight_grad_workspace.restype = C.c_size_t
+    for f in (d.nnk_conv_forward, d.nnk_conv_input_grad, d.nnk_conv_weight_grad):
+        f.restype = None
+    return d
+
+
+def _within(got, ref, floor):
+    err = np.abs(got.astype(np.float64) - ref) / np.maximum(np.maximum(np.abs(ref), floor), 1e-30)
+    assert float(err.max()) <= TOL
+
+
+@pytest.mark.parametrize("geom", GEOMS, ids=lambda g: "x".join(map(str, g)))
+def test_conv_products(L, rng, geom):
+    B, H, W, Ci, Co, K, s, p, off = geom
+    print(f"[case] conv products {geom}", flush=True)
+    d = _api(L)
+    Ho, Wo = (H + 2 * p - K) // s + 1, (W + 2 * p - K) // s + 1
+    x = rng.standard_normal((B, H, W, Ci)).astype(np.float32)
+    w = (rng.standard_normal((K * K * Ci, Co)) / np.sqrt(K * K * Ci)).astype(np.float32)
+    g = rng.standard_normal((B, Ho, Wo, Co)).astype(np.float32)
+    bias = rng.standard_normal(Co).astype(np.float32)
+
+    def dev(a):
+        t = L.alloc(a.size + off)
+        t.upload(np.concatenate([np.zeros(off, np.float32), a.ravel()]))
+        return t
+
+    def get(t, shape):
+        return t.download()[off:].reshape(shape)
+
+    xd, wd, gd, bd, gain = dev(x), dev(w), dev(g), L.to_device(bias), L.to_device(np.array([0.7], np.float32))
+    y, gx, gw, gb = L.alloc(g.size + off), L.alloc(x.size + off), L.alloc(w.size + off), L.alloc(Co)
+    o = off
+    geo = (B, H, W, Ci, Co, K, s, p, Ho, Wo)
+    d.nnk_conv_forward(y.offset(o), xd.offset(o), wd.offset(o), bd.p, None, *geo, None, None)
+    ws = L.alloc(max(1, d.nnk_conv_weight_grad_workspace(B, Ci, Co, K, Ho, Wo)))
+    d.nnk_conv_weight_grad(gw.offset(o), gb.p, xd.offset(o), gd.offset(o), *geo, ws.p, None)
+    if s == 1:
+        d.nnk_conv_input_grad(gx.offset(o), gd.offset(o), wd.offset(o), gain.p, B, H, W, Ci, Co, K, p, None, None)
+    L.sync()
+    L.check("conv products")
+    ref, floor = _conv64(x, w, K, s, p)
+    _within(get(y, ref.shape), ref + bias, floor)
+    # the gradients tap by tap
+    xp = np.pad(x.astype(np.float64), ((0, 0), (p, p), (p, p), (0, 0)))
+    g64 = g.astype(np.float64).reshape(-1, Co)
+    gxp, gxq = np.zeros_like(xp), np.zeros_like(xp)
+    rw, fw = [], []
+    for t in range(K * K):
+        i, j = divmod(t, K)
+        at = np.s_[:, i:i + s * (Ho - 1) + 1:s, j:j + s * (Wo - 1) + 1:s]
+        a = xp[at].reshape(-1, Ci)
+        rw.append(a.T @ g64)
+        fw.append(np.sqrt((a * a).T @ (g64 * g64)))
+        wt = w[t * Ci:(t + 1) * Ci].astype(np.float64)
+        gxp[at] += (g64 @ wt.T).reshape(B, Ho, Wo, Ci)
+        gxq[at] += ((g64 * g64) @ (wt * wt).T).reshape(B, Ho, Wo, Ci)
+    _within(get(gw, w.shape), np.concatenate(rw), np.concatenate(fw))
+    _within(gb.download(), g64.sum(0), np.sqrt((g64 * g64).sum(0)))
+    if s == 1:
+        cut = np.s_[:, p:p + H, p:p + W]
+        _within(get(gx, x.shape), 0.7 * gxp[cut], 0.7 * np.sqrt(gxq[cut]))
+
+
+@pytest.mark.parametrize("geom", [(2, 5, 6, 24, 40, 3, 1, 1), (1, 4, 4, 64, 64, 3, 1, 1)],
+                         ids=lambda g: "x".join(map(str, g)))
+def test_small_tiles_fused_epilogues(L, nn, rng, geom):
+    """The epilogues on the small tiles against the separate launches, bit for bit."""
+    B, H, W, Ci, Co, K, s, p = geom
+    print(f"[case] small tile epilogues {geom}", flush=True)
+    d = _api(L)
+    n = B * H * W * Co
+    xd = L.to_device(rng.standard_normal((B, H, W, Ci)).astype(np.float32))
+    wd = L.to_device((rng.standard_normal((K * K * Ci, Co)) / np.sqrt(K * K * Ci)).astype(np.float32))
+    gain = L.to_device(np.array([0.91], np.float32))
+    cond = L.to_device((0.5 * rng.standard_normal((B, Co))).astype(np.float32))
+    res = L.to_device(rng.standard_normal(n).astype(np.float32))
+    y, want, got, y2 = L.alloc(n), L.alloc(n), L.alloc(n), L.alloc(n)
+    geo = (B, H, W, Ci, Co, K, s, p, H, W)
+    d.nnk_conv_forward(y.p, xd.p, wd.p, None, gain.p, *geo, None, None)
+    f = nn.NnConvFusion(cond=cond.p, y2=y2.p, act=nn.ACT_MP_SILU)
+    d.nnk_conv_forward(got.p, xd.p, wd.p, None, gain.p, *geo, C.addressof(f), None)
+    L.launch_spatial_modulate_act_forward(want.p, y.p, cond.p, B, H * W, 1, Co, nn.ACT_MP_SILU, None)
+    L.sync()
+    assert_bits_equal(got.download(), y.download(), "y")
+    assert_bits_equal(y2.download(), want.download(), "y2")
+    f = nn.NnConvFusion(res=res.p, res_w=0.83, out_w=0.55)
+    d.nnk_conv_forward(got.p, xd.p, wd.p, None, gain.p, *geo, C.addressof(f), None)
+    L.launch_weighted_sum(want.p, res.p, y.p, 0.83, 0.55, n, None)
+    L.sync()
+    assert_bits_equal(got.download(), want.download(), "residual")
