@@ -23,17 +23,13 @@ constexpr int kBNmin = 64;  // output-channel tiles of 128 or 64
 // lanes along a row, 4 rows x 4 chunks.
 //   rowslot: the three planes of a row beside each other (the convolution's
 //     activations, read at any row offset);
-//   slot: a plane of its own, two rows to a 128-byte line, the halves of rows
-//     16 apart swapped for the transposing writes, 16 rows two apart (the
-//     weight gradient's tiles).
+//   stage_slot: a plane of its own with 16 k a row (the weight gradient's tiles):
+//     32 bytes a row, the two chunks swapped on alternate groups of 8 rows.
 __device__ __forceinline__ int swz(int row, int c) { return c ^ ((row >> 2) & 3); }
 constexpr int kRowSlots = 4 * kPlanes;  // uint4 per row of all planes
 __device__ __forceinline__ int rowslot(int row, int c) { return row * kRowSlots + swz(row, c); }
-constexpr int kRow4 = 4;  // uint4 per row of one plane
-__device__ __forceinline__ int slot(int row, int c) {
-    return (row >> 1) * 8 + ((row ^ (row >> 4)) & 1) * 4 + swz(row, c);
-}
-
+constexpr int kStage4 = 2;  // uint4 per row of one plane
+__device__ __forceinline__ int stage_slot(int row, int c) { return row * kStage4 + (c ^ ((row >> 3) & 1)); }
 // ... written stride uint4 apart
 __device__ __forceinline__ void put8(uint4* t, int stride, const float (&v)[8]) {
     uint4 p[kPlanes];
@@ -48,15 +44,16 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const float* p) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, -1, 0x00020000);
 }
 
-// The order of a step's instructions: after each MFMA up to six vector
-// instructions, and a load from LDS or memory where one is left.
-template <int MFMAS>
+// The order of a step's instructions: after each MFMA up to VALU
+// vector instructions, and an access of LDS or a load from memory where one is left.
+template <int MFMAS, int VALU = 6>
 __device__ __forceinline__ void sched() {
 #pragma unroll
     for (int i = 0; i < MFMAS; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // VALU
+        __builtin_amdgcn_sched_group_barrier(0x002, VALU, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
         __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // memory read
     }
 }
@@ -436,7 +433,7 @@ inline int conv_tile(const ConvShape& sh, bool flip) {
     const double KK = (double)sh.K * sh.K;
     const double steps = KK * ((sh.Cin + 15) / 16), slices = KK * ((sh.Cin + 31) / 32);
     const double cells = (double)((sh.M + 31) / 32) * ((sh.Cout + 31) / 32);
-    const double waves = steps <= 8 ? 4 : steps <= 24 ? 8 : 16;
+    const double waves = steps <= 4 ? 4 : steps <= 16 ? 8 : 16;
     const double trips = 1.15 * ceil(steps / waves), work = (flip ? 0.00050 : 0.00041) * cells * steps;
     double best = 3.5 + (trips > work ? trips : work);
     int bn = 0;
@@ -488,25 +485,42 @@ void conv_launch(float* Y, const float* X, const float* Wt, const ConvShape& sh,
 // workgroups per 128 x 128 output tile; split z writes its fixed-order partial
 // tile to part[z], and a second launch adds the S partials in split order.
 //
-// Per stage a workgroup stages 32 pixel rows m of A (its 128 k columns) and
-// of dY (its BN n columns) in LDS transposed and split: per plane and column,
-// 32 consecutive m, so that a lane's MFMA operands run along the pixel
-// reduction (slice_mfma).  Each loader thread gathers 8 consecutive pixel rows
-// of 2 columns, and its registers hold them transposed.  The pixels of a wave
-// are the same in all lanes, so they are decoded in scalar registers.
+// Per stage a workgroup stages 16 pixel rows m of A (its 128 k columns) and of
+// dY (its BN n columns) in LDS transposed and split: per plane and column, 16
+// consecutive m, so that a lane's MFMA operands run along the pixel reduction.
+// A loader thread's registers hold consecutive rows of a column, which is the
+// transpose.
+//
+// What bounds it is the vector work beside the MFMAs: each wave splits its share
+// of both operands and writes it to LDS in every stage (165 vector instructions
+// to 48 MFMAs).  So the stages are pipelined: three LDS buffers and one barrier a
+// stage, the next stage's fragment reads and splits and the one after's loads
+// spread between the MFMAs.  3x3 128 -> 128 at [128, 32, 32]: 264 us with two
+// barriers a stage, 247 so (337 on the fp32 MFMA); 256 -> 256 at [16, 64,
+// 64]: 484, 457.  The column sums of dY (a convolution's bias gradient) come from
+// the rows that the workgroups of the first k tile hold anyway, instead of a
+// pass over dY of two launches (5 us and more).
 // ---------------------------------------------------------------------------
+constexpr int kStage = 16;  // rows per stage
 constexpr int kWgM = 32;  // m rows per stage
 
-// RAGGED: any channel counts and alignments, columns loaded one by one; else
-// both counts are even and the pointers 8-byte aligned, columns in pairs.
-template <int BN, bool RAGGED>
-__global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part, const float* __restrict__ X,
-    const float* __restrict__ dY, ConvShape sh, int rows_per_split) {
-    constexpr int UT = BN / 64;               // 32-column accumulator tiles per wave
-    constexpr int PA = 128 * kRow4, PD = BN * kRow4;  // uint4 per plane
-    __shared__ uint4 As[kPlanes * PA];
-    __shared__ uint4 Ds[kPlanes * PD];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+// How the activation columns are loaded: kSingles one by one, for any channel
+// counts and alignments; kPairs two at a time (C_in even, x 8-byte aligned);
+// kQuads also with W_out a multiple of 4, so that the four consecutive pixels of
+// a loader thread lie in one output row and are decoded once (the decoding is
+// scalar work, which a wave issues in turn with the rest: 148 scalar
+// instructions beside 165 vector ones a stage without it).
+enum { kQuads = 0, kPairs = 1, kSingles = 2 };
+
+template <int BN, int LOADS>
+__global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part, float* __restrict__ sums,
+    size_t stride, const float* __restrict__ X, const float* __restrict__ dY, ConvShape sh, int rows_per_split) {
+    constexpr int UT = BN / 64;                                // 32-column accumulator tiles per wave
+    constexpr int PA = 128 * kStage4, PD = BN * kStage4;       // uint4 per plane
+    constexpr int kBuf = kPlanes * (PA + PD);                  // and per stage buffer
+    extern __shared__ uint4 lds[];                             // three stage buffers: A planes, dY planes
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 31, fh = lane >> 5;
     const int wk = w >> 1, wn = w & 1;
     // tile (k tile, n tile, split z), k tile fastest, in XCD-aware order
     const int KT = (sh.KKC + 127) / 128, NT = (sh.Cout + BN - 1) / BN;
@@ -514,100 +528,181 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
     const int k0 = (tl % KT) * 128, n0 = ((tl / KT) % NT) * BN, z = tl / (KT * NT);
     const int mbeg = z * rows_per_split;
     const int mend = min(sh.M, mbeg + rows_per_split);
-    // loader roles: A columns k0 + 2 pc, + 1 of the stage's pixel rows 8 ws ..
-    // + 7 (ws the wave); dY columns n0 + 2 pn, + 1 of rows 8 dg .. + 7 (with
-    // BN = 64 the upper two waves store no dY)
-    const int ws = __builtin_amdgcn_readfirstlane(w);
-    const int pn = tid % (BN / 2), dg = (tid / (BN / 2)) & 3;
-    const bool dput = BN == 128 || tid < 2 * BN;
-    constexpr int NC = RAGGED ? 2 : 1;  // column addresses of a pair
+    // loader roles.  A: columns k0 + 2 lane, + 1 of the stage's rows 4 w .. + 3
+    // (the pixels of a wave are the same in all lanes, so they are decoded in
+    // scalar registers); column 2 l + j goes to tile row l + 64 j, so that a
+    // wave's 8-byte writes go to consecutive rows.  dY: column n0 + nd of rows
+    // 8 md .. + 7 (with BN = 64 the upper two waves store none).
+    constexpr int NC = LOADS == kSingles ? 2 : 1;  // column addresses of a pair
     int kh[NC], kw[NC];
-    const float *xc[NC], *dc[NC];
+    uint32_t xo[NC];  // the column's offset from the output pixel's input pixel (wraps below it)
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
         // columns past the end compute the last ones, stored nowhere
-        const int kcol = min(k0 + 2 * lane + j, sh.KKC - (RAGGED ? 1 : 2)), tap = kcol / sh.Cin;
-        kh[j] = tap / sh.K;
-        kw[j] = tap - kh[j] * sh.K;
-        xc[j] = X + (kcol - tap * sh.Cin);
-        dc[j] = dY + min(n0 + 2 * pn + j, sh.Cout - (RAGGED ? 1 : 2));
+        const int kcol = min(k0 + 2 * lane + j, sh.KKC - (NC == 2 ? 1 : 2)), tap = kcol / sh.Cin;
+        kh[j] = tap / sh.K - sh.pad;
+        kw[j] = tap % sh.K - sh.pad;
+        xo[j] = (uint32_t)((kh[j] * sh.W + kw[j]) * sh.Cin + kcol - tap * sh.Cin);
     }
+    const int nd = tid % BN, md = (w / (BN / 64)) & 1;
+    const bool dput = tid < 2 * BN;
+    const int dlo = 4 * (min(n0 + nd, sh.Cout - 1) - n0);
 
-    // Every lane loads (rows past the end, padding and columns past K*K*C_in
-    // read a valid address): a branch around a load would make the compiler's
-    // later waits drain the whole vector-memory counter.  A's rows past the end
-    // and padding are zeroed when stored.  The next stage's loads are issued
-    // before the current stage's MFMAs and split after them.
-    float2 va[8], vd[8];
-    bool aok[NC][8];
+    // Every lane loads (rows past the end, padding and columns past the end read
+    // a valid address): a branch around a load would make the compiler's later
+    // waits drain the whole vector-memory counter.  A's rows past the end and
+    // padding are zeroed as they are split.
+    float2 va[4];
+    float vd[8];
+    uint32_t aok[NC][4];  // all ones where the pixel counts: a mask, as a select would become a branch
     auto load = [&](int ms) {
-        // decode the first of the 8 rows, then step along the output row
-        const int mf = ms + 8 * ws;
+        // decode the first of the 4 rows, then step along the output row
+        const int mf = ms + 4 * w;
         uint32_t t, ow, b, oh;
         sh.wo.divmod((uint32_t)(mf < sh.M ? mf : 0), t, ow);
         sh.ho.divmod(t, b, oh);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
+        for (int q = 0; q < 4; ++q) {
+            const int ih = (int)oh * sh.stride, iw = (int)(LOADS == kQuads ? ow + q : ow) * sh.stride;
+            // 32-bit element offsets (the host bounds x below 2^31 elements)
+            const uint32_t px = (((uint32_t)b * sh.H + ih) * sh.W + iw) * sh.Cin;
             float v[NC + 1];
 #pragma unroll
             for (int j = 0; j < NC; ++j) {
-                const int ih = (int)oh * sh.stride - sh.pad + kh[j], iw = (int)ow * sh.stride - sh.pad + kw[j];
-                aok[j][q] = (mf + q < mend) & ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
-                const int p = aok[j][q] ? ((int)b * sh.H + ih) * sh.W + iw : 0;
-                // 32-bit element offsets (the host bounds x and dy below 2^31 elements)
-                if constexpr (RAGGED) v[j] = xc[j][(uint32_t)(p * sh.Cin)];
-                else va[q] = *reinterpret_cast<const float2*>(xc[j] + (uint32_t)(p * sh.Cin));
+                aok[j][q] = -(uint32_t)((mf + q < mend) & ((unsigned)(ih + kh[j]) < (unsigned)sh.H) &
+                                        ((unsigned)(iw + kw[j]) < (unsigned)sh.W));
+                const uint32_t o = (px + xo[j]) & aok[j][q];
+                if constexpr (NC == 2) v[j] = X[o];
+                else va[q] = *reinterpret_cast<const float2*>(X + o);
             }
-            if constexpr (RAGGED) va[q] = make_float2(v[0], v[1]);
-            if (++ow == (uint32_t)sh.Wo) {
-                ow = 0;
-                if (++oh == (uint32_t)sh.Ho) {
-                    oh = 0;
-                    ++b;
+            if constexpr (NC == 2) va[q] = make_float2(v[0], v[1]);
+            if constexpr (LOADS != kQuads) {
+                if (++ow == (uint32_t)sh.Wo) {
+                    ow = 0;
+                    if (++oh == (uint32_t)sh.Ho) {
+                        oh = 0;
+                        ++b;
+                    }
                 }
             }
         }
+        const int dm = min(ms + 8 * md, mend - 1);
+        const auto db = buffer(dY + (size_t)dm * sh.Cout + n0);
+        const int dlim = 4 * min(7, mend - 1 - dm) * sh.Cout;  // rows past the end read the last
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const uint32_t o = (uint32_t)(min(ms + 8 * dg + q, mend - 1) * sh.Cout);
-            if constexpr (RAGGED) vd[q] = make_float2(dc[0][o], dc[NC - 1][o]);
-            else vd[q] = *reinterpret_cast<const float2*>(dc[0] + o);
+        for (int q = 0; q < 8; ++q)
+            vd[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(db, dlo,
+                min(4 * q * sh.Cout, dlim), 0));
+    };
+    const int wa = stage_slot(lane, w >> 1) * 2 + (w & 1), wb = stage_slot(lane + 64, w >> 1) * 2 + (w & 1);
+    const int wd = stage_slot(nd, md);
+    auto store = [&](uint4* buf) {
+        uint2* a2 = reinterpret_cast<uint2*>(buf);
+        uint32_t lo[kPlanes], hi[kPlanes];
+        split2(__uint_as_float(__float_as_uint(va[0].x) & aok[0][0]), __uint_as_float(__float_as_uint(va[1].x) & aok[0][1]), lo);
+        split2(__uint_as_float(__float_as_uint(va[2].x) & aok[0][2]), __uint_as_float(__float_as_uint(va[3].x) & aok[0][3]), hi);
+#pragma unroll
+        for (int p = 0; p < kPlanes; ++p) a2[p * PA * 2 + wa] = make_uint2(lo[p], hi[p]);
+        split2(__uint_as_float(__float_as_uint(va[0].y) & aok[NC - 1][0]), __uint_as_float(__float_as_uint(va[1].y) & aok[NC - 1][1]), lo);
+        split2(__uint_as_float(__float_as_uint(va[2].y) & aok[NC - 1][2]), __uint_as_float(__float_as_uint(va[3].y) & aok[NC - 1][3]), hi);
+#pragma unroll
+        for (int p = 0; p < kPlanes; ++p) a2[p * PA * 2 + wb] = make_uint2(lo[p], hi[p]);
+        uint4 d[kPlanes];
+        split8(vd, d);
+        if (BN == 128 || dput) {
+#pragma unroll
+            for (int p = 0; p < kPlanes; ++p) buf[kPlanes * PA + p * PD + wd] = d[p];
         }
+    };
+    // Column sums of dY, from the workgroups of the first k tile: the rows that
+    // are about to be split, once a stage (a uniform branch of its own, outside
+    // the scheduled parts).
+    const bool summing = sums != nullptr && k0 == 0;
+    float bs = 0.0f;
+    auto add_rows = [&](int ms) {
+        if (!summing) return;
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = ms + 8 * md + q < mend ? vd[q] : 0.0f;
+        bs += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
     };
     f32x16 acc[2][UT], cor[2][UT];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int u = 0; u < UT; ++u) acc[t][u] = cor[t][u] = (f32x16){};
-    const int fr = lane & 31, fh = lane >> 5;
-    const int nst = (mend - mbeg + kWgM - 1) / kWgM;
-    const int sa = slot(wk * 64 + fr, fh), sd = slot(wn * (BN / 2) + fr, fh);
-    if (nst > 0) load(mbeg);
-    for (int st = 0; st < nst; ++st) {
-        if (st) __syncthreads();  // the stage before has been read
-        put8(As + slot(2 * lane, ws), PA, {keep(va[0].x, aok[0][0]), keep(va[1].x, aok[0][1]), keep(va[2].x, aok[0][2]),
-                                       keep(va[3].x, aok[0][3]), keep(va[4].x, aok[0][4]), keep(va[5].x, aok[0][5]),
-                                       keep(va[6].x, aok[0][6]), keep(va[7].x, aok[0][7])});
-        put8(As + slot(2 * lane + 1, ws), PA, {keep(va[0].y, aok[NC - 1][0]), keep(va[1].y, aok[NC - 1][1]), keep(va[2].y, aok[NC - 1][2]),
-                                           keep(va[3].y, aok[NC - 1][3]), keep(va[4].y, aok[NC - 1][4]), keep(va[5].y, aok[NC - 1][5]),
-                                           keep(va[6].y, aok[NC - 1][6]), keep(va[7].y, aok[NC - 1][7])});
-        if (dput) {
-            put8(Ds + slot(2 * pn, dg), PD, {vd[0].x, vd[1].x, vd[2].x, vd[3].x, vd[4].x, vd[5].x, vd[6].x, vd[7].x});
-            put8(Ds + slot(2 * pn + 1, dg), PD, {vd[0].y, vd[1].y, vd[2].y, vd[3].y, vd[4].y, vd[5].y, vd[6].y, vd[7].y});
-        }
-        load(mbeg + min(st + 1, nst - 1) * kWgM);  // the last one again: harmless, and no branch
+
+    // Stages of 16 rows in three buffers: while stage s is computed, stage s + 2
+    // is split and written to the buffer that stage s - 1 left, the fragments of
+    // stage s + 1 are read and the rows of stage s + 3 loaded, all between the
+    // MFMAs (sched), with one barrier a stage.  Planes 1 and 2 of A and 0 and 1
+    // of dY are in registers when the stage begins (dY's in two sets, as both
+    // halves of a stage use them); the others are read during the first half.
+    const int sa = stage_slot(wk * 64 + fr, fh), sd = stage_slot(wn * (BN / 2) + fr, fh);
+    uint4 a[kPlanes][2], d2[UT], ds[2][2][UT];
+    auto frag_a = [&](const uint4* buf, int p) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) a[p][t] = buf[p * PA + 32 * t * kStage4 + sa];
+    };
+    auto frag_d = [&](const uint4* buf, int p, uint4 (&d)[UT]) {
+#pragma unroll
+        for (int u = 0; u < UT; ++u) d[u] = buf[kPlanes * PA + p * PD + 32 * u * kStage4 + sd];
+    };
+    auto mul = [&](int i, const uint4 (&d)[UT], f32x16 (&o)[2][UT]) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int u = 0; u < UT; ++u)
+                o[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[i][t]),
+                    __builtin_bit_cast(bf16x8, d[u]), o[t][u], 0, 0, 0);
+    };
+    const int nst = (mend - mbeg + kStage - 1) / kStage;
+    auto row = [&](int s) { return mbeg + min(s, nst - 1) * kStage; };  // past the last: a harmless reload
+    uint4 *b0 = lds, *b1 = lds + kBuf, *b2 = lds + 2 * kBuf;
+    auto stage = [&](int s, const uint4 (&d)[2][UT], uint4 (&dn)[2][UT]) {
+        add_rows(mbeg + (s + 2) * kStage);  // past the last stage: no rows
+        frag_a(b0, 0);
+        frag_d(b0, 2, d2);
+        mul(2, d[0], cor);
+        mul(1, d[1], cor);
+        mul(1, d[0], cor);
+        store(b2);
+        sched<6 * UT, 8>();
+        __builtin_amdgcn_sched_barrier(0);
+        frag_a(b1, 2);
+        frag_a(b1, 1);
+        frag_d(b1, 0, dn[0]);
+        frag_d(b1, 1, dn[1]);
+        load(row(s + 3));  // into the registers just split
+        mul(0, d2, cor);
+        mul(0, d[1], cor);
+        mul(0, d[0], acc);
+        sched<6 * UT>();
+        __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            uint4 a[kPlanes][2], d[kPlanes][UT];
-#pragma unroll
-            for (int p = 0; p < kPlanes; ++p) {
-#pragma unroll
-                for (int t = 0; t < 2; ++t) a[p][t] = As[p * PA + 32 * t * kRow4 + (sa ^ 2 * ks)];
-#pragma unroll
-                for (int u = 0; u < UT; ++u) d[p][u] = Ds[p * PD + 32 * u * kRow4 + (sd ^ 2 * ks)];
-            }
-            products<2, UT>(a, d, acc, cor);
+        uint4* t = b0;
+        b0 = b1;
+        b1 = b2;
+        b2 = t;
+    };
+    if (nst > 0) {
+        load(row(0));
+        add_rows(mbeg);
+        store(b0);
+        load(row(1));
+        add_rows(mbeg + kStage);
+        store(b1);
+        load(row(2));
+        __syncthreads();
+        frag_a(b0, 2);
+        frag_a(b0, 1);
+        frag_d(b0, 0, ds[0][0]);
+        frag_d(b0, 1, ds[0][1]);
+        for (int s = 0;;) {
+            stage(s, ds[0], ds[1]);
+            if (++s == nst) break;
+            stage(s, ds[1], ds[0]);
+            if (++s == nst) break;
         }
     }
 #pragma unroll
@@ -620,7 +715,7 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
         bool ck[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const int k = k0 + wk * 64 + 32 * t + fr;
+            const int k = k0 + 2 * (32 * t + fr) + wk;  // the column of tile row wk 64 + 32 t + fr
             ck[t] = k < sh.KKC;
             tp[t] = ck[t] ? k / sh.Cin : 0;
             cc[t] = ck[t] ? k - tp[t] * sh.Cin : 0;
@@ -654,23 +749,34 @@ __global__ __launch_bounds__(kTpb, 2) void igemm_wgrad(float* __restrict__ part,
                     acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[t], dv[u], acc[t][u], 0, 0, 0);
         }
     }
-    // partial tile (columns past the end are not stored): D[k][n], rows k = k0 + wk 64 + 32 t + 8 (r / 4) + 4 h + r % 4
-    float* pb = part + (size_t)z * sh.KKC * sh.Cout + (size_t)(k0 + wk * 64 + 4 * fh) * sh.Cout + n0 + wn * (BN / 2) + fr;
+    // partial tile: D[row][n], rows 32 t + 8 (r / 4) + 4 fh + r % 4 of the wave's
+    // 64, which hold the even (wk = 0) or odd columns k; past the end nothing is
+    // stored
+    float* pb = part + z * stride + n0 + wn * (BN / 2) + fr;
 #pragma unroll
     for (int u = 0; u < UT; ++u)
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int dk = 32 * t + 8 * (r >> 2) + (r & 3);
-                if (k0 + wk * 64 + 4 * fh + dk < sh.KKC && n0 + wn * (BN / 2) + 32 * u + fr < sh.Cout)
-                    pb[(size_t)dk * sh.Cout + 32 * u] = acc[t][u][r];
+                const int k = k0 + 2 * (32 * t + 8 * (r >> 2) + 4 * fh + (r & 3)) + wk;
+                if (k < sh.KKC && n0 + wn * (BN / 2) + 32 * u + fr < sh.Cout)
+                    pb[(size_t)k * sh.Cout + 32 * u] = acc[t][u][r];
             }
+    if (summing) {
+        // the two halves of the rows, in order (the tile loop left LDS behind its barrier)
+        float* l = reinterpret_cast<float*>(lds);
+        if (dput) l[tid] = bs;
+        __syncthreads();
+        if (tid < BN && n0 + tid < sh.Cout) sums[z * stride + n0 + tid] = l[tid] + l[tid + BN];
+    }
 }
 
-// gW[i] = part[0][i] + part[1][i] + ... (split order).
-__global__ __launch_bounds__(256) void wgrad_reduce(float* __restrict__ gW, const float* __restrict__ part, int S,
-    long long n) {
+// out[i] = part[0][i] + part[1][i] + ... (split order), n elements a split, of
+// which those from nw on (the column sums of dY, where they were asked for) go
+// to gb.
+__global__ __launch_bounds__(256) void wgrad_reduce(float* __restrict__ gW, float* __restrict__ gb,
+    const float* __restrict__ part, int S, long long n, long long nw) {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     // kB slices in flight, added in slice order
@@ -685,14 +791,18 @@ __global__ __launch_bounds__(256) void wgrad_reduce(float* __restrict__ gW, cons
         for (int u = 0; u < kB; ++u) t += v[u];
     }
     for (; z < S; ++z) t += part[(size_t)z * n + i];
-    gW[i] = t;
+    if (i < nw) gW[i] = t;
+    else gb[i - nw] = t;
 }
 
-// The same for many slices of few elements (S beyond kTallS): 16 waves share
-// the slices of 64 elements, eight in flight each, and add their sums in order.
+// The same for many slices (S beyond kTallS) of few elements (up to kTallN): 16
+// waves share the slices of 64 elements, eight in flight each, and add their
+// sums in order.  [27, 64] in 512 slices: 32 -> 5 us; at [1152, 128] in 56 the
+// elements alone fill the device, 7.6 us against 10.6.
 constexpr int kTallS = 24;
-__global__ __launch_bounds__(1024) void wgrad_reduce_tall(float* __restrict__ gW, const float* __restrict__ part, int S,
-    long long n) {
+constexpr long long kTallN = 32768;
+__global__ __launch_bounds__(1024) void wgrad_reduce_tall(float* __restrict__ gW, float* __restrict__ gb,
+    const float* __restrict__ part, int S, long long n, long long nw) {
     __shared__ float l[16][kWave];
     const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     const long long i = (long long)blockIdx.x * kWave + lane;
@@ -715,7 +825,8 @@ __global__ __launch_bounds__(1024) void wgrad_reduce_tall(float* __restrict__ gW
         float a = l[0][lane];
 #pragma unroll
         for (int w = 1; w < 16; ++w) a += l[w][lane];
-        gW[i] = a;
+        if (i < nw) gW[i] = a;
+        else gb[i - nw] = a;
     }
 }
 
@@ -743,17 +854,17 @@ inline WgradPlan wgrad_plan(int M, int KKC, int Cout) {
 
 // Whether the small tiles beat the tiled kernel, by times in us that fit the
 // sweep of conv_tile: the small tiles are bound by round trips or by their
-// vector work, the tiled kernel takes a stage's time for the stages of a split,
-// then the sum of the splits (and the column sums a launch of their own).  For
-// example [8, 7 x 7, 128 -> 128]: small 8.1, tiled 16.5 us; dense [128, 512 ->
-// 512]: 6.0, 13.3; [8, 28 x 28, 32 -> 32]: 61, 19; [16, 16 x 16, 256 -> 256]: 118,
-// 53.
+// vector work, the tiled kernel takes a time for every 32 rows of a split, then
+// the sum of the splits.  For example [8, 7 x 7, 128 -> 128]: small 8.2, tiled 17
+// us; dense [128, 512 -> 512]: 4.9, 14; [8, 28 x 28, 32 -> 32]: 59, 19; [16, 16 x
+// 16, 256 -> 256]: 113, 50.
 inline bool wgrad_small_wins(const ConvShape& sh) {
     const double steps = (sh.M + 15) / 16, cells = (double)((sh.KKC + 31) / 32) * ((sh.Cout + 31) / 32);
-    const double waves = steps <= 8 ? 4 : steps <= 24 ? 8 : 16;
-    const double trips = 2.3 * ceil(steps / waves), work = 0.00078 * cells * steps;
+    const double waves = steps <= 4 ? 4 : steps <= 16 ? 8 : 16;
+    const bool dense = sh.K == 1 && sh.stride == 1 && sh.pad == 0;  // no pixels to decode
+    const double trips = (dense ? 0.9 : 2.3) * ceil(steps / waves), work = (dense ? 0.0005 : 0.00078) * cells * steps;
     const WgradPlan p = wgrad_plan(sh.M, sh.KKC, sh.Cout);
-    const double stage = tile_n(sh.Cout) == 128 ? 3.3 : 2.0;
+    const double stage = tile_n(sh.Cout) == 128 ? 3.0 : 2.0;
     return 4.0 + (trips > work ? trips : work) < 12.0 + stage * (p.rows / kWgM);
 }
 
@@ -804,32 +915,49 @@ inline int dgrad_setup(const char* what, const float* dX, const float* dY, const
     return 1;
 }
 
-// The tiled weight gradient of a checked, non-empty shape.
-inline void wgrad_run(const char* what, float* gW, const float* X, const float* dY, const ConvShape& sh,
+// The tiled weight gradient of a checked, non-empty shape, and with gb non-null
+// the column sums of dY.
+inline void wgrad_run(const char* what, float* gW, float* gb, const float* X, const float* dY, const ConvShape& sh,
     float* workspace, hipStream_t s) {
     const WgradPlan p = wgrad_plan(sh.M, sh.KKC, sh.Cout);
-    float* part = gW;
+    const long long nw = (long long)sh.KKC * sh.Cout, n = nw + (gb ? sh.Cout : 0);
+    float *part = gW, *sums = gb;
     bool pooled = false;
     if (p.S > 1) {
         if (workspace) {
             part = workspace;
         } else {
-            part = nnk_scratch_acquire((size_t)p.S * sh.KKC * sh.Cout, s, what);
+            part = nnk_scratch_acquire((size_t)p.S * n, s, what);
             if (!part) return;
             pooled = true;
         }
+        if (gb) sums = part + nw;
     }
     const int BN = tile_n(sh.Cout);
     const dim3 grid((unsigned)((sh.KKC + 127) / 128) * (unsigned)((sh.Cout + BN - 1) / BN) * (unsigned)p.S);
-    const bool pairs = sh.Cin % 2 == 0 && sh.Cout % 2 == 0 && (uintptr_t)X % 8 == 0 && (uintptr_t)dY % 8 == 0;
-    if (BN == 128 && pairs) igemm_wgrad<128, false><<<grid, kTpb, 0, s>>>(part, X, dY, sh, p.rows);
-    else if (BN == 128) igemm_wgrad<128, true><<<grid, kTpb, 0, s>>>(part, X, dY, sh, p.rows);
-    else if (pairs) igemm_wgrad<64, false><<<grid, kTpb, 0, s>>>(part, X, dY, sh, p.rows);
-    else igemm_wgrad<64, true><<<grid, kTpb, 0, s>>>(part, X, dY, sh, p.rows);
+    const int loads = sh.Cin % 2 || (uintptr_t)X % 8 ? kSingles : sh.Wo % 4 ? kPairs : kQuads;
+    const size_t lds = (size_t)3 * kPlanes * (128 + BN) * kStage4 * sizeof(uint4);
+#define NNK_WGRAD(BN_, LOADS_)                                                                                 \
+    do {                                                                                                       \
+        static const hipError_t once = hipFuncSetAttribute((const void*)igemm_wgrad<BN_, LOADS_>,              \
+            hipFuncAttributeMaxDynamicSharedMemorySize, 81920);                                                \
+        (void)once;                                                                                            \
+        igemm_wgrad<BN_, LOADS_><<<grid, kTpb, lds, s>>>(part, sums, (size_t)n, X, dY, sh, p.rows);            \
+    } while (0)
+#define NNK_WGRAD_LOADS(BN_)                            \
+    do {                                                \
+        if (loads == kQuads) NNK_WGRAD(BN_, kQuads);    \
+        else if (loads == kPairs) NNK_WGRAD(BN_, kPairs); \
+        else NNK_WGRAD(BN_, kSingles);                  \
+    } while (0)
+    if (BN == 128) NNK_WGRAD_LOADS(128);
+    else NNK_WGRAD_LOADS(64);
+#undef NNK_WGRAD_LOADS
+#undef NNK_WGRAD
     if (p.S > 1) {
-        const long long n = (long long)sh.KKC * sh.Cout;
-        if (p.S > kTallS) wgrad_reduce_tall<<<(unsigned)((n + kWave - 1) / kWave), 1024, 0, s>>>(gW, part, p.S, n);
-        else wgrad_reduce<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(gW, part, p.S, n);
+        if (p.S > kTallS && n <= kTallN)
+            wgrad_reduce_tall<<<(unsigned)((n + kWave - 1) / kWave), 1024, 0, s>>>(gW, gb, part, p.S, n, nw);
+        else wgrad_reduce<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(gW, gb, part, p.S, n, nw);
     }
     if (pooled) nnk_scratch_release(part, s);
 }
@@ -854,7 +982,7 @@ inline void wgrad_launch(const char* what, float* gW, const float* X, const floa
     ConvShape sh{batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, batch * H_out * W_out, KKC,
         FastDiv((uint32_t)W_out), FastDiv((uint32_t)H_out)};
     if (wgrad_small_wins(sh)) nnk_wgrad_small(gW, nullptr, X, dY, sh, s);
-    else wgrad_run(what, gW, X, dY, sh, workspace, s);
+    else wgrad_run(what, gW, nullptr, X, dY, sh, workspace, s);
     nnk_after_launch(what, s);
 }
 

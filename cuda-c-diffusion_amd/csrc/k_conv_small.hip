@@ -161,7 +161,8 @@ __global__ __launch_bounds__(64 * WAVES) void conv_small(float* __restrict__ Y, 
 // gW[k, n] = sum_m A[m, k] dY[m, n], A gathered from X; gb[n] = sum_m dY[m, n]
 // from the workgroups of the first k tile.  A step is 16 rows m; all loads are
 // 4 bytes a lane along k and n, so any channel counts and alignments do.
-template <int WAVES>
+// DENSE: 1 x 1, stride 1, no padding: the input pixel is the output pixel.
+template <int WAVES, bool DENSE>
 __global__ __launch_bounds__(64 * WAVES) void wgrad_small(float* __restrict__ gW, float* __restrict__ gb,
     const float* __restrict__ X, const float* __restrict__ dY, ConvShape sh) {
     __shared__ float lds[WAVES * kT * kT];
@@ -184,6 +185,16 @@ __global__ __launch_bounds__(64 * WAVES) void wgrad_small(float* __restrict__ gW
     Ops o[kAhead];
     auto load = [&](Ops& r, int s) {
         int m = 16 * s + 8 * fh;
+        if constexpr (DENSE) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t mm = (uint32_t)min(m + i, sh.M - 1);
+                r.in[i] = m + i < sh.M;
+                r.va[i] = X[mm * (uint32_t)sh.Cin + (uint32_t)ci];
+                r.vd[i] = dY[mm * (uint32_t)sh.Cout + (uint32_t)nc];
+            }
+            return;
+        }
         uint32_t q, ow, b, oh;
         sh.wo.divmod((uint32_t)min(m, sh.M - 1), q, ow);
         sh.ho.divmod(q, b, oh);
@@ -256,9 +267,8 @@ __global__ __launch_bounds__(64 * WAVES) void wgrad_small(float* __restrict__ gW
     }
 }
 
-// Waves by the steps of a tile: about two steps each, while loads of more waves
-// in flight shorten a tile's time.
-int waves_for(int steps) { return steps <= 8 ? 4 : steps <= 24 ? 8 : 16; }
+// Waves by the steps of a tile: one or two steps each.
+int waves_for(int steps) { return steps <= 4 ? 4 : steps <= 16 ? 8 : 16; }
 
 }  // namespace
 
@@ -288,7 +298,14 @@ void nnk_conv_small(bool flip, int xe, float* Y, const float* X, const float* Wt
 void nnk_wgrad_small(float* gW, float* gb, const float* X, const float* dY, const ConvShape& sh, hipStream_t s) {
     const unsigned grid = (unsigned)((sh.KKC + kT - 1) / kT) * (unsigned)((sh.Cout + kT - 1) / kT);
     const int waves = waves_for((sh.M + 15) / 16);
-    if (waves == 4) wgrad_small<4><<<grid, 256, 0, s>>>(gW, gb, X, dY, sh);
-    else if (waves == 8) wgrad_small<8><<<grid, 512, 0, s>>>(gW, gb, X, dY, sh);
-    else wgrad_small<16><<<grid, 1024, 0, s>>>(gW, gb, X, dY, sh);
+    const bool dense = sh.K == 1 && sh.stride == 1 && sh.pad == 0;
+#define NNK_WSMALL(W_)                                                                             \
+    do {                                                                                           \
+        if (dense) wgrad_small<W_, true><<<grid, 64 * W_, 0, s>>>(gW, gb, X, dY, sh);              \
+        else wgrad_small<W_, false><<<grid, 64 * W_, 0, s>>>(gW, gb, X, dY, sh);                   \
+    } while (0)
+    if (waves == 4) NNK_WSMALL(4);
+    else if (waves == 8) NNK_WSMALL(8);
+    else NNK_WSMALL(16);
+#undef NNK_WSMALL
 }

@@ -20,8 +20,10 @@
 // vendor library holds 1250 TFLOP/s, because the clock falls to 1.7 GHz under
 // that load, so 208 is what to expect.  Measured: cfg3 forward (3x3, 128 -> 128,
 // [128, 32, 32]) 320 -> 191 us (202 TFLOP/s), 256 -> 256 at [16, 64, 64] 627 ->
-// 351 us (220), their input gradients 317 -> 193 and 620 -> 359 us; the matrix
-// cores are busy 0.69 of the time at 1.67 GHz.  On the way: the fp32 kernel's
+// 351 us (220), their input gradients 317 -> 193 and 620 -> 359 us, their weight
+// gradients 337 -> 254 and 657 -> 454 us; the forward's matrix cores are busy 0.69
+// of the time at 1.67 GHz, the weight gradient's 0.46 (it splits each operand
+// again in all nine k tiles, and decodes pixels).  On the way: the fp32 kernel's
 // staging (both operands through LDS per tap, a split of each) 230-260 us;
 // activations staged once per 32 channels for all taps, weights split in
 // registers by the one wave that needs them 205-214; the next step's loads and
@@ -135,7 +137,7 @@ size_t nnk_conv_weight_grad_workspace(int batch, int C_in, int C_out, int K, int
     const long long M = (long long)batch * H_out * W_out;
     if (M <= 0 || M >= (1LL << 31)) return 0;
     const WgradPlan p = wgrad_plan((int)M, K * K * C_in, C_out);
-    return p.S > 1 ? (size_t)p.S * K * K * C_in * C_out : 0;
+    return p.S > 1 ? (size_t)p.S * (K * K * C_in + 1) * C_out : 0;
 }
 
 void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy, int batch, int H, int W, int C_in,
@@ -152,12 +154,8 @@ void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy,
         FastDiv((uint32_t)W_out), FastDiv((uint32_t)H_out)};
     // a capture may not need scratch that the stream does not have: without a
     // workspace it takes the small tiles, which need none
-    if (wgrad_small_wins(sh) || (!workspace && nnk_capturing(s))) {
-        nnk_wgrad_small(gw, gb, x, dy, sh, s);
-    } else {
-        wgrad_run(what, gw, x, dy, sh, workspace, s);
-        if (gb) launch_bias_grad(gb, dy, sh.M, C_out, s);
-    }
+    if (wgrad_small_wins(sh) || (!workspace && nnk_capturing(s))) nnk_wgrad_small(gw, gb, x, dy, sh, s);
+    else wgrad_run(what, gw, gb, x, dy, sh, workspace, s);
     nnk_after_launch(what, s);
 }
 
