@@ -63,8 +63,18 @@ __device__ __forceinline__ void split8(const float (&v)[8], uint4 (&p)[kPlanes])
 }
 __device__ __forceinline__ float keep(float v, bool ok) { return __uint_as_float(__float_as_uint(v) & (ok ? ~0u : 0u)); }
 
-// A wave's products over 16 k: T x U accumulators of 32 x 32 from the planes of
-// its row tiles' fragments (lane l: row l % 32, k 8 (l / 32) .. + 7).  The
+// d += a b over the k of a fragment of 8 k a lane: 16 k and a tile of 32 x 32
+// (lane l: row l % 32, k 8 (l / 32) .. + 7), or 32 k and 16 x 16 (row l % 16, k 8
+// (l / 16) .. + 7).
+__device__ __forceinline__ void mfma(const uint4& a, const uint4& b, f32x16& d) {
+    d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), d, 0, 0, 0);
+}
+__device__ __forceinline__ void mfma(const uint4& a, const uint4& b, f32x4& d) {
+    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), d, 0, 0, 0);
+}
+
+// A wave's products over a fragment's k: T x U accumulators from the planes of
+// its row tiles' fragments.  The
 // matrix core cuts off what an addend has below the last place of the largest
 // one, towards minus infinity.  p0 q0 products lie on a coarse grid and lose
 // next to nothing; the five small products, added to the same accumulator,
@@ -75,28 +85,24 @@ __device__ __forceinline__ float keep(float v, bool ok) { return __uint_as_float
 // normal operands, against 5.2e-7 (mean -6e-8) with one accumulator and 6.1e-7
 // with the fp32 MFMA.  Each product runs over all T x U accumulators, so
 // consecutive MFMAs rarely wait for each other's result.
-template <int T, int U>
-__device__ __forceinline__ void products(const uint4 (&a)[kPlanes][T], const uint4 (&b)[kPlanes][U],
-    f32x16 (&acc)[T][U], f32x16 (&cor)[T][U]) {
+template <int T, int U, class V>
+__device__ __forceinline__ void products(const uint4 (&a)[kPlanes][T], const uint4 (&b)[kPlanes][U], V (&acc)[T][U],
+    V (&cor)[T][U]) {
     constexpr int PI[6] = {0, 2, 0, 1, 1, 0}, PJ[6] = {0, 0, 2, 1, 0, 1};
 #pragma unroll
     for (int x = 0; x < 6; ++x)
 #pragma unroll
         for (int t = 0; t < T; ++t)
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                f32x16& d = x ? cor[t][u] : acc[t][u];
-                d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[PI[x]][t]),
-                    __builtin_bit_cast(bf16x8, b[PJ[x]][u]), d, 0, 0, 0);
-            }
+            for (int u = 0; u < U; ++u) mfma(a[PI[x]][t], b[PJ[x]][u], x ? cor[t][u] : acc[t][u]);
 }
 
 // Whether a wave's results must be formed again from the unsplit operands: a
 // value that is not finite (an infinite or NaN operand, or one that rounds to
 // infinity in bf16, splits into NaN planes), or values all so small that an
 // operand may lie below the split's range.
-template <int T, int U>
-__device__ __forceinline__ bool split_failed(const f32x16 (&acc)[T][U]) {
+template <int T, int U, class V>
+__device__ __forceinline__ bool split_failed(const V (&acc)[T][U]) {
     bool bad = false;
     float mx = 0.0f;
 #pragma unroll
@@ -104,7 +110,7 @@ __device__ __forceinline__ bool split_failed(const f32x16 (&acc)[T][U]) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
+            for (int r = 0; r < (int)(sizeof(V) / sizeof(float)); ++r) {
                 const float v = fabsf(acc[t][u][r]);
                 bad |= !(v <= 3.402823466e38f);
                 mx = fmaxf(mx, v);
@@ -149,6 +155,28 @@ __device__ __forceinline__ void epilogue_store(float* __restrict__ Y, float v, i
         const float z = act_fwd<ACT_SILU, false>(v * (ep.cond[co] + 1.0f));
         ep.y2[o] = ep.mp ? z * kMpSiluScale : z;
     }
+}
+
+// Waves of a small tile by its steps: one or two steps each.
+inline int waves_for(int steps) { return steps <= 4 ? 4 : steps <= 16 ? 8 : 16; }
+
+// The time of the small tiles of t x t outputs, in us, as fitted to the sweep of
+// conv_tile.  Tiles of 16 take 32 k a step and spread over four times the
+// workgroups, so they win while a wave's round trips of loads count, and lose
+// with twice the vector work per output where that does.  32 / 16 measured:
+// forward [8, 7 x 7, 128 -> 128] 9.3 / 6.2, its input gradient 11.6 / 6.9; [1, 8 x
+// 8, 448 -> 448] 22 / 14; dense [128, 512 -> 512] 6.2 / 4.9, [1024, 256 -> 256] 5.2
+// / 6.7; [8, 28 x 28, 32 -> 32] 5.4 / 6.4; [4, 16 x 16, 256 -> 256] 16 / 25; 5x5
+// input gradient 320 -> 4 at [22, 5, 8] 37 / 21.
+inline double small_us(const ConvShape& sh, bool flip, int t) {
+    const bool t32 = t == 32;
+    const int sk = 512 / t, steps = sh.K * sh.K * ((sh.Cin + sk - 1) / sk);
+    const double cells = (double)((sh.M + t - 1) / t) * ((sh.Cout + t - 1) / t);
+    const double trips = (t32 ? 1.15 : flip ? 1.3 : 1.2) * ((steps + waves_for(steps) - 1) / waves_for(steps));
+    double step = flip ? t32 ? 0.00045 : 0.00040 : t32 ? 0.00036 : 0.00031;
+    if (sh.Cin % 8) step *= 1.8;  // one element a load
+    const double work = cells * (steps * step + (t32 ? 0.005 : 0.0015));
+    return (t32 ? 3.8 : 3.5) + (trips > work ? trips : work);
 }
 
 }  // namespace conv

@@ -416,32 +416,35 @@ inline int conv_mode(const ConvShape& sh, const float* X, const float* Wt, bool 
 
 // Columns per workgroup of the tiled kernels, or 0 for the small tiles: the
 // least of the times, in us, that fit a sweep of 23 shapes (1x1 to 5x5, 3 to
-// 1024 channels, 3 to 131072 rows).  A tiled workgroup by itself takes `lone` us
-// per slice of 32 channels and tap, and the device `full` us per slice and tile;
-// the small tiles are bound by a wave's round trips of loads or by their vector
-// work (which a flipped weight's scattered rows lengthen).  For example, forward
-// at [8, 7 x 7, 128 -> 128]: small 9.3, 32 / 64 / 128 columns 25 / 33 / 46; [64, 8
-// x 8, 448 -> 448]: 180, 117 / 107 / 138; [20, 40 x 40, 80 -> 200]: 177, 88 / 81 /
+// 1024 channels, 3 to 131072 rows).  A tiled workgroup by itself takes 0.75 us to
+// stage a slice of 32 channels and `lone` us for each of its taps; the filled
+// device 0.0014 us for a slice, `full` for a tap and 0.005 for the rest of each
+// tile.  The small tiles (small_us) are bound by a wave's round trips of loads or by
+// their vector work (which a flipped weight's scattered rows lengthen).  Forward
+// at [8, 7 x 7, 128 -> 128]: small 6.2, 32 / 64 / 128 columns 25 / 33 / 46; [64, 8
+// x 8, 448 -> 448]: 169, 111 / 103 / 138; [20, 40 x 40, 80 -> 200]: 177, 88 / 81 /
 // 74; [4, 16 x 16, 256 -> 256]: 15, 45 / 59 / 80; [16, 16 x 16, 256 -> 256]: 56,
 // 46 / 59 / 80.
-inline int conv_tile(const ConvShape& sh, bool flip) {
+inline int conv_tile(const ConvShape& sh, bool flip, double* best_us = nullptr) {
     struct Tile {
         int bn;
         double lone, full;
     };
-    constexpr Tile kTiles[] = {{128, 1.15, 0.0050}, {64, 0.82, 0.0027}, {32, 0.62, 0.0017}};
+    const Tile kTiles[] = {{128, 1.07, 0.00485}, {64, 0.74, 0.00255}, {32, 0.54, flip ? 0.00195 : 0.00175}};
     const double KK = (double)sh.K * sh.K;
-    const double steps = KK * ((sh.Cin + 15) / 16), slices = KK * ((sh.Cin + 31) / 32);
-    const double cells = (double)((sh.M + 31) / 32) * ((sh.Cout + 31) / 32);
-    const double waves = steps <= 4 ? 4 : steps <= 16 ? 8 : 16;
-    const double trips = 1.15 * ceil(steps / waves), work = (flip ? 0.00050 : 0.00041) * cells * steps;
-    double best = 3.5 + (trips > work ? trips : work);
+    const double slices = (sh.Cin + 31) / 32;
+    const double s16 = small_us(sh, flip, 16), s32 = small_us(sh, flip, 32);
+    double best = s16 < s32 ? s16 : s32;
     int bn = 0;
     for (const Tile& t : kTiles) {
         const double tiles = (double)((sh.M + kBM - 1) / kBM) * ((sh.Cout + t.bn - 1) / t.bn);
-        const double us = 5.0 + slices * (t.lone > t.full * tiles ? t.lone : t.full * tiles);
+        // 128 columns reach the full rate with two workgroups on each CU only
+        const double lone = slices * (0.75 + KK * t.lone);
+        const double full = tiles * (slices * (0.0014 + KK * t.full) + 0.005) * (t.bn == 128 && tiles < 512 ? 1.16 : 1.0);
+        const double us = 5.0 + (lone > full ? lone : full);
         if (us < best) best = us, bn = t.bn;
     }
+    if (best_us) *best_us = best;
     return bn;
 }
 
@@ -860,7 +863,7 @@ inline WgradPlan wgrad_plan(int M, int KKC, int Cout) {
 // 16, 256 -> 256]: 113, 50.
 inline bool wgrad_small_wins(const ConvShape& sh) {
     const double steps = (sh.M + 15) / 16, cells = (double)((sh.KKC + 31) / 32) * ((sh.Cout + 31) / 32);
-    const double waves = steps <= 4 ? 4 : steps <= 16 ? 8 : 16;
+    const double waves = waves_for((int)steps);
     const bool dense = sh.K == 1 && sh.stride == 1 && sh.pad == 0;  // no pixels to decode
     const double trips = (dense ? 0.9 : 2.3) * ceil(steps / waves), work = (dense ? 0.0005 : 0.00078) * cells * steps;
     const WgradPlan p = wgrad_plan(sh.M, sh.KKC, sh.Cout);

@@ -1,23 +1,26 @@
 // k_conv_small.hip -- convolutions and dense layers (a convolution of one pixel)
-// with few output tiles: 32 x 32 outputs a workgroup, whose waves share the k
-// range, so that a few hundred rows still spread over the device.  The tiled
-// kernels (igemm.h) put the reference DDPM's 7 x 7 x 128 level (392 rows) on
+// with few output tiles: 32 x 32 or 16 x 16 outputs a workgroup, whose waves share
+// the k range, so that a few hundred rows still spread over the device.  The
+// tiled kernels (igemm.h) put the reference DDPM's 7 x 7 x 128 level (392 rows) on
 // four workgroups.
 //
-// A wave loads the fragments of its steps of 16 k straight from memory (lane l:
-// row or column l % 32, k 8 (l / 32) .. + 7), a step ahead, splits both operands
-// in registers and adds up its part of the tile; the parts are added in wave
-// order through LDS and go through the epilogue, so one launch does all and
-// nothing is kept in memory between.  Both operands are split per 32 x 32 tile,
-// four times as often as in the tiled kernels: ~90 vector instructions beside 6
-// MFMAs a step bound it, at about half the tiled kernels' full rate, but from
-// the first workgroup on.  The rules between the two are conv_tile and
-// wgrad_small_wins (igemm.h).
+// A wave loads the fragments of its steps of 16 or 32 k straight from memory
+// (eight k of a row or column a lane), a step ahead, splits both operands in
+// registers and adds up its part of the tile; the parts are added in wave order
+// through LDS and go through the epilogue, so one launch does all and nothing is
+// kept in memory between.  Both operands are split per tile, four times as often
+// as in the tiled kernels (eight with tiles of 16): ~90 vector instructions beside
+// 6 MFMAs a step bound it, at about half the tiled kernels' full rate, but from
+// the first workgroup on; with few tiles, the round trips of loads.  The rules
+// between them are small_us (conv_common.h), conv_tile and wgrad_small_wins
+// (igemm.h).
 // Against im2col, rocBLAS and the bias pass at [8, 7 x 7, 128 -> 128]: forward 17 ->
-// 9.3 us, input gradient 12 -> 11.6, weight gradient with the bias gradient 30 ->
-// 8.1; dense [128, 512 -> 512] with bias 8 -> 6.2, its weight and bias gradients 11
-// -> 6.0.
+// 6.2 us, input gradient 12 -> 6.9, weight gradient with the bias gradient 30 ->
+// 8.2; dense [128, 512 -> 512] with bias 8 -> 4.9, its weight and bias gradients 11
+// -> 4.9.
 #include "conv_common.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -30,34 +33,46 @@ constexpr int kT = 32;     // tile edge
 constexpr int kAhead = 1;
 
 // Parts in LDS, [wave][row][column]; accumulator register r of lane l holds row
-// 8 (r / 4) + 4 (l / 32) + r % 4 of column l % 32.
-__device__ __forceinline__ void put_part(float* lds, int w, int fr, int fh, const f32x16& v) {
+// 8 (r / 4) + 4 (l / 32) + r % 4 of column l % 32 (tiles of 16: row 4 (l / 16) + r
+// of column l % 16).
+template <int T, class V>
+__device__ __forceinline__ void put_part(float* lds, int w, int fr, int fh, const V& v) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) lds[w * kT * kT + (8 * (r >> 2) + 4 * fh + (r & 3)) * kT + fr] = v[r];
+    for (int r = 0; r < T * T / 64; ++r) lds[w * T * T + (8 * (r >> 2) + 4 * fh + (r & 3)) * T + fr] = v[r];
 }
 
 // the sum of the waves' parts of element i, in wave order
-template <int WAVES>
+template <int T, int WAVES>
 __device__ __forceinline__ float sum_parts(const float* lds, int i) {
     float v = lds[i];
 #pragma unroll
-    for (int q = 1; q < WAVES; ++q) v += lds[q * kT * kT + i];
+    for (int q = 1; q < WAVES; ++q) v += lds[q * T * T + i];
     return v;
+}
+
+// fp32 products of 2 k (tiles of 32) or 4 k (tiles of 16), one a lane
+__device__ __forceinline__ void mfma_f32(float a, float b, f32x16& d) {
+    d = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, d, 0, 0, 0);
+}
+__device__ __forceinline__ void mfma_f32(float a, float b, f32x4& d) {
+    d = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, d, 0, 0, 0);
 }
 
 // VEC: channel counts are multiples of 8 and the pointers 16-byte aligned, so
 // that 8 k of a pixel (and of a flipped weight's row) are two 16-byte loads.
-template <int WAVES, bool FLIP, bool VEC>
+template <int T, int WAVES, bool FLIP, bool VEC>
 __global__ __launch_bounds__(64 * WAVES) void conv_small(float* __restrict__ Y, const float* __restrict__ X,
     const float* __restrict__ Wt, ConvShape sh, ConvEpi ep, int xe) {
-    __shared__ float lds[WAVES * kT * kT];
+    using Acc = std::conditional_t<T == 32, f32x16, f32x4>;
+    constexpr int SK = 512 / T;  // k a step, 8 a lane
+    __shared__ float lds[WAVES * T * T];
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int fr = lane & 31, fh = lane >> 5;
-    const int nt = (sh.Cout + kT - 1) / kT;
+    const int fr = lane % T, fh = lane / T;
+    const int nt = (sh.Cout + T - 1) / T;
     const int tl = xcd_order((int)blockIdx.x, (int)gridDim.x);
-    const int m0 = tl / nt * kT, n0 = tl % nt * kT;
+    const int m0 = tl / nt * T, n0 = tl % nt * T;
     const int nc = min(n0 + fr, sh.Cout - 1);
-    const int KK = sh.K * sh.K, nk = (sh.Cin + 15) / 16, steps = KK * nk;
+    const int KK = sh.K * sh.K, nk = (sh.Cin + SK - 1) / SK, steps = KK * nk;
     const int per = (steps + WAVES - 1) / WAVES, s0 = w * per, s1 = min(steps, s0 + per);
     uint32_t q, ow, b, oh;
     sh.wo.divmod((uint32_t)min(m0 + fr, sh.M - 1), q, ow);  // a row past the end computes the last, stores nothing
@@ -73,12 +88,12 @@ __global__ __launch_bounds__(64 * WAVES) void conv_small(float* __restrict__ Y, 
         int c;
     };
     Ops o[kAhead];
-    int tap = s0 / nk, c16 = s0 - tap * nk;
+    int tap = s0 / nk, cs = s0 - tap * nk;
     auto load = [&](Ops& r) {
         const int kh = tap / sh.K, kw = tap - kh * sh.K, ih = ih0 + kh, iw = iw0 + kw;
         r.ok = ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
         const float* x = xb + (size_t)(r.ok ? ih * sh.W + iw : 0) * sh.Cin;
-        r.c = 16 * c16 + 8 * fh;
+        r.c = SK * cs + 8 * fh;
         const size_t wt = FLIP ? ((size_t)(KK - 1 - tap) * sh.Cout + nc) * sh.Cin : (size_t)tap * sh.Cin * sh.Cout + nc;
         if constexpr (VEC) {
             const int cc = min(r.c, sh.Cin - 8);
@@ -101,10 +116,10 @@ __global__ __launch_bounds__(64 * WAVES) void conv_small(float* __restrict__ Y, 
                 r.vw[i] = Wt[FLIP ? wt + cc : wt + (size_t)cc * sh.Cout];
             }
         }
-        if (++c16 == nk) c16 = 0, tap = min(tap + 1, KK - 1);  // past the last step: a harmless reload
+        if (++cs == nk) cs = 0, tap = min(tap + 1, KK - 1);  // past the last step: a harmless reload
     };
-    f32x16 acc[1][1], cor[1][1];
-    acc[0][0] = cor[0][0] = (f32x16){};
+    Acc acc[1][1], cor[1][1];
+    acc[0][0] = cor[0][0] = (Acc){};
     if (s0 < s1) {
 #pragma unroll
         for (int u = 0; u < kAhead; ++u) load(o[u]);
@@ -126,26 +141,25 @@ __global__ __launch_bounds__(64 * WAVES) void conv_small(float* __restrict__ Y, 
     }
     acc[0][0] += cor[0][0];
     if (split_failed<1, 1>(acc)) {
-        // straight from memory in fp32, 2 k per MFMA; rare, so simple
-        acc[0][0] = (f32x16){};
+        // straight from memory in fp32, one k a lane; rare, so simple
+        acc[0][0] = (Acc){};
         for (int s = s0; s < s1; ++s) {
             const int t = s / nk, kh = t / sh.K, kw = t - kh * sh.K, ih = ih0 + kh, iw = iw0 + kw;
             const bool in = ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
-            for (int i = 0; i < 16; i += 2) {
-                const int ci = 16 * (s - t * nk) + i + fh, cc = min(ci, sh.Cin - 1);
+            for (int i = 0; i < SK; i += 64 / T) {
+                const int ci = SK * (s - t * nk) + i + fh, cc = min(ci, sh.Cin - 1);
                 const float x = xb[(size_t)(in ? ih * sh.W + iw : 0) * sh.Cin + cc];
                 const float y = FLIP ? Wt[((size_t)(KK - 1 - t) * sh.Cout + nc) * sh.Cin + cc]
                                      : Wt[((size_t)t * sh.Cin + cc) * sh.Cout + nc];
-                acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(in && ci < sh.Cin ? x : 0.0f, ci < sh.Cin ? y : 0.0f,
-                    acc[0][0], 0, 0, 0);
+                mfma_f32(in && ci < sh.Cin ? x : 0.0f, ci < sh.Cin ? y : 0.0f, acc[0][0]);
             }
         }
     }
-    put_part(lds, w, fr, fh, acc[0][0]);
+    put_part<T>(lds, w, fr, fh, acc[0][0]);
     __syncthreads();
     const float gain = ep.gain ? ep.gain[0] : 1.0f;
-    for (int i = tid; i < kT * kT; i += 64 * WAVES) {
-        const int m = m0 + i / kT, n = n0 + i % kT;
+    for (int i = tid; i < T * T; i += 64 * WAVES) {
+        const int m = m0 + i / T, n = n0 + i % T;
         if (m >= sh.M || n >= sh.Cout) continue;
         uint32_t co = 0;
         if (xe & kXeMod) {
@@ -153,7 +167,7 @@ __global__ __launch_bounds__(64 * WAVES) void conv_small(float* __restrict__ Y, 
             ep.hw.divmod((uint32_t)m, bb, r);
             co = bb * (uint32_t)sh.Cout + (uint32_t)n;
         }
-        epilogue_store(Y, sum_parts<WAVES>(lds, i), xe, (uint32_t)m * (uint32_t)sh.Cout + (uint32_t)n, co, ep,
+        epilogue_store(Y, sum_parts<T, WAVES>(lds, i), xe, (uint32_t)m * (uint32_t)sh.Cout + (uint32_t)n, co, ep,
             ep.bias ? ep.bias[n] : 0.0f, gain);
     }
 }
@@ -249,15 +263,15 @@ __global__ __launch_bounds__(64 * WAVES) void wgrad_small(float* __restrict__ gW
             const bool inside = (m < sh.M) & ((unsigned)ih < (unsigned)sh.H) & ((unsigned)iw < (unsigned)sh.W);
             const float x = X[(size_t)(inside ? ((int)b * sh.H + ih) * sh.W + iw : 0) * sh.Cin + ci];
             const float y = dY[(size_t)min(m, sh.M - 1) * sh.Cout + nc];
-            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(inside ? x : 0.0f, m < sh.M ? y : 0.0f, acc[0][0], 0, 0, 0);
+            mfma_f32(inside ? x : 0.0f, m < sh.M ? y : 0.0f, acc[0][0]);
         }
     }
-    put_part(lds, w, fr, fh, acc[0][0]);
+    put_part<kT>(lds, w, fr, fh, acc[0][0]);
     if (sums) bl[w][lane] = bs;
     __syncthreads();
     for (int i = tid; i < kT * kT; i += 64 * WAVES) {
         const int kk = k0 + i / kT, n = n0 + i % kT;
-        if (kk < sh.KKC && n < sh.Cout) gW[(size_t)kk * sh.Cout + n] = sum_parts<WAVES>(lds, i);
+        if (kk < sh.KKC && n < sh.Cout) gW[(size_t)kk * sh.Cout + n] = sum_parts<kT, WAVES>(lds, i);
     }
     if (sums && tid < kT && n0 + tid < sh.Cout) {
         float t = 0.0f;
@@ -267,30 +281,34 @@ __global__ __launch_bounds__(64 * WAVES) void wgrad_small(float* __restrict__ gW
     }
 }
 
-// Waves by the steps of a tile: one or two steps each.
-int waves_for(int steps) { return steps <= 4 ? 4 : steps <= 16 ? 8 : 16; }
-
 }  // namespace
 
 void nnk_conv_small(bool flip, int xe, float* Y, const float* X, const float* Wt, const ConvShape& sh,
     const ConvEpi& ep, hipStream_t s) {
-    const unsigned grid = (unsigned)((sh.M + kT - 1) / kT) * (unsigned)((sh.Cout + kT - 1) / kT);
-    const int waves = waves_for(sh.K * sh.K * ((sh.Cin + 15) / 16));
+    const int t = small_us(sh, flip, 16) < small_us(sh, flip, 32) ? 16 : 32;
+    const unsigned grid = (unsigned)((sh.M + t - 1) / t) * (unsigned)((sh.Cout + t - 1) / t);
+    const int waves = waves_for(sh.K * sh.K * ((sh.Cin + 512 / t - 1) / (512 / t)));
     const bool vec = sh.Cin % 8 == 0 && aligned16(X) && (!flip || aligned16(Wt));
-#define NNK_SMALL(W_, F_, V_) conv_small<W_, F_, V_><<<grid, 64 * W_, 0, s>>>(Y, X, Wt, sh, ep, xe)
-#define NNK_SMALL_W(F_, V_)                    \
-    do {                                       \
-        if (waves == 4) NNK_SMALL(4, F_, V_);  \
-        else if (waves == 8) NNK_SMALL(8, F_, V_); \
-        else NNK_SMALL(16, F_, V_);            \
+#define NNK_SMALL(T_, W_, F_, V_) conv_small<T_, W_, F_, V_><<<grid, 64 * W_, 0, s>>>(Y, X, Wt, sh, ep, xe)
+#define NNK_SMALL_W(T_, F_, V_)                        \
+    do {                                               \
+        if (waves == 4) NNK_SMALL(T_, 4, F_, V_);      \
+        else if (waves == 8) NNK_SMALL(T_, 8, F_, V_); \
+        else NNK_SMALL(T_, 16, F_, V_);                \
+    } while (0)
+#define NNK_SMALL_T(F_, V_)                  \
+    do {                                     \
+        if (t == 16) NNK_SMALL_W(16, F_, V_); \
+        else NNK_SMALL_W(32, F_, V_);        \
     } while (0)
     if (flip) {
-        if (vec) NNK_SMALL_W(true, true);
-        else NNK_SMALL_W(true, false);
+        if (vec) NNK_SMALL_T(true, true);
+        else NNK_SMALL_T(true, false);
     } else {
-        if (vec) NNK_SMALL_W(false, true);
-        else NNK_SMALL_W(false, false);
+        if (vec) NNK_SMALL_T(false, true);
+        else NNK_SMALL_T(false, false);
     }
+#undef NNK_SMALL_T
 #undef NNK_SMALL_W
 #undef NNK_SMALL
 }

@@ -119,13 +119,35 @@ void nnk_conv_forward(float* y, const float* x, const float* w, const float* bia
     nnk_after_launch(what, s);
 }
 
+static ConvShape dgrad_shape(int batch, int H, int W, int C_in, int C_out, int K, int pad) {
+    return ConvShape{batch, H + 2 * pad - K + 1, W + 2 * pad - K + 1, C_out, C_in, K, 1, K - 1 - pad, H, W,
+        batch * H * W, K * K * C_out, FastDiv((uint32_t)W), FastDiv((uint32_t)H)};
+}
+
+// With few input channels the direct kernel's columns are mostly padding (its
+// tiles have 32 or 16), K * K times over; the product dY W^T has K * K * C_in of
+// them.  Times in us: conv_tile's of both products, and for the pass that sums
+// the columns a launch and its bytes at 4.5 TB/s; a quarter and 2 us of margin,
+// for the fit and the buffer.  Direct / by columns measured: 3x3 3 -> 64 [64, 32,
+// 32] 22.5 / 18.7, 16 -> 64 22 / 38; 8 -> 64 [28, 56, 57] 27 / 43; 128 -> 128 [8, 7,
+// 7] 6.6 / 15.5; 5x5 8 -> 448 [53, 11, 11] 68 / 43, 16 -> 256 [43, 14, 14] 67 / 40.
+int nnk_conv_input_grad_by_columns(int batch, int H, int W, int C_in, int C_out, int K, int pad) {
+    const int Ho = H + 2 * pad - K + 1, Wo = W + 2 * pad - K + 1;
+    const long long rows = (long long)batch * Ho * Wo, kg = (long long)K * K * C_in;
+    if (K == 1 || rows <= 0 || rows >= (1LL << 31) || !nnk_conv_fits((int)rows, 1, 1, (int)kg, C_out, 1, 1, 1)) return 0;
+    double direct, product;
+    conv_tile(dgrad_shape(batch, H, W, C_in, C_out, K, pad), true, &direct);
+    conv_tile(dgrad_shape((int)rows, 1, 1, (int)kg, C_out, 1, 0), true, &product);
+    const double pass = 3.0 + 4.0 * ((double)rows * kg + (double)batch * H * W * C_in) / 4.5e6;
+    return 1.25 * (product + pass) + 2.0 < direct;
+}
+
 void nnk_conv_input_grad(float* dx, const float* dy, const float* w, const float* gain, int batch, int H, int W,
     int C_in, int C_out, int K, int pad, const NnConvFusion* f, hipStream_t s) {
     const char* what = "conv2d input gradient";
     NNK_REQUIRE(nnk_conv_fits(batch, H, W, C_in, C_out, K, H + 2 * pad - K + 1, W + 2 * pad - K + 1), what, "%s: tensor exceeds the 32-bit index range", what);
     if (batch <= 0) return;
-    const ConvShape sh{batch, H + 2 * pad - K + 1, W + 2 * pad - K + 1, C_out, C_in, K, 1, K - 1 - pad, H, W,
-        batch * H * W, K * K * C_out, FastDiv((uint32_t)W), FastDiv((uint32_t)H)};
+    const ConvShape sh = dgrad_shape(batch, H, W, C_in, C_out, K, pad);
     ConvEpi ep{};
     ep.gain = gain;
     if (f) nnk_conv_input_grad_fused(dx, dy, w, sh, ep, *f, s);

@@ -26,6 +26,10 @@ void nnk_conv_forward(float* y, const float* x, const float* w, const float* bia
    in launch_conv2d_input_grad_implicit_fused. */
 void nnk_conv_input_grad(float* dx, const float* dy, const float* w, const float* gain, int batch, int H, int W,
     int C_in, int C_out, int K, int pad, const NnConvFusion* f, hipStream_t s);
+/* Whether that is faster as the product dy w^T (a dense layer's input gradient
+   with C_in * K * K inputs, into batch * H_out * W_out rows of memory of the
+   caller's) and launch_col2im_set. */
+int nnk_conv_input_grad_by_columns(int batch, int H, int W, int C_in, int C_out, int K, int pad);
 /* gw, and with gb non-NULL the column sums of dy.  workspace:
    nnk_conv_weight_grad_workspace floats, enough for every smaller batch. */
 void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy, int batch, int H, int W, int C_in,

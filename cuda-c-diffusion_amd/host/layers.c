@@ -371,8 +371,12 @@ Module* sinusoidal_create(int num_channels, float max_period)
  * The matrix-core kernels (conv_api.h) take every forward and weight gradient
  * and the input gradient of stride 1 with pad <= K - 1, at any channel counts,
  * bias or gain in the epilogue, the weight in its own layout.  The input
- * gradient of other strides is rocBLAS and the gather col2im, which needs no
- * memset of grad_in.  NNHIP_CONV_PATH=gemm forces the reference's sequence of
+ * gradient of other strides, and of few input channels, is the product dy w^T
+ * (rocBLAS, and the kernels for few channels: 3x3 64 -> 128 of stride 2 at [32,
+ * 64, 64] takes rocBLAS 48 us, the kernels' 128-column tiles 59, storing 576
+ * columns of 128 terms each) and the gather col2im, which needs no memset of
+ * grad_in.
+ * NNHIP_CONV_PATH=gemm forces the reference's sequence of
  * im2col, GEMM and bias/gain pass.  Its im2col matrix (max_batch * H_out * W_out
  * * K*K*C_in floats, 604 MB at cfg3) is allocated only for a path the kernels do
  * not take, or when the variable is set as the module is created; forcing the
@@ -440,14 +444,20 @@ static void conv_bwd(Layer* L, const float* in, const float* out, const float* g
     }
     if (!grad_in) return;
     const float* gain = d[CD_MP] ? L->buf[CB_AUX] : NULL;
-    if (d[CD_DGRAD] && !forced) {
+    const int by_cols = col && d[CD_DGRAD] && !forced &&
+                        nnk_conv_input_grad_by_columns(batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_P]);
+    if (d[CD_DGRAD] && !by_cols && !forced) {
         /* stride 1: dx = conv(dy, flipped kernel, pad K-1-pad), times the gain in mp mode */
         nnk_conv_input_grad(grad_in, grad_out, w, gain, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K],
             d[CD_P], NULL, ctx->stream);
         return;
     }
-    nn_gemm_dX(ctx->blas, 1.0f, w, grad_out, col, rows, kg, d[CD_COUT]);
-    if (gain) launch_scale_by_scalar(col, gain, rows * kg, ctx->stream);
+    if (by_cols) {
+        nnk_conv_input_grad(col, grad_out, w, gain, rows, 1, 1, kg, d[CD_COUT], 1, 0, NULL, ctx->stream);
+    } else {
+        nn_gemm_dX(ctx->blas, 1.0f, w, grad_out, col, rows, kg, d[CD_COUT]);
+        if (gain) launch_scale_by_scalar(col, gain, rows * kg, ctx->stream);
+    }
     launch_col2im_set(grad_in, col, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_K], d[CD_S], d[CD_P], d[CD_HO],
         d[CD_WO], ctx->stream);
 }
@@ -566,8 +576,13 @@ Module* conv2d_create(Context* ctx, int C_in, int C_out, int K, int stride, int 
     layer_buf(L, nw, 0);
     layer_buf(L, (size_t)aux_n, 1);
     layer_buf(L, (size_t)aux_n, 0);
-    /* the im2col matrix, for the paths the matrix-core kernels do not take */
-    const int need_col = !d[CD_FWD] || !d[CD_WGRAD] || !d[CD_DGRAD] || conv_gemm_forced();
+    /* the im2col matrix, for what the matrix-core kernels do not take and for
+       input gradients that go by it; also where it is small or the channel
+       counts are odd, so that the reference's sequence can be asked for later */
+    const int need_col = !d[CD_FWD] || !d[CD_WGRAD] || !d[CD_DGRAD] || conv_gemm_forced() ||
+                         !nnhip_conv2d_implicit_supported(C_in, C_out) ||
+                         (size_t)max_batch * Ho * Wo * kg <= ((size_t)1 << 25) ||
+                         nnk_conv_input_grad_by_columns(max_batch, H, W, C_in, C_out, K, pad);
     layer_buf(L, need_col ? (size_t)max_batch * Ho * Wo * kg : 0, 0);
     layer_buf(L, d[CD_WGRAD] ? nnk_conv_weight_grad_workspace(max_batch, C_in, C_out, K, Ho, Wo) : 0, 0);
     layer_buf(L, mp_mode ? nnhip_weight_normalize_backward_workspace(C_out) : 0, 1);

@@ -1,11 +1,12 @@
 """The products of the conv2d, linear and mp_linear modules (host/conv_api.h) at
 any channel counts and alignment, at the edges of the small tiles (32 x 32
-outputs, 16 k a step, 4 / 8 / 16 waves) and of the tiled kernels' ragged forms,
+outputs and 16 k a step, or 16 x 16 and 32 k, 4 / 8 / 16 waves) and of the tiled kernels' ragged forms,
 against double; bar as in test_gpu_conv_implicit.py.  Geometries past each rule
 of the choice between them: few tiles (small), many (128, 64 or 32 columns)."""
 from __future__ import annotations
 
 import ctypes as C
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -25,6 +26,10 @@ GEOMS = [
     (5, 1, 1, 64, 96, 1, 1, 0, 1),      # dense, misaligned
     (8, 7, 7, 128, 128, 3, 1, 1, 0),    # small tiles, 72 steps
     (2, 6, 5, 40, 33, 3, 1, 1, 0),      # C_in no multiple of 16
+    (1, 17, 1, 72, 17, 1, 1, 0, 0),     # tiles of 16 with one row and column more, 4 waves
+    (1, 5, 3, 248, 16, 1, 1, 0, 1),     # fewer rows than one, misaligned, 8 waves
+    (2, 5, 8, 4, 320, 5, 1, 2, 0),      # a long k range, few outputs: 250 steps on 16 waves
+    (4, 16, 16, 256, 96, 3, 1, 1, 0),   # tiles of 32 forward and back, many of them
     (64, 32, 32, 3, 64, 3, 1, 1, 0),    # an image in: ragged rows, tiled
     (64, 32, 32, 64, 3, 3, 1, 1, 0),    # an image out
     (3, 65, 64, 20, 70, 3, 1, 1, 0),    # ragged, 128 columns of which 70 are
@@ -133,3 +138,39 @@ def test_small_tiles_fused_epilogues(L, nn, rng, geom):
     L.launch_weighted_sum(want.p, res.p, y.p, 0.83, 0.55, n, None)
     L.sync()
     assert_bits_equal(got.download(), want.download(), "residual")
+
+
+COLUMNS = [
+    # B, H, W, C_in, C_out, K, stride, pad, mp: input gradients by columns
+    (64, 32, 32, 3, 64, 3, 1, 1, 0),   # an image in
+    (20, 11, 11, 8, 448, 5, 1, 2, 1),  # a long k range, gain in the product's epilogue
+    (3, 9, 8, 40, 24, 3, 2, 1, 1),     # strided: the library product
+    (2, 10, 7, 5, 33, 5, 3, 0, 0),     # stride past the padding: pixels that no column reaches
+]
+
+
+@pytest.mark.parametrize("geom", COLUMNS, ids=lambda g: "x".join(map(str, g)))
+def test_input_gradient_by_columns(L, geom):
+    """The conv2d module against its im2col + GEMM + col2im sequence: different
+    summation orders of the same fp32 products, so 4 sqrt(terms) 2^-24 relative
+    to max(|v|, rms(v)); the longest sum has 25 * 448 terms (2.5e-5)."""
+    lib = C.CDLL(str(Path(__file__).resolve().parent / "_build" / "libgradcheck.so"))
+    lib.nn_convcheck.argtypes = [C.c_int] * 10 + [C.POINTER(C.c_float)]
+    lib.nn_convcheck.restype = C.c_double
+    print(f"[case] input gradient by columns {geom}", flush=True)
+    B, H, W, Ci, Co, K, s, p, mp = geom
+    by = L.dll.nnk_conv_input_grad_by_columns
+    by.argtypes, by.restype = [I] * 7, I
+    assert s > 1 or by(B, H, W, Ci, Co, K, p)
+    worst = lib.nn_convcheck(*geom, 1, (C.c_float * 4)())
+    terms = max(K * K * Ci, K * K * Co, B * ((H + 2 * p - K) // s + 1) * ((W + 2 * p - K) // s + 1))
+    assert worst <= 4 * terms ** 0.5 * 2.0 ** -24
+
+
+def test_rule_for_columns(L):
+    by = L.dll.nnk_conv_input_grad_by_columns
+    by.argtypes, by.restype = [I] * 7, I
+    assert not by(8, 7, 7, 128, 128, 3, 1)
+    assert not by(128, 32, 32, 128, 128, 3, 1)
+    assert not by(64, 32, 32, 3, 64, 1, 0)       # one tap: nothing to sum
+    assert not by(1 << 20, 64, 64, 3, 64, 3, 1)  # rows past 32 bits
