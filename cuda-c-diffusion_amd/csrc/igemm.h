@@ -840,13 +840,19 @@ struct WgradPlan {
 // 128 columns a workgroup above 64: a tile of 64 takes more than half as long.
 inline int tile_n(int Cout) { return Cout > 64 ? 128 : 64; }
 
-inline WgradPlan wgrad_plan(int M, int KKC, int Cout) {
+// At most as many splits as one round of resident workgroups holds (two per CU
+// on 256 CUs) and as there are stages of rows.  A plan may have fewer, its rows
+// being whole stages, so the splits do not grow with M (3x3 64 -> 64: 52 at
+// 3300 rows, 100 at 3200); this bound does, and sizes the workspaces, which
+// serve every smaller batch.
+inline int wgrad_most_splits(int M, int KKC, int Cout) {
     const int tiles = ((KKC + 127) / 128) * ((Cout + tile_n(Cout) - 1) / tile_n(Cout));
-    // one round of resident workgroups (two per CU on 256 CUs)
-    int S = tiles >= 512 ? 1 : 512 / tiles;
-    const int smax = (M + kWgM - 1) / kWgM;
-    if (S > smax) S = smax;
-    if (S < 1) S = 1;
+    const int S = tiles >= 512 ? 1 : 512 / tiles, smax = (M + kWgM - 1) / kWgM;
+    return S > smax ? smax : S;
+}
+
+inline WgradPlan wgrad_plan(int M, int KKC, int Cout) {
+    const int S = wgrad_most_splits(M, KKC, Cout);
     int rows = (M + S - 1) / S;
     rows = (rows + kWgM - 1) / kWgM * kWgM;
     WgradPlan p;

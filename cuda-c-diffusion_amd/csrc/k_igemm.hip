@@ -85,8 +85,8 @@ size_t nnhip_conv2d_wgrad_workspace(int batch, int C_in, int C_out, int K, int H
     if (batch <= 0 || !nnhip_conv2d_wgrad_implicit_supported(C_in, C_out)) return 0;
     const long long M = (long long)batch * H_out * W_out;
     if (M <= 0 || M >= (1LL << 31)) return 0;
-    const WgradPlan p = wgrad_plan((int)M, K * K * C_in, C_out);
-    return p.S > 1 ? (size_t)p.S * K * K * C_in * C_out : 0;
+    const int S = wgrad_most_splits((int)M, K * K * C_in, C_out);
+    return S > 1 ? (size_t)S * K * K * C_in * C_out : 0;
 }
 
 void launch_conv2d_weight_grad_implicit(float* gW, const float* X, const float* dY, int batch, int H, int W,
@@ -158,8 +158,8 @@ void nnk_conv_input_grad(float* dx, const float* dy, const float* w, const float
 size_t nnk_conv_weight_grad_workspace(int batch, int C_in, int C_out, int K, int H_out, int W_out) {
     const long long M = (long long)batch * H_out * W_out;
     if (M <= 0 || M >= (1LL << 31)) return 0;
-    const WgradPlan p = wgrad_plan((int)M, K * K * C_in, C_out);
-    return p.S > 1 ? (size_t)p.S * (K * K * C_in + 1) * C_out : 0;
+    const int S = wgrad_most_splits((int)M, K * K * C_in, C_out);
+    return S > 1 ? (size_t)S * (K * K * C_in + 1) * C_out : 0;
 }
 
 void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy, int batch, int H, int W, int C_in,

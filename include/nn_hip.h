@@ -248,8 +248,8 @@ int nnhip_conv2d_implicit_supported(int C_in, int C_out);
    gathered from x tile by tile.  Replaces the reference's launch_im2col +
    gemm_dW (src/conv2d.c:44-47).  The reduction over the batch*H_out*W_out
    rows is split over workgroups and the partials are added in a fixed order
-   (`workspace` of nnhip_conv2d_wgrad_workspace floats, or NULL: library
-   scratch).  Needs C_in % 4 == 0 and C_out % 64 == 0; x, dy 16-byte aligned. */
+   (`workspace` of nnhip_conv2d_wgrad_workspace floats, which serves every
+   smaller batch too, or NULL: library scratch).  Needs C_in % 4 == 0 and C_out % 64 == 0; x, dy 16-byte aligned. */
 void launch_conv2d_weight_grad_implicit(float* gW, const float* x, const float* dy, int batch, int H,
     int W, int C_in, int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace,
     hipStream_t s);

@@ -162,3 +162,17 @@ def test_layernorm_workspace_grows_with_batch(nn, c):
     L = nn.lib()
     sizes = [L.nnhip_layernorm_backward_workspace(b, c) for b in list(range(1, 200)) + [4095, 4096, 4097, 65536]]
     assert all(a <= b for a, b in zip(sizes, sizes[1:])), sizes
+
+
+@pytest.mark.parametrize("ci,co,k,hw", [(64, 64, 3, 4), (128, 128, 3, 8), (32, 192, 1, 5), (4, 64, 5, 3)])
+def test_weight_gradient_workspace_serves_smaller_batches(nn, ci, co, k, hw):
+    """A module's workspace has the size for its max_batch and serves every
+    smaller batch, whose rows may be split into more parts."""
+    L = nn.lib()
+    own = L.dll.nnk_conv_weight_grad_workspace
+    own.argtypes, own.restype = [ctypes.c_int] * 6, ctypes.c_size_t
+    for size in (L.nnhip_conv2d_wgrad_workspace, own):
+        sizes = [size(b, ci, co, k, hw, hw) for b in range(1, 400)]
+        assert sizes == sorted(sizes)
+        # as many parts as there are stages of 32 rows, until the device is full
+        assert sizes[39] >= min(512 // (-(-k * k * ci // 128) * -(-co // 128)), -(-40 * hw * hw // 32)) * k * k * ci * co
