@@ -469,7 +469,8 @@ static const LayerKind kConv2d = {"conv2d", conv_fwd, conv_bwd};
    Where they do not take it (channel counts that are no multiple of 8, which
    the kernels' epilogues do not serve at full speed, NNHIP_CONV_PATH=gemm), the
    module's own forward/backward runs and the pass follows as a launch of its
-   own, the reference's sequence.  The results are the same either way. */
+   own, the reference's sequence.  The results are the same either way, to
+   rounding where that input gradient goes by columns. */
 
 static int conv_fused_fwd(const Layer* L) { return L->dim[CD_FWD] && L->dim[CD_CIN] % 8 == 0 && !conv_gemm_path(L); }
 static int conv_fused_bwd(const Layer* L)
