@@ -35,6 +35,9 @@ int nnk_conv_input_grad_by_columns(int batch, int H, int W, int C_in, int C_out,
 void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy, int batch, int H, int W, int C_in,
     int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace, hipStream_t s);
 size_t nnk_conv_weight_grad_workspace(int batch, int C_in, int C_out, int K, int H_out, int W_out);
+/* launch_weight_normalize_backward_ws with *g_gain overwritten. */
+void nnk_weight_normalize_backward_set(float* gW, const float* Wn, const float* gain, float* g_gain, int in,
+    int out, float* workspace, hipStream_t s);
 
 #ifdef __cplusplus
 }

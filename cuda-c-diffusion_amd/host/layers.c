@@ -206,7 +206,7 @@ void groupnorm_shift_backward(Module* gn, const float* x, const float* shift, co
  * dense layers, each product a 1 x 1 convolution of one pixel (conv_api.h) with
  * bias or gain in its epilogue:
  *   mp_linear (src/mp_linear.c:12-39): W normalised in place every forward,
- *     Y = X W * gain; backward gW = X^T dY, g_gain zeroed then accumulated,
+ *     Y = X W * gain; backward gW = X^T dY, g_gain overwritten,
  *     gW projected and scaled, dX = dY W^T * gain;
  *   linear (src/linear.c:12-30): Y = X W + b; gW = X^T dY, gb = column sums,
  *     dX = dY W^T.
@@ -267,8 +267,7 @@ static void mpl_bwd(Layer* L, const float* in, const float* out, const float* gr
 {
     (void)out;
     dense_wgrad(L, in, grad_out, NULL, batch, ctx);
-    nnhip_fill_f32(L->buf[DB_GAUX], 0.0f, 1, ctx->stream);
-    launch_weight_normalize_backward_ws(L->buf[DB_GW], L->buf[DB_W], L->buf[DB_AUX], L->buf[DB_GAUX], L->dim[DD_IN],
+    nnk_weight_normalize_backward_set(L->buf[DB_GW], L->buf[DB_W], L->buf[DB_AUX], L->buf[DB_GAUX], L->dim[DD_IN],
         L->dim[DD_OUT], L->buf[DB_WNWS], ctx->stream);
     if (grad_in) dense_dgrad(L, grad_out, grad_in, L->buf[DB_AUX], batch, ctx);
 }
@@ -438,8 +437,7 @@ static void conv_bwd(Layer* L, const float* in, const float* out, const float* g
         if (gb) launch_bias_grad(gb, grad_out, rows, d[CD_COUT], ctx->stream);
     }
     if (d[CD_MP]) {
-        nnhip_fill_f32(L->buf[CB_GAUX], 0.0f, 1, ctx->stream);
-        launch_weight_normalize_backward_ws(gw, w, L->buf[CB_AUX], L->buf[CB_GAUX], kg, d[CD_COUT],
+        nnk_weight_normalize_backward_set(gw, w, L->buf[CB_AUX], L->buf[CB_GAUX], kg, d[CD_COUT],
             L->buf[CB_WNWS], ctx->stream);
     }
     if (!grad_in) return;

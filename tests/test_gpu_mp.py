@@ -257,3 +257,24 @@ def test_launcher_scratch_dropped_with_its_stream(L, orc, rng):
         finally:
             L.dll.nnhip_stream_synchronize(s)
             assert L.dll.nnhip_stream_destroy(s) == 0
+
+
+@pytest.mark.parametrize("n_in,n_out", [(1, 1), (5, 3), (1024, 4), (1152, 130), (4500, 9)])
+def test_weight_normalize_backward_set_gain(L, rng, n_in, n_out):
+    """The modules' form, which overwrites the gain gradient, against the
+    accumulating one on zero, bit for bit; twice, for the re-armed counter."""
+    import ctypes as C
+    f = L.dll.nnk_weight_normalize_backward_set
+    f.argtypes, f.restype = [C.c_void_p] * 4 + [C.c_int] * 2 + [C.c_void_p] * 2, None
+    w = L.to_device(rng.standard_normal((n_in, n_out)).astype(np.float32) / np.float32(np.sqrt(n_in)))
+    g = rng.standard_normal((n_in, n_out)).astype(np.float32)
+    gain = L.to_device(np.array([0.7], np.float32))
+    ws = L.to_device(np.zeros(L.nnhip_weight_normalize_backward_workspace(n_out), np.float32))
+    want, want_gain = L.to_device(g), L.to_device(np.zeros(1, np.float32))
+    L.launch_weight_normalize_backward_ws(want.p, w.p, gain.p, want_gain.p, n_in, n_out, ws.p, None)
+    for before in (3.0, np.nan):
+        got, got_gain = L.to_device(g), L.to_device(np.array([before], np.float32))
+        f(got.p, w.p, gain.p, got_gain.p, n_in, n_out, ws.p, None)
+        L.sync()
+        assert_bits_equal(got.download(), want.download(), "gW")
+        assert_bits_equal(got_gain.download(), want_gain.download(), "g_gain")
