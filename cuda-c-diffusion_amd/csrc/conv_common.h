@@ -10,6 +10,10 @@ namespace conv {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
+constexpr int kBM = 128, kBK = 32;  // rows and k slices of the tiled kernels
+constexpr int kBNmin = 64;          // columns that the launchers of nn_hip.h need
+constexpr int kWgM = 32;            // rows that a split of the weight gradient is made of
+
 struct ConvShape {
     int B, H, W, Cin, Cout, K, stride, pad, Ho, Wo;
     int M;    // B * Ho * Wo
@@ -155,6 +159,77 @@ __device__ __forceinline__ void epilogue_store(float* __restrict__ Y, float v, i
         const float z = act_fwd<ACT_SILU, false>(v * (ep.cond[co] + 1.0f));
         ep.y2[o] = ep.mp ? z * kMpSiluScale : z;
     }
+}
+
+// Checks shared by the forward launchers (plain and fused): -1 after
+// recording an error, 0 when there is nothing to do (batch 0), 1 with `sh`
+// filled in.
+inline int fwd_setup(const char* what, const float* Y, const float* X, const float* Wt, const float* bias,
+    const float* gain, int batch, int H, int W, int C_in, int C_out, int K, int stride, int pad, int H_out,
+    int W_out, ConvShape& sh) {
+    NNK_REQUIRE_RET(batch >= 0 && H > 0 && W > 0 && K > 0 && stride > 0 && pad >= 0, -1, what,
+        "%s: bad geometry", what);
+    NNK_REQUIRE_RET(nnhip_conv2d_implicit_supported(C_in, C_out), -1, what,
+        "%s: needs C_in %% %d == 0 and C_out %% %d == 0 (C_in=%d C_out=%d)", what, kBK, kBNmin, C_in, C_out);
+    NNK_REQUIRE_RET(H_out == (H + 2 * pad - K) / stride + 1 && W_out == (W + 2 * pad - K) / stride + 1 &&
+                        H_out > 0 && W_out > 0,
+        -1, what, "%s: output size %dx%d does not match the geometry", what, H_out, W_out);
+    NNK_REQUIRE_RET((long long)batch * H * W * C_in < (1LL << 31) &&
+                        (long long)batch * H_out * W_out * C_out < (1LL << 31),
+        -1, what, "%s: tensor exceeds the 32-bit index range", what);
+    NNK_REQUIRE_RET(!(bias && gain), -1, what, "%s: bias and gain are exclusive", what);
+    if (batch == 0) return 0;
+    NNK_REQUIRE_RET(Y && X && Wt, -1, what, "%s: null pointer", what);
+    NNK_REQUIRE_RET(aligned16(X) && aligned16(Wt), -1, what, "%s: x and the weight must be 16-byte aligned", what);
+    sh = ConvShape{batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, batch * H_out * W_out, K * K * C_in,
+        FastDiv((uint32_t)W_out), FastDiv((uint32_t)H_out)};
+    return 1;
+}
+
+// Checks shared by the input-gradient launchers; `sh` is then the stride-1
+// convolution of dy (Ho x Wo x C_out) with the flipped kernel and padding
+// K-1-pad, whose output is H x W x C_in.
+inline int dgrad_setup(const char* what, const float* dX, const float* dY, const float* Wt, int batch, int H, int W,
+    int C_in, int C_out, int K, int pad, ConvShape& sh) {
+    NNK_REQUIRE_RET(batch >= 0 && H > 0 && W > 0 && K > 0 && pad >= 0, -1, what, "%s: bad geometry", what);
+    NNK_REQUIRE_RET(nnhip_conv2d_input_grad_implicit_supported(C_in, C_out, K, 1, pad), -1, what,
+        "%s: needs pad <= K - 1, C_out %% %d == 0 and C_in %% %d == 0 (C_in=%d C_out=%d K=%d pad=%d)", what, kBK,
+        kBNmin, C_in, C_out, K, pad);
+    const int Ho = H + 2 * pad - K + 1, Wo = W + 2 * pad - K + 1;
+    NNK_REQUIRE_RET(Ho > 0 && Wo > 0, -1, what, "%s: empty output for this geometry", what);
+    NNK_REQUIRE_RET((long long)batch * H * W * C_in < (1LL << 31) && (long long)batch * Ho * Wo * C_out < (1LL << 31) &&
+                        (long long)K * K * C_in * C_out < (1LL << 31),
+        -1, what, "%s: tensor exceeds the 32-bit index range", what);
+    if (batch == 0) return 0;
+    NNK_REQUIRE_RET(dX && dY && Wt, -1, what, "%s: null pointer", what);
+    NNK_REQUIRE_RET(aligned16(dY) && aligned16(Wt), -1, what, "%s: dy and the weight must be 16-byte aligned", what);
+    sh = ConvShape{batch, Ho, Wo, C_out, C_in, K, 1, K - 1 - pad, H, W, batch * H * W, K * K * C_out,
+        FastDiv((uint32_t)W), FastDiv((uint32_t)H)};
+    return 1;
+}
+
+// Checks of the weight-gradient launchers; batch 0 clears gW.
+inline int wgrad_setup(const char* what, float* gW, const float* X, const float* dY, int batch, int H, int W, int C_in,
+    int C_out, int K, int stride, int pad, int H_out, int W_out, hipStream_t s, ConvShape& sh) {
+    NNK_REQUIRE_RET(batch >= 0 && H > 0 && W > 0 && K > 0 && stride > 0 && pad >= 0, -1, what, "%s: bad geometry", what);
+    NNK_REQUIRE_RET(nnhip_conv2d_wgrad_implicit_supported(C_in, C_out), -1, what,
+        "%s: needs C_in %% 4 == 0 and C_out %% %d == 0 (C_in=%d C_out=%d)", what, kBNmin, C_in, C_out);
+    NNK_REQUIRE_RET(H_out == (H + 2 * pad - K) / stride + 1 && W_out == (W + 2 * pad - K) / stride + 1 && H_out > 0 &&
+                        W_out > 0,
+        -1, what, "%s: output size %dx%d does not match the geometry", what, H_out, W_out);
+    NNK_REQUIRE_RET((long long)batch * H * W * C_in < (1LL << 31) &&
+                        (long long)batch * H_out * W_out * C_out < (1LL << 31),
+        -1, what, "%s: tensor exceeds the 32-bit index range", what);
+    NNK_REQUIRE_RET(gW && (batch == 0 || (X && dY)), -1, what, "%s: null pointer", what);
+    const int KKC = K * K * C_in;
+    if (batch == 0) {
+        nnhip_fill_f32(gW, 0.0f, (size_t)KKC * C_out, s);
+        return 0;
+    }
+    NNK_REQUIRE_RET(aligned16(X) && aligned16(dY), -1, what, "%s: X and dY must be 16-byte aligned", what);
+    sh = ConvShape{batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, batch * H_out * W_out, KKC,
+        FastDiv((uint32_t)W_out), FastDiv((uint32_t)H_out)};
+    return 1;
 }
 
 // Waves of a small tile by its steps: one or two steps each.

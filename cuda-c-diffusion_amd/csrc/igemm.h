@@ -12,8 +12,7 @@ namespace {
 using namespace nnk;
 using namespace nnk::conv;
 
-constexpr int kBM = 128, kBK = 32, kTpb = 256;
-constexpr int kBNmin = 64;  // output-channel tiles of 128 or 64
+constexpr int kTpb = 256;
 
 // LDS tiles hold rows of 32 k, 64 bytes (four 16-byte chunks) a plane, and
 // every access is 16 bytes a lane.  The order of a row's chunks depends on the
@@ -505,7 +504,6 @@ void conv_launch(float* Y, const float* X, const float* Wt, const ConvShape& sh,
 // pass over dY of two launches (5 us and more).
 // ---------------------------------------------------------------------------
 constexpr int kStage = 16;  // rows per stage
-constexpr int kWgM = 32;  // m rows per stage
 
 // How the activation columns are loaded: kSingles one by one, for any channel
 // counts and alignments; kPairs two at a time (C_in even, x 8-byte aligned);
@@ -877,53 +875,6 @@ inline bool wgrad_small_wins(const ConvShape& sh) {
     return 4.0 + (trips > work ? trips : work) < 12.0 + stage * (p.rows / kWgM);
 }
 
-// Checks shared by the forward launchers (plain and fused): -1 after
-// recording an error, 0 when there is nothing to do (batch 0), 1 with `sh`
-// filled in.
-inline int fwd_setup(const char* what, const float* Y, const float* X, const float* Wt, const float* bias,
-    const float* gain, int batch, int H, int W, int C_in, int C_out, int K, int stride, int pad, int H_out,
-    int W_out, ConvShape& sh) {
-    NNK_REQUIRE_RET(batch >= 0 && H > 0 && W > 0 && K > 0 && stride > 0 && pad >= 0, -1, what,
-        "%s: bad geometry", what);
-    NNK_REQUIRE_RET(nnhip_conv2d_implicit_supported(C_in, C_out), -1, what,
-        "%s: needs C_in %% %d == 0 and C_out %% %d == 0 (C_in=%d C_out=%d)", what, kBK, kBNmin, C_in, C_out);
-    NNK_REQUIRE_RET(H_out == (H + 2 * pad - K) / stride + 1 && W_out == (W + 2 * pad - K) / stride + 1 &&
-                        H_out > 0 && W_out > 0,
-        -1, what, "%s: output size %dx%d does not match the geometry", what, H_out, W_out);
-    NNK_REQUIRE_RET((long long)batch * H * W * C_in < (1LL << 31) &&
-                        (long long)batch * H_out * W_out * C_out < (1LL << 31),
-        -1, what, "%s: tensor exceeds the 32-bit index range", what);
-    NNK_REQUIRE_RET(!(bias && gain), -1, what, "%s: bias and gain are exclusive", what);
-    if (batch == 0) return 0;
-    NNK_REQUIRE_RET(Y && X && Wt, -1, what, "%s: null pointer", what);
-    NNK_REQUIRE_RET(aligned16(X) && aligned16(Wt), -1, what, "%s: x and the weight must be 16-byte aligned", what);
-    sh = ConvShape{batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, batch * H_out * W_out, K * K * C_in,
-        FastDiv((uint32_t)W_out), FastDiv((uint32_t)H_out)};
-    return 1;
-}
-
-// Checks shared by the input-gradient launchers; `sh` is then the stride-1
-// convolution of dy (Ho x Wo x C_out) with the flipped kernel and padding
-// K-1-pad, whose output is H x W x C_in.
-inline int dgrad_setup(const char* what, const float* dX, const float* dY, const float* Wt, int batch, int H, int W,
-    int C_in, int C_out, int K, int pad, ConvShape& sh) {
-    NNK_REQUIRE_RET(batch >= 0 && H > 0 && W > 0 && K > 0 && pad >= 0, -1, what, "%s: bad geometry", what);
-    NNK_REQUIRE_RET(nnhip_conv2d_input_grad_implicit_supported(C_in, C_out, K, 1, pad), -1, what,
-        "%s: needs pad <= K - 1, C_out %% %d == 0 and C_in %% %d == 0 (C_in=%d C_out=%d K=%d pad=%d)", what, kBK,
-        kBNmin, C_in, C_out, K, pad);
-    const int Ho = H + 2 * pad - K + 1, Wo = W + 2 * pad - K + 1;
-    NNK_REQUIRE_RET(Ho > 0 && Wo > 0, -1, what, "%s: empty output for this geometry", what);
-    NNK_REQUIRE_RET((long long)batch * H * W * C_in < (1LL << 31) && (long long)batch * Ho * Wo * C_out < (1LL << 31) &&
-                        (long long)K * K * C_in * C_out < (1LL << 31),
-        -1, what, "%s: tensor exceeds the 32-bit index range", what);
-    if (batch == 0) return 0;
-    NNK_REQUIRE_RET(dX && dY && Wt, -1, what, "%s: null pointer", what);
-    NNK_REQUIRE_RET(aligned16(dY) && aligned16(Wt), -1, what, "%s: dy and the weight must be 16-byte aligned", what);
-    sh = ConvShape{batch, Ho, Wo, C_out, C_in, K, 1, K - 1 - pad, H, W, batch * H * W, K * K * C_out,
-        FastDiv((uint32_t)W), FastDiv((uint32_t)H)};
-    return 1;
-}
-
 // The tiled weight gradient of a checked, non-empty shape, and with gb non-null
 // the column sums of dY.
 inline void wgrad_run(const char* what, float* gW, float* gb, const float* X, const float* dY, const ConvShape& sh,
@@ -973,23 +924,8 @@ inline void wgrad_run(const char* what, float* gW, float* gb, const float* X, co
 
 inline void wgrad_launch(const char* what, float* gW, const float* X, const float* dY, int batch, int H, int W, int C_in,
     int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace, hipStream_t s) {
-    NNK_REQUIRE(batch >= 0 && H > 0 && W > 0 && K > 0 && stride > 0 && pad >= 0, what, "%s: bad geometry", what);
-    NNK_REQUIRE(nnhip_conv2d_wgrad_implicit_supported(C_in, C_out), what,
-        "%s: needs C_in %% 4 == 0 and C_out %% %d == 0 (C_in=%d C_out=%d)", what, kBNmin, C_in, C_out);
-    NNK_REQUIRE(H_out == (H + 2 * pad - K) / stride + 1 && W_out == (W + 2 * pad - K) / stride + 1 && H_out > 0 &&
-                    W_out > 0,
-        what, "%s: output size %dx%d does not match the geometry", what, H_out, W_out);
-    NNK_REQUIRE((long long)batch * H * W * C_in < (1LL << 31) && (long long)batch * H_out * W_out * C_out < (1LL << 31),
-        what, "%s: tensor exceeds the 32-bit index range", what);
-    NNK_REQUIRE(gW && (batch == 0 || (X && dY)), what, "%s: null pointer", what);
-    const int KKC = K * K * C_in;
-    if (batch == 0) {
-        nnhip_fill_f32(gW, 0.0f, (size_t)KKC * C_out, s);
-        return;
-    }
-    NNK_REQUIRE(aligned16(X) && aligned16(dY), what, "%s: X and dY must be 16-byte aligned", what);
-    ConvShape sh{batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, batch * H_out * W_out, KKC,
-        FastDiv((uint32_t)W_out), FastDiv((uint32_t)H_out)};
+    ConvShape sh;
+    if (wgrad_setup(what, gW, X, dY, batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, s, sh) <= 0) return;
     if (wgrad_small_wins(sh)) nnk_wgrad_small(gW, nullptr, X, dY, sh, s);
     else wgrad_run(what, gW, nullptr, X, dY, sh, workspace, s);
     nnk_after_launch(what, s);

@@ -1,5 +1,5 @@
-/* conv_api.h -- the products inside the conv2d, linear and mp_linear modules,
- * on the matrix-core kernels (csrc/igemm.h, csrc/k_conv_small.hip).  Unlike the
+/* conv_api.h -- the products inside the conv2d and linear modules, on the
+ * matrix-core kernels (csrc/igemm.h, csrc/k_conv_small.hip).  Unlike the
  * launchers of nn_hip.h they take any channel counts and 4-byte alignment, and
  * pick the tiled or the small-tile kernels by the work's size.  A dense layer
  * is a convolution with H = W = K = 1.  Tensors below 2^31 elements
@@ -35,6 +35,18 @@ int nnk_conv_input_grad_by_columns(int batch, int H, int W, int C_in, int C_out,
 void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy, int batch, int H, int W, int C_in,
     int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace, hipStream_t s);
 size_t nnk_conv_weight_grad_workspace(int batch, int C_in, int C_out, int K, int H_out, int W_out);
+/* The same sums on the fp32 matrix cores, for conv2d modules with a gain
+   (csrc/k_igemm_f32.hip says why): channel counts, alignment and index range as
+   the launchers of nn_hip.h, outputs times gain[0].  f (may be NULL): res, or cond
+   and y2 with MP-SiLU; for the input gradient act_in with MP-SiLU, and res.
+   workspace as above. */
+void nnk_conv_f32_forward(float* y, const float* x, const float* w, const float* gain, int batch, int H, int W,
+    int C_in, int C_out, int K, int stride, int pad, int H_out, int W_out, const NnConvFusion* f, hipStream_t s);
+void nnk_conv_f32_input_grad(float* dx, const float* dy, const float* w, const float* gain, int batch, int H, int W,
+    int C_in, int C_out, int K, int pad, const NnConvFusion* f, hipStream_t s);
+void nnk_conv_f32_weight_grad(float* gw, const float* x, const float* dy, int batch, int H, int W, int C_in,
+    int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace, hipStream_t s);
+size_t nnk_conv_f32_weight_grad_workspace(int batch, int C_in, int C_out, int K, int H_out, int W_out);
 /* launch_weight_normalize_backward_ws with *g_gain overwritten. */
 void nnk_weight_normalize_backward_set(float* gW, const float* Wn, const float* gain, float* g_gain, int in,
     int out, float* workspace, hipStream_t s);

@@ -203,86 +203,69 @@ void groupnorm_shift_backward(Module* gn, const float* x, const float* shift, co
 }
 
 /* ------------------------------------------------------------------------
- * dense layers, each product a 1 x 1 convolution of one pixel (conv_api.h) with
- * bias or gain in its epilogue:
+ * dense layers:
  *   mp_linear (src/mp_linear.c:12-39): W normalised in place every forward,
  *     Y = X W * gain; backward gW = X^T dY, g_gain overwritten,
- *     gW projected and scaled, dX = dY W^T * gain;
+ *     gW projected and scaled, dX = dY W^T * gain.  The products are rocBLAS's:
+ *     the gain gradient keeps its summation order (csrc/k_igemm_f32.hip);
  *   linear (src/linear.c:12-30): Y = X W + b; gW = X^T dY, gb = column sums,
- *     dX = dY W^T.
- * A product outside the kernels' index range is rocBLAS and a pass of its own.
+ *     dX = dY W^T, each product a 1 x 1 convolution of one pixel (conv_api.h) with
+ *     the bias in its epilogue, or rocBLAS and a pass of its own outside the
+ *     kernels' index range.
  * ------------------------------------------------------------------------ */
 
 enum { DB_W, DB_GW, DB_AUX, DB_GAUX, DB_WNWS };
 enum { DD_IN, DD_OUT };
 
-/* Y = X W + bias | * gain[0] */
-static void dense_fwd(const Layer* L, const float* in, float* out, const float* bias, const float* gain, int batch,
-    Context* ctx)
-{
-    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
-    if (nnk_conv_fits(batch, 1, 1, ni, no, 1, 1, 1)) {
-        nnk_conv_forward(out, in, L->buf[DB_W], bias, gain, batch, 1, 1, ni, no, 1, 1, 0, 1, 1, NULL, ctx->stream);
-        return;
-    }
-    nn_gemm_forward(ctx->blas, 1.0f, in, L->buf[DB_W], out, batch, ni, no);
-    if (bias) launch_add_bias(out, bias, batch, no, ctx->stream);
-    if (gain) launch_scale_by_scalar(out, gain, batch * no, ctx->stream);
-}
-
-/* gW = X^T dY and, with gb, the column sums of dY */
-static void dense_wgrad(const Layer* L, const float* in, const float* grad_out, float* gb, int batch, Context* ctx)
-{
-    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
-    /* no workspace is lent: the library's scratch where the rows are split */
-    if (nnk_conv_fits(batch, 1, 1, ni, no, 1, 1, 1)) {
-        nnk_conv_weight_grad(L->buf[DB_GW], gb, in, grad_out, batch, 1, 1, ni, no, 1, 1, 0, 1, 1, NULL, ctx->stream);
-        return;
-    }
-    nn_gemm_dW(ctx->blas, 1.0f, in, grad_out, L->buf[DB_GW], batch, ni, no);
-    if (gb) launch_bias_grad(gb, grad_out, batch, no, ctx->stream);
-}
-
-/* dX = dY W^T * gain[0] */
-static void dense_dgrad(const Layer* L, const float* grad_out, float* grad_in, const float* gain, int batch,
-    Context* ctx)
-{
-    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
-    if (nnk_conv_fits(batch, 1, 1, ni, no, 1, 1, 1)) {
-        nnk_conv_input_grad(grad_in, grad_out, L->buf[DB_W], gain, batch, 1, 1, ni, no, 1, 0, NULL, ctx->stream);
-        return;
-    }
-    nn_gemm_dX(ctx->blas, 1.0f, L->buf[DB_W], grad_out, grad_in, batch, ni, no);
-    if (gain) launch_scale_by_scalar(grad_in, gain, batch * ni, ctx->stream);
-}
-
 static void mpl_fwd(Layer* L, const float* in, float* out, int batch, Context* ctx)
 {
-    launch_weight_normalize(L->buf[DB_W], L->dim[DD_IN], L->dim[DD_OUT], L->k[0], ctx->stream);
-    dense_fwd(L, in, out, NULL, L->buf[DB_AUX], batch, ctx);
+    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
+    launch_weight_normalize(L->buf[DB_W], ni, no, L->k[0], ctx->stream);
+    nn_gemm_forward(ctx->blas, 1.0f, in, L->buf[DB_W], out, batch, ni, no);
+    launch_scale_by_scalar(out, L->buf[DB_AUX], batch * no, ctx->stream);
 }
 
 static void mpl_bwd(Layer* L, const float* in, const float* out, const float* grad_out, float* grad_in, int batch,
     Context* ctx)
 {
     (void)out;
-    dense_wgrad(L, in, grad_out, NULL, batch, ctx);
-    nnk_weight_normalize_backward_set(L->buf[DB_GW], L->buf[DB_W], L->buf[DB_AUX], L->buf[DB_GAUX], L->dim[DD_IN],
-        L->dim[DD_OUT], L->buf[DB_WNWS], ctx->stream);
-    if (grad_in) dense_dgrad(L, grad_out, grad_in, L->buf[DB_AUX], batch, ctx);
+    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
+    nn_gemm_dW(ctx->blas, 1.0f, in, grad_out, L->buf[DB_GW], batch, ni, no);
+    nnk_weight_normalize_backward_set(L->buf[DB_GW], L->buf[DB_W], L->buf[DB_AUX], L->buf[DB_GAUX], ni, no,
+        L->buf[DB_WNWS], ctx->stream);
+    if (!grad_in) return;
+    nn_gemm_dX(ctx->blas, 1.0f, L->buf[DB_W], grad_out, grad_in, batch, ni, no);
+    launch_scale_by_scalar(grad_in, L->buf[DB_AUX], batch * ni, ctx->stream);
 }
 
 static void lin_fwd(Layer* L, const float* in, float* out, int batch, Context* ctx)
 {
-    dense_fwd(L, in, out, L->buf[DB_AUX], NULL, batch, ctx);
+    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
+    if (nnk_conv_fits(batch, 1, 1, ni, no, 1, 1, 1)) {
+        nnk_conv_forward(out, in, L->buf[DB_W], L->buf[DB_AUX], NULL, batch, 1, 1, ni, no, 1, 1, 0, 1, 1, NULL,
+            ctx->stream);
+        return;
+    }
+    nn_gemm_forward(ctx->blas, 1.0f, in, L->buf[DB_W], out, batch, ni, no);
+    launch_add_bias(out, L->buf[DB_AUX], batch, no, ctx->stream);
 }
 
 static void lin_bwd(Layer* L, const float* in, const float* out, const float* grad_out, float* grad_in, int batch,
     Context* ctx)
 {
     (void)out;
-    dense_wgrad(L, in, grad_out, L->buf[DB_GAUX], batch, ctx);
-    if (grad_in) dense_dgrad(L, grad_out, grad_in, NULL, batch, ctx);
+    const int ni = L->dim[DD_IN], no = L->dim[DD_OUT];
+    if (nnk_conv_fits(batch, 1, 1, ni, no, 1, 1, 1)) {
+        /* no workspace is lent: the library's scratch where the rows are split */
+        nnk_conv_weight_grad(L->buf[DB_GW], L->buf[DB_GAUX], in, grad_out, batch, 1, 1, ni, no, 1, 1, 0, 1, 1, NULL,
+            ctx->stream);
+        if (grad_in)
+            nnk_conv_input_grad(grad_in, grad_out, L->buf[DB_W], NULL, batch, 1, 1, ni, no, 1, 0, NULL, ctx->stream);
+        return;
+    }
+    nn_gemm_dW(ctx->blas, 1.0f, in, grad_out, L->buf[DB_GW], batch, ni, no);
+    launch_bias_grad(L->buf[DB_GAUX], grad_out, batch, no, ctx->stream);
+    if (grad_in) nn_gemm_dX(ctx->blas, 1.0f, L->buf[DB_W], grad_out, grad_in, batch, ni, no);
 }
 
 static const LayerKind kMpLinear = {"mp_linear", mpl_fwd, mpl_bwd};
@@ -367,14 +350,20 @@ Module* sinusoidal_create(int num_channels, float max_period)
 /* ------------------------------------------------------------------------
  * conv2d, NHWC, plain (bias) or magnitude-preserving (forced weight norm and
  * gain), weights [K*K*C_in, C_out] row-major (src/conv2d.c:17-66).
- * The matrix-core kernels (conv_api.h) take every forward and weight gradient
- * and the input gradient of stride 1 with pad <= K - 1, at any channel counts,
- * bias or gain in the epilogue, the weight in its own layout.  The input
+ * Plain: the matrix-core kernels (conv_api.h) take every forward and weight
+ * gradient and the input gradient of stride 1 with pad <= K - 1, at any channel
+ * counts, the bias in the epilogue, the weight in its own layout.  The input
  * gradient of other strides, and of few input channels, is the product dy w^T
  * (rocBLAS, and the kernels for few channels: 3x3 64 -> 128 of stride 2 at [32,
  * 64, 64] takes rocBLAS 48 us, the kernels' 128-column tiles 59, storing 576
  * columns of 128 terms each) and the gather col2im, which needs no memset of
  * grad_in.
+ * With a gain: the fp32 matrix cores' kernels (nnk_conv_f32_*) where the channel
+ * counts allow them (forward C_in % 32 == 0, C_out % 64 == 0; weight gradient C_in
+ * % 4, C_out % 64; stride-1 input gradient C_out % 32, C_in % 64) and, for forward
+ * and input gradient, where they beat im2col + rocBLAS at max_batch
+ * (NNHIP_CONV_PATH=implicit at creation: wherever allowed); the gain in their
+ * epilogue.  Otherwise im2col, rocBLAS, the gain pass and col2im.
  * NNHIP_CONV_PATH=gemm forces the reference's sequence of
  * im2col, GEMM and bias/gain pass.  Its im2col matrix (max_batch * H_out * W_out
  * * K*K*C_in floats, 604 MB at cfg3) is allocated only for a path the kernels do
@@ -391,6 +380,30 @@ static int conv_gemm_forced(void)
     return e && strcmp(e, "gemm") == 0;
 }
 
+static int conv_implicit_forced(void)
+{
+    const char* e = getenv("NNHIP_CONV_PATH");
+    return e && strcmp(e, "implicit") == 0;
+}
+
+/* Whether the fp32 matrix-core kernels (the forward, and the stride-1 input
+   gradient) beat im2col + rocBLAS for an M x N x K product, by a cost
+   model fitted on MI355X.  A 128 x BN output tile takes ~2.25 us per 32-deep k
+   slice with one workgroup per CU (3x3 128 -> 128 at [128, 32, 32]: 36 slices, 1024
+   tiles, four tiles per CU: 320 us), so few tiles leave the device idle: at
+   7 x 7 x 128 (M = 392 at batch 8, 4 tiles) the kernel takes ~83 us where the
+   GEMM path takes ~10.  The GEMM path: ~10 us of fixed cost, the GEMM at ~70
+   TFLOP/s (rocBLAS fp32, measured at the first of these) and the im2col matrix
+   written and read at ~6 TB/s. */
+static int conv_f32_wins(long long M, int N, int K)
+{
+    const int bn = N % 128 == 0 ? 128 : 64;
+    const double tiles = (double)((M + 127) / 128) * ((N + bn - 1) / bn);
+    const double t_impl = (K / 32.0) * 2.25 * ceil(tiles / 256.0);
+    const double t_gemm = 10.0 + 2.0 * (double)M * N * K / 70e6 + 8.0 * (double)M * K / 6e6;
+    return t_impl <= t_gemm;
+}
+
 /* the reference's sequence asked for at this call (needs the im2col buffer) */
 static int conv_gemm_path(const Layer* L)
 {
@@ -400,6 +413,48 @@ static int conv_gemm_path(const Layer* L)
     return 1;
 }
 
+/* The fp32 matrix-core kernels take 128-bit loads of the activations they
+   gather; a misaligned tensor would make them refuse and leave the output
+   unwritten, so the module stops with a message instead. */
+static void conv_require_aligned(const float* p, const char* what)
+{
+    if (((uintptr_t)p & 15u) != 0) {
+        fprintf(stderr, "conv2d: %s at %p is not 16-byte aligned (the implicit-GEMM path needs it)\n", what,
+            (const void*)p);
+        exit(1);
+    }
+}
+
+/* forward on the matrix cores, with the neighbour in f (may be NULL) */
+static void conv_fwd_cores(Layer* L, const float* in, float* out, int batch, const NnConvFusion* f, Context* ctx)
+{
+    const int* d = L->dim;
+    float *w = L->buf[CB_W], *aux = L->buf[CB_AUX];
+    if (d[CD_MP]) {
+        conv_require_aligned(in, "the forward input");
+        nnk_conv_f32_forward(out, in, w, aux, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_S],
+            d[CD_P], d[CD_HO], d[CD_WO], f, ctx->stream);
+        return;
+    }
+    nnk_conv_forward(out, in, w, aux, NULL, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_S],
+        d[CD_P], d[CD_HO], d[CD_WO], f, ctx->stream);
+}
+
+/* stride 1: dx = conv(dy, flipped kernel, pad K-1-pad), times the gain in mp mode */
+static void conv_dgrad_cores(Layer* L, const float* grad_out, float* grad_in, int batch, const NnConvFusion* f,
+    Context* ctx)
+{
+    const int* d = L->dim;
+    if (d[CD_MP]) {
+        conv_require_aligned(grad_out, "the output gradient");
+        nnk_conv_f32_input_grad(grad_in, grad_out, L->buf[CB_W], L->buf[CB_AUX], batch, d[CD_HI], d[CD_WI],
+            d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_P], f, ctx->stream);
+        return;
+    }
+    nnk_conv_input_grad(grad_in, grad_out, L->buf[CB_W], NULL, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT],
+        d[CD_K], d[CD_P], f, ctx->stream);
+}
+
 static void conv_fwd(Layer* L, const float* in, float* out, int batch, Context* ctx)
 {
     const int* d = L->dim;
@@ -407,8 +462,7 @@ static void conv_fwd(Layer* L, const float* in, float* out, int batch, Context* 
     float *w = L->buf[CB_W], *aux = L->buf[CB_AUX];
     if (d[CD_MP]) launch_weight_normalize(w, kg, d[CD_COUT], L->k[0], ctx->stream);
     if (d[CD_FWD] && !conv_gemm_path(L)) {
-        nnk_conv_forward(out, in, w, d[CD_MP] ? NULL : aux, d[CD_MP] ? aux : NULL, batch, d[CD_HI], d[CD_WI],
-            d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_S], d[CD_P], d[CD_HO], d[CD_WO], NULL, ctx->stream);
+        conv_fwd_cores(L, in, out, batch, NULL, ctx);
         return;
     }
     launch_im2col(L->buf[CB_COL], in, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_K], d[CD_S], d[CD_P], d[CD_HO],
@@ -427,35 +481,33 @@ static void conv_bwd(Layer* L, const float* in, const float* out, const float* g
     const int forced = conv_gemm_path(L);
     float *w = L->buf[CB_W], *gw = L->buf[CB_GW], *col = L->buf[CB_COL];
     float* gb = d[CD_MP] ? NULL : L->buf[CB_GAUX];
-    if (d[CD_WGRAD] && !forced) {
-        nnk_conv_weight_grad(gw, gb, in, grad_out, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K],
-            d[CD_S], d[CD_P], d[CD_HO], d[CD_WO], L->buf[CB_WGWS], ctx->stream);
-    } else {
+    if (!d[CD_WGRAD] || forced) {
         launch_im2col(col, in, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_K], d[CD_S], d[CD_P], d[CD_HO], d[CD_WO],
             ctx->stream);
         nn_gemm_dW(ctx->blas, 1.0f, col, grad_out, gw, rows, kg, d[CD_COUT]);
         if (gb) launch_bias_grad(gb, grad_out, rows, d[CD_COUT], ctx->stream);
+    } else if (d[CD_MP]) {
+        conv_require_aligned(in, "the forward input");
+        conv_require_aligned(grad_out, "the output gradient");
+        nnk_conv_f32_weight_grad(gw, in, grad_out, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K],
+            d[CD_S], d[CD_P], d[CD_HO], d[CD_WO], L->buf[CB_WGWS], ctx->stream);
+    } else {
+        nnk_conv_weight_grad(gw, gb, in, grad_out, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K],
+            d[CD_S], d[CD_P], d[CD_HO], d[CD_WO], L->buf[CB_WGWS], ctx->stream);
     }
-    if (d[CD_MP]) {
+    if (d[CD_MP])
         nnk_weight_normalize_backward_set(gw, w, L->buf[CB_AUX], L->buf[CB_GAUX], kg, d[CD_COUT],
             L->buf[CB_WNWS], ctx->stream);
-    }
     if (!grad_in) return;
-    const float* gain = d[CD_MP] ? L->buf[CB_AUX] : NULL;
-    const int by_cols = col && d[CD_DGRAD] && !forced &&
+    const int by_cols = !d[CD_MP] && col && d[CD_DGRAD] && !forced &&
                         nnk_conv_input_grad_by_columns(batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_P]);
     if (d[CD_DGRAD] && !by_cols && !forced) {
-        /* stride 1: dx = conv(dy, flipped kernel, pad K-1-pad), times the gain in mp mode */
-        nnk_conv_input_grad(grad_in, grad_out, w, gain, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K],
-            d[CD_P], NULL, ctx->stream);
+        conv_dgrad_cores(L, grad_out, grad_in, batch, NULL, ctx);
         return;
     }
-    if (by_cols) {
-        nnk_conv_input_grad(col, grad_out, w, gain, rows, 1, 1, kg, d[CD_COUT], 1, 0, NULL, ctx->stream);
-    } else {
-        nn_gemm_dX(ctx->blas, 1.0f, w, grad_out, col, rows, kg, d[CD_COUT]);
-        if (gain) launch_scale_by_scalar(col, gain, rows * kg, ctx->stream);
-    }
+    if (by_cols) nnk_conv_input_grad(col, grad_out, w, NULL, rows, 1, 1, kg, d[CD_COUT], 1, 0, NULL, ctx->stream);
+    else nn_gemm_dX(ctx->blas, 1.0f, w, grad_out, col, rows, kg, d[CD_COUT]);
+    if (d[CD_MP]) launch_scale_by_scalar(col, L->buf[CB_AUX], rows * kg, ctx->stream);
     launch_col2im_set(grad_in, col, batch, d[CD_HI], d[CD_WI], d[CD_CIN], d[CD_K], d[CD_S], d[CD_P], d[CD_HO],
         d[CD_WO], ctx->stream);
 }
@@ -475,14 +527,18 @@ static int conv_fused_bwd(const Layer* L)
 {
     return L->dim[CD_WGRAD] && L->dim[CD_DGRAD] && L->dim[CD_COUT] % 8 == 0 && !conv_gemm_path(L);
 }
+/* the kernels' epilogues: both activations, with a gain the blocks' own */
+static int conv_act_fuses(const Layer* L, Activation act)
+{
+    return act == ACT_MP_SILU || (act == ACT_SILU && !L->dim[CD_MP]);
+}
 
 static void conv_fused_forward(Layer* L, const float* in, float* out, int batch, const NnConvFusion* f, Context* ctx)
 {
     const int* d = L->dim;
-    float *w = L->buf[CB_W], *aux = L->buf[CB_AUX];
-    if (d[CD_MP]) launch_weight_normalize(w, d[CD_K] * d[CD_K] * d[CD_CIN], d[CD_COUT], L->k[0], ctx->stream);
-    nnk_conv_forward(out, in, w, d[CD_MP] ? NULL : aux, d[CD_MP] ? aux : NULL, batch, d[CD_HI], d[CD_WI],
-        d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_S], d[CD_P], d[CD_HO], d[CD_WO], f, ctx->stream);
+    if (d[CD_MP])
+        launch_weight_normalize(L->buf[CB_W], d[CD_K] * d[CD_K] * d[CD_CIN], d[CD_COUT], L->k[0], ctx->stream);
+    conv_fwd_cores(L, in, out, batch, f, ctx);
 }
 
 void conv2d_forward_residual(Module* m, const float* in, float* out, const float* res, float res_w, float out_w,
@@ -508,7 +564,7 @@ void conv2d_forward_modulate_act(Module* m, const float* in, float* out, float* 
 {
     Layer* L = as_layer(m);
     const int* d = L->dim;
-    if (!conv_fused_fwd(L) || (act != ACT_SILU && act != ACT_MP_SILU)) {
+    if (!conv_fused_fwd(L) || !conv_act_fuses(L, act)) {
         conv_fwd(L, in, out, batch, ctx);
         launch_spatial_modulate_act_forward(out2, out, cond, batch, d[CD_HO] * d[CD_WO], 1, d[CD_COUT], act,
             ctx->stream);
@@ -528,7 +584,7 @@ void conv2d_backward_act_residual(Module* m, const float* in, const float* grad_
     Layer* L = as_layer(m);
     const int* d = L->dim;
     const int n_in = batch * d[CD_HI] * d[CD_WI] * d[CD_CIN];
-    if (!conv_fused_bwd(L) || (act != ACT_SILU && act != ACT_MP_SILU)) {
+    if (!conv_fused_bwd(L) || !conv_act_fuses(L, act)) {
         conv_bwd(L, in, NULL, grad_out, tmp, batch, ctx);
         launch_activation_backward(grad_in, tmp, act_in, n_in, act, ctx->stream);
         launch_weighted_sum(grad_in, res, grad_in, res_w, 1.0f, n_in, ctx->stream);
@@ -543,8 +599,7 @@ void conv2d_backward_act_residual(Module* m, const float* in, const float* grad_
     f.res = res;
     f.res_w = res_w;
     f.out_w = 1.0f;
-    nnk_conv_input_grad(grad_in, grad_out, L->buf[CB_W], d[CD_MP] ? L->buf[CB_AUX] : NULL, batch, d[CD_HI],
-        d[CD_WI], d[CD_CIN], d[CD_COUT], d[CD_K], d[CD_P], &f, ctx->stream);
+    conv_dgrad_cores(L, grad_out, grad_in, batch, &f, ctx);
 }
 
 Module* conv2d_create(Context* ctx, int C_in, int C_out, int K, int stride, int pad, int H, int W, int max_batch,
@@ -565,10 +620,19 @@ Module* conv2d_create(Context* ctx, int C_in, int C_out, int K, int stride, int 
     d[CD_HO] = Ho;
     d[CD_WO] = Wo;
     d[CD_MP] = mp_mode != 0;
-    const int fits = nnk_conv_fits(max_batch, H, W, C_in, C_out, K, Ho, Wo);
-    d[CD_FWD] = fits;
-    d[CD_WGRAD] = fits;
-    d[CD_DGRAD] = fits && stride == 1 && pad <= K - 1;
+    if (mp_mode) {
+        const int forced = conv_implicit_forced();
+        d[CD_FWD] = nnhip_conv2d_implicit_supported(C_in, C_out) &&
+                    (forced || conv_f32_wins((long long)max_batch * Ho * Wo, C_out, kg));
+        d[CD_WGRAD] = nnhip_conv2d_wgrad_implicit_supported(C_in, C_out);
+        d[CD_DGRAD] = nnhip_conv2d_input_grad_implicit_supported(C_in, C_out, K, stride, pad) &&
+                      (forced || conv_f32_wins((long long)max_batch * H * W, C_in, K * K * C_out));
+    } else {
+        const int fits = nnk_conv_fits(max_batch, H, W, C_in, C_out, K, Ho, Wo);
+        d[CD_FWD] = fits;
+        d[CD_WGRAD] = fits;
+        d[CD_DGRAD] = fits && stride == 1 && pad <= K - 1;
+    }
     L->k[0] = 1e-4f;
     const int aux_n = mp_mode ? 1 : C_out;
     layer_buf(L, nw, 0);
@@ -579,11 +643,13 @@ Module* conv2d_create(Context* ctx, int C_in, int C_out, int K, int stride, int 
        input gradients that go by it; also where it is small or the channel
        counts are odd, so that the reference's sequence can be asked for later */
     const int need_col = !d[CD_FWD] || !d[CD_WGRAD] || !d[CD_DGRAD] || conv_gemm_forced() ||
-                         !nnhip_conv2d_implicit_supported(C_in, C_out) ||
-                         (size_t)max_batch * Ho * Wo * kg <= ((size_t)1 << 25) ||
-                         nnk_conv_input_grad_by_columns(max_batch, H, W, C_in, C_out, K, pad);
+                         (!mp_mode && (!nnhip_conv2d_implicit_supported(C_in, C_out) ||
+                                          (size_t)max_batch * Ho * Wo * kg <= ((size_t)1 << 25) ||
+                                          nnk_conv_input_grad_by_columns(max_batch, H, W, C_in, C_out, K, pad)));
     layer_buf(L, need_col ? (size_t)max_batch * Ho * Wo * kg : 0, 0);
-    layer_buf(L, d[CD_WGRAD] ? nnk_conv_weight_grad_workspace(max_batch, C_in, C_out, K, Ho, Wo) : 0, 0);
+    layer_buf(L, !d[CD_WGRAD] ? 0
+                     : mp_mode ? nnk_conv_f32_weight_grad_workspace(max_batch, C_in, C_out, K, Ho, Wo)
+                               : nnk_conv_weight_grad_workspace(max_batch, C_in, C_out, K, Ho, Wo), 0);
     layer_buf(L, mp_mode ? nnhip_weight_normalize_backward_workspace(C_out) : 0, 1);
     layer_param(L, CB_W, CB_GW, (int)nw);
     layer_param(L, CB_AUX, CB_GAUX, aux_n);
