@@ -21,6 +21,13 @@ struct ConvShape {
     FastDiv wo, ho;  // output pixel decode m -> (b, oh, ow)
 };
 
+// The tiled kernels address up to 31 rows of a weight, or 15 of dY, by 32-bit byte
+// offsets from the first: below this many channels in and out.  Wider shapes
+// take the small tiles (launchers of nn_hip.h) or the library's products (modules).
+constexpr int kMostChannels = 1 << 24;
+// Rows, channels and k that leave room in 32 bits for a tile past the end.
+constexpr long long kMostIndex = (1LL << 31) - 4096;
+
 // XCD-aware tile order.  Workgroups are dispatched round-robin over the
 // device's 8 XCDs (workgroup L on XCD L % 8), each with its own L2.  Tile
 // L' = xcd_order(L) gives XCD x a contiguous range of tiles, so tiles that

@@ -434,6 +434,8 @@ inline int conv_tile(const ConvShape& sh, bool flip, double* best_us = nullptr) 
     const double slices = (sh.Cin + 31) / 32;
     const double s16 = small_us(sh, flip, 16), s32 = small_us(sh, flip, 32);
     double best = s16 < s32 ? s16 : s32;
+    if (best_us) *best_us = best;
+    if (sh.Cin >= kMostChannels || sh.Cout >= kMostChannels) return 0;
     int bn = 0;
     for (const Tile& t : kTiles) {
         const double tiles = (double)((sh.M + kBM - 1) / kBM) * ((sh.Cout + t.bn - 1) / t.bn);
@@ -866,6 +868,7 @@ inline WgradPlan wgrad_plan(int M, int KKC, int Cout) {
 // us; dense [128, 512 -> 512]: 4.9, 14; [8, 28 x 28, 32 -> 32]: 59, 19; [16, 16 x
 // 16, 256 -> 256]: 113, 50.
 inline bool wgrad_small_wins(const ConvShape& sh) {
+    if (sh.Cout >= kMostChannels) return true;
     const double steps = (sh.M + 15) / 16, cells = (double)((sh.KKC + 31) / 32) * ((sh.Cout + 31) / 32);
     const double waves = waves_for((int)steps);
     const bool dense = sh.K == 1 && sh.stride == 1 && sh.pad == 0;  // no pixels to decode

@@ -98,9 +98,10 @@ void launch_conv2d_weight_grad_implicit(float* gW, const float* X, const float* 
 // ---- the host modules' products (conv_api.h) ----
 
 int nnk_conv_fits(int batch, int H, int W, int C_in, int C_out, int K, int H_out, int W_out) {
-    const long long most = 1LL << 31;
-    return (long long)batch * H * W * C_in < most && (long long)batch * H_out * W_out * C_out < most &&
-           (long long)K * K * C_in * C_out < most;
+    const long long most = 1LL << 31, kk = (long long)K * K * C_in;
+    return C_in < kMostChannels && C_out < kMostChannels && kk < kMostIndex && kk * C_out < most &&
+           (long long)batch * H * W < kMostIndex && (long long)batch * H * W * C_in < most &&
+           (long long)batch * H_out * W_out < kMostIndex && (long long)batch * H_out * W_out * C_out < most;
 }
 
 void nnk_conv_forward(float* y, const float* x, const float* w, const float* bias, const float* gain, int batch,
@@ -117,6 +118,18 @@ void nnk_conv_forward(float* y, const float* x, const float* w, const float* bia
     if (f) nnk_conv_forward_fused(y, x, w, sh, ep, *f, s);
     else conv_launch<false, kXeNone>(y, x, w, sh, ep, s);
     nnk_after_launch(what, s);
+}
+
+int nnk_conv_tile(int batch, int H, int W, int C_in, int C_out, int K, int stride, int pad, int flip) {
+    const int Ho = (H + 2 * pad - K) / stride + 1, Wo = (W + 2 * pad - K) / stride + 1;
+    return conv_tile(ConvShape{batch, H, W, C_in, C_out, K, stride, pad, Ho, Wo, batch * Ho * Wo, K * K * C_in,
+        FastDiv((uint32_t)Wo), FastDiv((uint32_t)Ho)}, flip != 0);
+}
+
+int nnk_conv_weight_grad_tiled(int batch, int H, int W, int C_in, int C_out, int K, int stride, int pad) {
+    const int Ho = (H + 2 * pad - K) / stride + 1, Wo = (W + 2 * pad - K) / stride + 1;
+    return !wgrad_small_wins(ConvShape{batch, H, W, C_in, C_out, K, stride, pad, Ho, Wo, batch * Ho * Wo, K * K * C_in,
+        FastDiv((uint32_t)Wo), FastDiv((uint32_t)Ho)});
 }
 
 static ConvShape dgrad_shape(int batch, int H, int W, int C_in, int C_out, int K, int pad) {

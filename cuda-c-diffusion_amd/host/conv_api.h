@@ -2,8 +2,8 @@
  * matrix-core kernels (csrc/igemm.h, csrc/k_conv_small.hip).  Unlike the
  * launchers of nn_hip.h they take any channel counts and 4-byte alignment, and
  * pick the tiled or the small-tile kernels by the work's size.  A dense layer
- * is a convolution with H = W = K = 1.  Tensors below 2^31 elements
- * (nnk_conv_fits); errors go to the launch layer's record.
+ * is a convolution with H = W = K = 1.  Tensors below 2^31 elements, fewer than
+ * 2^24 channels (nnk_conv_fits); errors go to the launch layer's record.
  */
 #ifndef NN_CONV_API_H
 #define NN_CONV_API_H
@@ -14,7 +14,7 @@
 extern "C" {
 #endif
 
-/* Whether every tensor of the convolution is within the index range. */
+/* Whether every tensor of the convolution is within the kernels' index range. */
 int nnk_conv_fits(int batch, int H, int W, int C_in, int C_out, int K, int H_out, int W_out);
 
 /* y = conv(x) + bias | * gain[0], then the neighbour in f (may be NULL) as in
@@ -35,6 +35,11 @@ int nnk_conv_input_grad_by_columns(int batch, int H, int W, int C_in, int C_out,
 void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy, int batch, int H, int W, int C_in,
     int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace, hipStream_t s);
 size_t nnk_conv_weight_grad_workspace(int batch, int C_in, int C_out, int K, int H_out, int W_out);
+/* Which kernel a forward takes (flip: an input gradient, given as the convolution
+   of dy with the flipped kernel): 128, 64 or 32 columns a workgroup, 0 the small
+   tiles; whether a weight gradient takes the tiled kernel. */
+int nnk_conv_tile(int batch, int H, int W, int C_in, int C_out, int K, int stride, int pad, int flip);
+int nnk_conv_weight_grad_tiled(int batch, int H, int W, int C_in, int C_out, int K, int stride, int pad);
 /* The same sums on the fp32 matrix cores, for conv2d modules with a gain
    (csrc/k_igemm_f32.hip says why): channel counts, alignment and index range as
    the launchers of nn_hip.h, outputs times gain[0].  f (may be NULL): res, or cond

@@ -176,3 +176,24 @@ def test_weight_gradient_workspace_serves_smaller_batches(nn, ci, co, k, hw):
         assert sizes == sorted(sizes)
         # as many parts as there are stages of 32 rows, until the device is full
         assert sizes[39] >= min(512 // (-(-k * k * ci // 128) * -(-co // 128)), -(-40 * hw * hw // 32)) * k * k * ci * co
+
+
+def test_convolution_kernels_stay_in_their_index_range(nn):
+    """The tiled kernels hold byte offsets of up to 31 rows in 32 bits (7 rows of
+    80 million floats wrap: the weight gradient then read one row eight times),
+    and rows, channels and k with a tile past the end.  Modules take the
+    library's products outside that range, launchers the small tiles, whose
+    offsets are elements."""
+    L = nn.lib()
+    I = ctypes.c_int
+    fits, tile, tiled = L.dll.nnk_conv_fits, L.dll.nnk_conv_tile, L.dll.nnk_conv_weight_grad_tiled
+    fits.argtypes, tile.argtypes, tiled.argtypes = [I] * 8, [I] * 9, [I] * 8
+    wide = 80_000_000
+    assert 28 * wide >= 2 ** 31 > 28 * (2 ** 24 - 1) and 2 ** 31 > 4 * (31 * (2 ** 24 - 1) + 8) + 32
+    assert not fits(8, 1, 1, 16, wide, 1, 1, 1) and not fits(8, 1, 1, wide, 16, 1, 1, 1)
+    assert tile(8, 1, 1, 16, wide, 1, 1, 0, 0) == 0 and tile(8, 1, 1, wide, 16, 1, 1, 0, 1) == 0
+    assert not tiled(8, 1, 1, 16, wide, 1, 1, 0)
+    assert fits(8, 1, 1, 16, 2 ** 24 - 1, 1, 1, 1) and fits(128, 32, 32, 128, 128, 3, 32, 32)
+    # one channel in and out: rows up to 2^31
+    assert not fits(2 ** 31 - 64, 1, 1, 1, 1, 1, 1, 1) and fits(2 ** 30, 1, 1, 1, 1, 1, 1, 1)
+    assert not fits(1, 1, 1, 1, 2 ** 31 - 1, 1, 1, 1)
