@@ -229,10 +229,11 @@ __global__ __launch_bounds__(kBgTpb) void column_sum(float* __restrict__ out, co
     const int lane = threadIdx.x & (kWave - 1);
     const int wid = threadIdx.x / kWave;
     const int n = blockIdx.x * kWave + lane;
-    const int r0 = blockIdx.y * chunk, r1 = min(rows, r0 + chunk);
+    // no index passes rows, which may lie just below 2^31
+    const uint32_t r0 = blockIdx.y * (uint32_t)chunk, r1 = r0 + min((uint32_t)chunk, (uint32_t)rows - r0);
     float s = 0.0f;
     if (n < N) {
-        int r = r0 + wid;
+        uint32_t r = r0 + wid;
         for (; r + (kBgBatch - 1) * kBgWaves < r1; r += kBgBatch * kBgWaves) {
             float v[kBgBatch];
 #pragma unroll
@@ -503,9 +504,9 @@ void launch_bias_grad(float* gb, const float* grad_out, int batch, int N, hipStr
     int chunk = batch;
     if (batch > kBgDirect) {
         const int most = cols < kBgBlocks / 2 ? kBgBlocks / cols : 2;
-        chunk = ((batch + most - 1) / most + per - 1) / per * per;
+        chunk = ((batch - 1) / most / per + 1) * per;
     }
-    const int chunks = (batch + chunk - 1) / chunk;
+    const int chunks = (batch - 1) / chunk + 1;
     // taken in every case, so that a capture is refused or not whatever the rows
     float* part = nnk_scratch_acquire((size_t)chunks * N, s, "launch_bias_grad");
     if (!part) return;

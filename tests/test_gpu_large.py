@@ -146,3 +146,15 @@ def test_north_star_full_size_groupnorm_silu(L, orc):
     # floor: the root of the summed squared per-sample terms bounds the sums' scale
     assert rel_err(ggd.download(), gg_ref, floor=np.sqrt(sq_g)) <= TOL
     assert rel_err(gbd.download(), gb_ref, floor=np.sqrt(sq_b)) <= TOL
+
+
+def test_bias_grad_rows_near_the_index_limit(L):
+    """One column of 2^31 - 1000 rows, 512 chunks: the last chunk ends within a chunk of 2^31."""
+    rows = 2 ** 31 - 1000
+    print(f"[case] bias grad of {rows} rows", flush=True)
+    g, out = L.alloc(rows), L.alloc(1)
+    L.nnhip_fill_f32(g.p, 1.0, rows, None)
+    L.launch_bias_grad(out.p, g.p, rows, 1, None)
+    L.sync()
+    # sums of ones: exact up to 2^24, 512 roundings after
+    assert abs(out.download()[0] / rows - 1) <= 512 * 2.0 ** -24
