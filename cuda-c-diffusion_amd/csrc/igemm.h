@@ -878,6 +878,12 @@ inline bool wgrad_small_wins(const ConvShape& sh) {
     return 4.0 + (trips > work ? trips : work) < 12.0 + stage * (p.rows / kWgM);
 }
 
+// Floats of partial sums that the tiled kernel leaves, 0 where it writes the result.
+inline size_t wgrad_scratch(const ConvShape& sh, bool sums) {
+    const WgradPlan p = wgrad_plan(sh.M, sh.KKC, sh.Cout);
+    return p.S > 1 ? (size_t)p.S * ((size_t)sh.KKC * sh.Cout + (sums ? sh.Cout : 0)) : 0;
+}
+
 // The tiled weight gradient of a checked, non-empty shape, and with gb non-null
 // the column sums of dY.
 inline void wgrad_run(const char* what, float* gW, float* gb, const float* X, const float* dY, const ConvShape& sh,

@@ -187,10 +187,19 @@ void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy,
     }
     const ConvShape sh{batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, batch * H_out * W_out, KKC,
         FastDiv((uint32_t)W_out), FastDiv((uint32_t)H_out)};
-    // a capture may not need scratch that the stream does not have: without a
-    // workspace it takes the small tiles, which need none
-    if (wgrad_small_wins(sh) || (!workspace && nnk_capturing(s))) nnk_wgrad_small(gw, gb, x, dy, sh, s);
-    else wgrad_run(what, gw, gb, x, dy, sh, workspace, s);
+    if (wgrad_small_wins(sh)) {
+        nnk_wgrad_small(gw, gb, x, dy, sh, s);
+    } else if (const size_t n = workspace || !nnk_capturing(s) ? 0 : wgrad_scratch(sh, gb != nullptr)) {
+        // A capture cannot allocate: the block that the same call left on the stream
+        // when it ran eagerly, so that a replay gives what it gave, bit for bit; a
+        // stream that has none takes the small tiles, which need none.
+        float* part = nnk_scratch_cached(n, s);
+        if (part) wgrad_run(what, gw, gb, x, dy, sh, part, s);
+        else nnk_wgrad_small(gw, gb, x, dy, sh, s);
+        nnk_scratch_release(part, s);
+    } else {
+        wgrad_run(what, gw, gb, x, dy, sh, workspace, s);
+    }
     nnk_after_launch(what, s);
 }
 

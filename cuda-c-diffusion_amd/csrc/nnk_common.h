@@ -456,6 +456,9 @@ int nnk_device_cus(hipStream_t s);
 void nnk_path_note(const char* fmt, ...);
 // Stream-ordered scratch for launchers that need partial sums.
 float* nnk_scratch_acquire(size_t n_floats, hipStream_t s, const char* what);
+// The stream's cached block if it is free and large enough, else null (no error, no
+// allocation); released as the other.
+float* nnk_scratch_cached(size_t n_floats, hipStream_t s);
 void nnk_scratch_release(float* p, hipStream_t s);
 void nnk_scratch_forget_stream(hipStream_t s);
 // Zero n_floats words of a workspace drawn from the scratch pool (a fill

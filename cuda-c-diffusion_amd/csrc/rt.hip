@@ -258,6 +258,23 @@ float* nnk_scratch_acquire(size_t n_floats, hipStream_t s, const char* what) {
     return static_cast<float*>(slot->p);
 }
 
+float* nnk_scratch_cached(size_t n_floats, hipStream_t s) {
+    int dev = -1;
+    const hipError_t ed = s ? hipStreamGetDevice(s, &dev) : hipGetDevice(&dev);
+    if (ed != hipSuccess) return nullptr;
+    const bool capturing = nnk_capturing(s);
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    for (int i = 0; i < g_nslots; ++i) {
+        Slot& slot = g_slots[i];
+        if (slot.dev != dev || slot.stream != s) continue;
+        if (slot.busy || slot.bytes < n_floats * sizeof(float) + 256) return nullptr;
+        if (capturing) slot.captured = true;
+        slot.busy = true;
+        return static_cast<float*>(slot.p);
+    }
+    return nullptr;
+}
+
 // Drop stream s's cached block (freed in stream order).  Called before the
 // stream goes away: a later stream could otherwise be handed the same handle
 // value, find the slot and use the block while the old stream's work on it is
