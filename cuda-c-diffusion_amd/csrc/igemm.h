@@ -5,6 +5,8 @@
 #pragma once
 #include <math.h>
 
+#include <atomic>
+
 #include "conv_common.h"
 
 namespace {
@@ -449,6 +451,23 @@ inline int conv_tile(const ConvShape& sh, bool flip, double* best_us = nullptr) 
     return bn;
 }
 
+// Raises kernel fn's LDS limit to 80 KB (two workgroups a CU) on the current device,
+// once a device: `done` has a bit for each that it was raised on.  False after
+// recording an error.
+inline bool lds_raised(const void* fn, std::atomic<unsigned long long>& done, const char* what) {
+    int dev = -1;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess && dev >= 64) e = hipErrorInvalidDevice;
+    if (e == hipSuccess && !(done.load(std::memory_order_relaxed) >> dev & 1)) {
+        e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 81920);
+        if (e == hipSuccess) done.fetch_or(1ull << dev, std::memory_order_relaxed);
+    }
+    if (e == hipSuccess) return true;
+    (void)hipGetLastError();
+    nnk_set_error((int)e, "%s: LDS of 80 KB on device %d: %s", what, dev, hipGetErrorString(e));
+    return false;
+}
+
 template <bool FLIP, int XE>
 void conv_launch(float* Y, const float* X, const float* Wt, const ConvShape& sh, const ConvEpi& ep, hipStream_t s) {
     const int BN = conv_tile(sh, FLIP), mode = conv_mode(sh, X, Wt, FLIP);
@@ -462,9 +481,8 @@ void conv_launch(float* Y, const float* X, const float* Wt, const ConvShape& sh,
 #define NNK_CONV(BN_, MODE_)                                                                                      \
     do {                                                                                                          \
         if (MODE_ == kHalo) {                                                                                     \
-            static const hipError_t once = hipFuncSetAttribute((const void*)conv_x3<BN_, MODE_, FLIP, XE>,         \
-                hipFuncAttributeMaxDynamicSharedMemorySize, 81920);                                               \
-            (void)once;                                                                                           \
+            static std::atomic<unsigned long long> done;                                                          \
+            if (!lds_raised((const void*)conv_x3<BN_, MODE_, FLIP, XE>, done, "convolution")) return;             \
         }                                                                                                         \
         conv_x3<BN_, MODE_, FLIP, XE><<<grid, kTpb, lds, s>>>(Y, X, Wt, sh, ep);                                  \
     } while (0)
@@ -906,11 +924,11 @@ inline void wgrad_run(const char* what, float* gW, float* gb, const float* X, co
     const dim3 grid((unsigned)((sh.KKC + 127) / 128) * (unsigned)((sh.Cout + BN - 1) / BN) * (unsigned)p.S);
     const int loads = sh.Cin % 2 || (uintptr_t)X % 8 ? kSingles : sh.Wo % 4 ? kPairs : kQuads;
     const size_t lds = (size_t)3 * kPlanes * (128 + BN) * kStage4 * sizeof(uint4);
+    bool ok = false;
 #define NNK_WGRAD(BN_, LOADS_)                                                                                 \
     do {                                                                                                       \
-        static const hipError_t once = hipFuncSetAttribute((const void*)igemm_wgrad<BN_, LOADS_>,              \
-            hipFuncAttributeMaxDynamicSharedMemorySize, 81920);                                                \
-        (void)once;                                                                                            \
+        static std::atomic<unsigned long long> done;                                                           \
+        if (!(ok = lds_raised((const void*)igemm_wgrad<BN_, LOADS_>, done, what))) break;                      \
         igemm_wgrad<BN_, LOADS_><<<grid, kTpb, lds, s>>>(part, sums, (size_t)n, X, dY, sh, p.rows);            \
     } while (0)
 #define NNK_WGRAD_LOADS(BN_)                            \
@@ -923,7 +941,7 @@ inline void wgrad_run(const char* what, float* gW, float* gb, const float* X, co
     else NNK_WGRAD_LOADS(64);
 #undef NNK_WGRAD_LOADS
 #undef NNK_WGRAD
-    if (p.S > 1) {
+    if (ok && p.S > 1) {
         if (p.S > kTallS && n <= kTallN)
             wgrad_reduce_tall<<<(unsigned)((n + kWave - 1) / kWave), 1024, 0, s>>>(gW, gb, part, p.S, n, nw);
         else wgrad_reduce<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(gW, gb, part, p.S, n, nw);
