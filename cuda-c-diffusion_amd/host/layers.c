@@ -620,19 +620,17 @@ Module* conv2d_create(Context* ctx, int C_in, int C_out, int K, int stride, int 
     d[CD_HO] = Ho;
     d[CD_WO] = Wo;
     d[CD_MP] = mp_mode != 0;
-    if (mp_mode) {
-        const int forced = conv_implicit_forced();
-        d[CD_FWD] = nnhip_conv2d_implicit_supported(C_in, C_out) &&
+    /* what the fp32 matrix-core kernels take, or would take of a plain module */
+    const int forced = conv_implicit_forced();
+    const int fwd = nnhip_conv2d_implicit_supported(C_in, C_out) &&
                     (forced || conv_f32_wins((long long)max_batch * Ho * Wo, C_out, kg));
-        d[CD_WGRAD] = nnhip_conv2d_wgrad_implicit_supported(C_in, C_out);
-        d[CD_DGRAD] = nnhip_conv2d_input_grad_implicit_supported(C_in, C_out, K, stride, pad) &&
+    const int wgrad = nnhip_conv2d_wgrad_implicit_supported(C_in, C_out);
+    const int dgrad = nnhip_conv2d_input_grad_implicit_supported(C_in, C_out, K, stride, pad) &&
                       (forced || conv_f32_wins((long long)max_batch * H * W, C_in, K * K * C_out));
-    } else {
-        const int fits = nnk_conv_fits(max_batch, H, W, C_in, C_out, K, Ho, Wo);
-        d[CD_FWD] = fits;
-        d[CD_WGRAD] = fits;
-        d[CD_DGRAD] = fits && stride == 1 && pad <= K - 1;
-    }
+    const int fits = nnk_conv_fits(max_batch, H, W, C_in, C_out, K, Ho, Wo);
+    d[CD_FWD] = mp_mode ? fwd : fits;
+    d[CD_WGRAD] = mp_mode ? wgrad : fits;
+    d[CD_DGRAD] = mp_mode ? dgrad : fits && stride == 1 && pad <= K - 1;
     L->k[0] = 1e-4f;
     const int aux_n = mp_mode ? 1 : C_out;
     layer_buf(L, nw, 0);
@@ -640,12 +638,11 @@ Module* conv2d_create(Context* ctx, int C_in, int C_out, int K, int stride, int 
     layer_buf(L, (size_t)aux_n, 1);
     layer_buf(L, (size_t)aux_n, 0);
     /* the im2col matrix, for what the matrix-core kernels do not take and for
-       input gradients that go by it; also where it is small or the channel
-       counts are odd, so that the reference's sequence can be asked for later */
-    const int need_col = !d[CD_FWD] || !d[CD_WGRAD] || !d[CD_DGRAD] || conv_gemm_forced() ||
-                         (!mp_mode && (!nnhip_conv2d_implicit_supported(C_in, C_out) ||
-                                          (size_t)max_batch * Ho * Wo * kg <= ((size_t)1 << 25) ||
-                                          nnk_conv_input_grad_by_columns(max_batch, H, W, C_in, C_out, K, pad)));
+       input gradients that go by columns.  Also where the fp32 kernels take
+       less: such modules always had it, and with it take NNHIP_CONV_PATH=gemm at
+       any call */
+    const int need_col = !fwd || !wgrad || !dgrad || conv_gemm_forced() || !d[CD_FWD] || !d[CD_WGRAD] || !d[CD_DGRAD] ||
+                         (!mp_mode && nnk_conv_input_grad_by_columns(max_batch, H, W, C_in, C_out, K, pad));
     layer_buf(L, need_col ? (size_t)max_batch * Ho * Wo * kg : 0, 0);
     layer_buf(L, !d[CD_WGRAD] ? 0
                      : mp_mode ? nnk_conv_f32_weight_grad_workspace(max_batch, C_in, C_out, K, Ho, Wo)

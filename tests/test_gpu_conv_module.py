@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 from helpers import TOL, assert_bits_equal
+from module_abi import Module
 from test_gpu_conv_split import _conv64
 
 pytestmark = pytest.mark.gpu
@@ -174,3 +175,27 @@ def test_rule_for_columns(L):
     assert not by(128, 32, 32, 128, 128, 3, 1)
     assert not by(64, 32, 32, 3, 64, 1, 0)       # one tap: nothing to sum
     assert not by(1 << 20, 64, 64, 3, 64, 3, 1)  # rows past 32 bits
+
+
+def test_module_holds_no_im2col_matrix(L):
+    """A convolution whose products all go by the kernels: weights, gradients and partial sums, without the 75 MB of
+    an im2col matrix that nothing reads."""
+    print("[case] conv module memory", flush=True)
+    hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+
+    def now():
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    small = Module(L, "conv2d_create", 8, 8, 1, 1, 0, 2, 2, 1, 0, 1.0)  # the context and what the library keeps for it
+    L.sync()
+    before = now()
+    m = L.dll.conv2d_create(C.byref(small.ctx), 128, 128, 3, 1, 1, 32, 32, 16, 0, C.c_float(1.0))
+    assert not L.dll.nnk_conv_input_grad_by_columns(16, 32, 32, 128, 128, 3, 1)
+    own = 2 * 4 * (9 * 128 * 128 + 128)
+    ws = L.dll.nnk_conv_weight_grad_workspace
+    ws.argtypes, ws.restype = [I] * 6, C.c_size_t
+    assert before - now() <= own + 4 * ws(16, 128, 128, 3, 32, 32) + (8 << 20)  # allocation granularity
+    m.contents.free(m)
+    small.free()
