@@ -46,8 +46,7 @@ def bc(L):
                          ids=["small", "streaming-gn"])
 def test_ddpm_block_graph_replay(bc, shape):
     """The fused DDPM block's forward + backward (lent workspaces, implicit
-    convolutions, streaming GroupNorm at the larger shape, rocBLAS for the
-    time projection) captured into one HIP graph: every replay reproduces the
+    convolutions, streaming GroupNorm at the larger shape) captured into one HIP graph: every replay reproduces the
     eager output, input gradient and embedding gradient bit for bit, with an
     eager forward on the same buffers between replays."""
     print(f"[case] DDPM block graph {shape}", flush=True)
