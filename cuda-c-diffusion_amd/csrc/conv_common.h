@@ -41,10 +41,11 @@ __device__ __forceinline__ int xcd_order(int L, int total) {
 // ---------------------------------------------------------------------------
 // fp32 operands on the bf16 matrix cores.  v = p0 + p1 + p2 with p0 = bf16(v),
 // p1 = bf16(v - p0), p2 = v - p0 - p1: 8 + 8 + 8 significand bits, so the sum
-// is exact for every v of 2^-110 and above (below it p2 reaches under the
-// smallest subnormal bf16).  a b is then the sum of the products p_i q_j; the
-// six with i + j <= 2 are taken, the other three are below 2^-25 |a b|.  Each
-// product of two bf16 is exact and the matrix core adds in fp32.
+// is exact for every v of 2^-103 and above (below it p2 may lie under the
+// smallest normal number).  a b is then the sum of the products p_i q_j; the
+// six with i + j <= 2 are taken, the other three are each below 2^-25 |a b|, below
+// 2^-24 together.  Each product of two bf16 is exact and the matrix core adds in
+// fp32.  What smaller operands lose: split_failed.
 // ---------------------------------------------------------------------------
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -108,26 +109,63 @@ __device__ __forceinline__ void products(const uint4 (&a)[kPlanes][T], const uin
             for (int u = 0; u < U; ++u) mfma(a[PI[x]][t], b[PJ[x]][u], x ? cor[t][u] : acc[t][u]);
 }
 
-// Whether a wave's results must be formed again from the unsplit operands: a
-// value that is not finite (an infinite or NaN operand, or one that rounds to
-// infinity in bf16, splits into NaN planes), or values all so small that an
-// operand may lie below the split's range.
+// Whether a wave's results must be formed again from the unsplit operands.  Not
+// finite: an infinite or NaN operand, or one that rounds to infinity in bf16,
+// splits into NaN planes.  Small: an operand below 2^-103 may lose up to 2^-126, so
+// n products with operands up to b lose up to 2^-126 n b of a result.  A result
+// below 2^-80 is formed again, which leaves 2^-24 of a result for n b up to 2^22; so
+// is a row or column of the tile that has none of 2^-55, as one has whose operands
+// are all that small: 2^-24 of the row's largest for n b up to 2^47.  What is left
+// is an operand below 2^-103 in sums with some of 2^47 / n and above.  A zero is
+// taken for one (a masked row, an operand of zeros), also where all operands of a
+// sum lie below 2^-126.
 template <int T, int U, class V>
 __device__ __forceinline__ bool split_failed(const V (&acc)[T][U]) {
-    bool bad = false;
-    float mx = 0.0f;
+    constexpr int N = (int)(sizeof(V) / sizeof(float)), L = N == 16 ? 32 : 16;  // L lanes to a row
+    constexpr float kElement = 0x1p-80f, kLine = 0x1p-55f;
+    // of the bits of |v|, and of those less one, which leaves zeros out (a wave whose
+    // taps lie outside the image has many)
+    uint32_t most = 0, least = ~0u;
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int r = 0; r < (int)(sizeof(V) / sizeof(float)); ++r) {
-                const float v = fabsf(acc[t][u][r]);
-                bad |= !(v <= 3.402823466e38f);
-                mx = fmaxf(mx, v);
+            for (int r = 0; r < N; ++r) {
+                const float v = acc[t][u][r];
+                const uint32_t b = __float_as_uint(v) & 0x7fffffffu;
+                most = max(most, b);
+                least = min(least, b - 1);
             }
-    if (__any(bad)) return true;
-    return !__any(mx >= 0x1p-80f) && __any(mx > 0.0f);
+    bool bad = most >= 0x7f800000u;
+    if (!__any(bad || least < __float_as_uint(kLine) - 1)) return false;
+    auto small = [](float v, float limit) { return v > 0.0f && v < limit; };
+    float column[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) column[u] = 0.0f;
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int r = 0; r < N; ++r) {
+            float row = 0.0f;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float v = fabsf(acc[t][u][r]);
+                bad |= small(v, kElement);
+                row = fmaxf(row, v);
+                column[u] = fmaxf(column[u], v);
+            }
+#pragma unroll
+            for (int o = 1; o < L; o <<= 1) row = fmaxf(row, __shfl_xor(row, o, kWave));
+            bad |= small(row, kLine);
+        }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int o = L; o < kWave; o <<= 1) column[u] = fmaxf(column[u], __shfl_xor(column[u], o, kWave));
+        bad |= small(column[u], kLine);
+    }
+    return __any(bad);
 }
 
 // Fused neighbours of the forward / input-gradient kernel (bit flags), with v

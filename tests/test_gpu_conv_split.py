@@ -120,6 +120,19 @@ def test_scales_outside_the_split(L, rng, scale):
     _check(_forward(L, x, w, 3, 1, 1), *_conv64(x, w, 3, 1, 1))
 
 
+@pytest.mark.parametrize("images,weight", [((1.0, 1e-36), 1.0), ((1e-35, 1.0), 1.0), ((1e-36, 1e-36), 1e15), ((1.0, 1e-35), 1e12)],
+                         ids=str)
+def test_small_operands_beside_others(L, rng, images, weight):
+    """Operands below the split's range where not all results are small: an image of
+    them beside an ordinary one in the same tile, and against large weights."""
+    print(f"[case] conv of images scaled by {images}, weight by {weight}", flush=True)
+    x = rng.standard_normal((2, 5, 5, 64)).astype(np.float32)
+    for b, f in enumerate(images):
+        x[b] *= np.float32(f)
+    w = (rng.standard_normal((9 * 64, 128)) / 24 * weight).astype(np.float32)
+    _check(_forward(L, x, w, 3, 1, 1), *_conv64(x, w, 3, 1, 1))
+
+
 def test_outputs_are_not_shifted(L, rng):
     """The matrix core cuts addends off towards minus infinity; with the small
     products in the large one's accumulator the mean of the outputs' errors is
