@@ -302,6 +302,13 @@ inline double small_us(const ConvShape& sh, bool flip, int t) {
 }  // namespace conv
 }  // namespace nnk
 
+// Which form of a kernel runs, where a caller names it: columns a workgroup (0: the
+// small tiles) and the staging (conv_x3's MODE, igemm_wgrad's LOADS; a more special
+// one than the shape allows is not taken).  Negative: by the rules.
+struct ConvPick {
+    int columns = -1, staging = -1;
+};
+
 // Few output tiles: 32 x 32 outputs a workgroup, the k range split over its
 // waves (k_conv_small.hip).  `flip`, `xe`: as conv_x3's parameters.
 void nnk_conv_small(bool flip, int xe, float* Y, const float* X, const float* Wt, const nnk::conv::ConvShape& sh,
@@ -311,6 +318,6 @@ void nnk_wgrad_small(float* gW, float* gb, const float* X, const float* dY, cons
     hipStream_t s);
 // The tiled kernels with a neighbour folded in, of checked shapes (k_igemm_fused.hip).
 void nnk_conv_forward_fused(float* Y, const float* X, const float* Wt, const nnk::conv::ConvShape& sh,
-    nnk::conv::ConvEpi ep, const NnConvFusion& f, hipStream_t s);
+    nnk::conv::ConvEpi ep, const NnConvFusion& f, hipStream_t s, ConvPick pick = {});
 void nnk_conv_input_grad_fused(float* dX, const float* dY, const float* Wt, const nnk::conv::ConvShape& sh,
-    nnk::conv::ConvEpi ep, const NnConvFusion& f, hipStream_t s);
+    nnk::conv::ConvEpi ep, const NnConvFusion& f, hipStream_t s, ConvPick pick = {});

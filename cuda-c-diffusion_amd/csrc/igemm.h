@@ -294,6 +294,9 @@ __global__ __launch_bounds__(kTpb, 2) void conv_x3(float* __restrict__ Y, const 
             if (cs) __syncthreads();  // the slice before has been read
             stage_halo(cs);
             __syncthreads();
+            // vmcnt(0): the slice's first weights came with the rows, and the waits in the
+            // loop over taps are for its own loads (to the compiler, else, for all of them)
+            __builtin_amdgcn_s_waitcnt(0x0f70);
             rows_of(0, 0, as);
             frag(2, as, 0);
             frag(1, as, 0);
@@ -469,8 +472,10 @@ inline bool lds_raised(const void* fn, std::atomic<unsigned long long>& done, co
 }
 
 template <bool FLIP, int XE>
-void conv_launch(float* Y, const float* X, const float* Wt, const ConvShape& sh, const ConvEpi& ep, hipStream_t s) {
-    const int BN = conv_tile(sh, FLIP), mode = conv_mode(sh, X, Wt, FLIP);
+void conv_launch(float* Y, const float* X, const float* Wt, const ConvShape& sh, const ConvEpi& ep, hipStream_t s,
+    ConvPick pick = {}) {
+    const int BN = pick.columns >= 0 ? pick.columns : conv_tile(sh, FLIP);
+    const int own = conv_mode(sh, X, Wt, FLIP), mode = own > pick.staging ? own : pick.staging;
     if (BN == 0) {
         nnk_conv_small(FLIP, XE, Y, X, Wt, sh, ep, s);
         return;
@@ -905,7 +910,7 @@ inline size_t wgrad_scratch(const ConvShape& sh, bool sums) {
 // The tiled weight gradient of a checked, non-empty shape, and with gb non-null
 // the column sums of dY.
 inline void wgrad_run(const char* what, float* gW, float* gb, const float* X, const float* dY, const ConvShape& sh,
-    float* workspace, hipStream_t s) {
+    float* workspace, hipStream_t s, ConvPick pick = {}) {
     const WgradPlan p = wgrad_plan(sh.M, sh.KKC, sh.Cout);
     const long long nw = (long long)sh.KKC * sh.Cout, n = nw + (gb ? sh.Cout : 0);
     float *part = gW, *sums = gb;
@@ -922,7 +927,8 @@ inline void wgrad_run(const char* what, float* gW, float* gb, const float* X, co
     }
     const int BN = tile_n(sh.Cout);
     const dim3 grid((unsigned)((sh.KKC + 127) / 128) * (unsigned)((sh.Cout + BN - 1) / BN) * (unsigned)p.S);
-    const int loads = sh.Cin % 2 || (uintptr_t)X % 8 ? kSingles : sh.Wo % 4 ? kPairs : kQuads;
+    const int own = sh.Cin % 2 || (uintptr_t)X % 8 ? kSingles : sh.Wo % 4 ? kPairs : kQuads;
+    const int loads = own > pick.staging ? own : pick.staging;
     const size_t lds = (size_t)3 * kPlanes * (128 + BN) * kStage4 * sizeof(uint4);
     bool ok = false;
 #define NNK_WGRAD(BN_, LOADS_)                                                                                 \

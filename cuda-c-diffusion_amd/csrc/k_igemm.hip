@@ -104,9 +104,9 @@ int nnk_conv_fits(int batch, int H, int W, int C_in, int C_out, int K, int H_out
            (long long)batch * H_out * W_out < kMostIndex && (long long)batch * H_out * W_out * C_out < most;
 }
 
-void nnk_conv_forward(float* y, const float* x, const float* w, const float* bias, const float* gain, int batch,
-    int H, int W, int C_in, int C_out, int K, int stride, int pad, int H_out, int W_out, const NnConvFusion* f,
-    hipStream_t s) {
+void nnk_conv_forward_as(int columns, int staging, float* y, const float* x, const float* w, const float* bias,
+    const float* gain, int batch, int H, int W, int C_in, int C_out, int K, int stride, int pad, int H_out, int W_out,
+    const NnConvFusion* f, hipStream_t s) {
     const char* what = "conv2d forward";
     NNK_REQUIRE(nnk_conv_fits(batch, H, W, C_in, C_out, K, H_out, W_out), what, "%s: tensor exceeds the 32-bit index range", what);
     if (batch <= 0) return;
@@ -115,9 +115,16 @@ void nnk_conv_forward(float* y, const float* x, const float* w, const float* bia
     ConvEpi ep{};
     ep.bias = bias;
     ep.gain = gain;
-    if (f) nnk_conv_forward_fused(y, x, w, sh, ep, *f, s);
-    else conv_launch<false, kXeNone>(y, x, w, sh, ep, s);
+    const ConvPick pick{columns, staging};
+    if (f) nnk_conv_forward_fused(y, x, w, sh, ep, *f, s, pick);
+    else conv_launch<false, kXeNone>(y, x, w, sh, ep, s, pick);
     nnk_after_launch(what, s);
+}
+
+void nnk_conv_forward(float* y, const float* x, const float* w, const float* bias, const float* gain, int batch,
+    int H, int W, int C_in, int C_out, int K, int stride, int pad, int H_out, int W_out, const NnConvFusion* f,
+    hipStream_t s) {
+    nnk_conv_forward_as(-1, -1, y, x, w, bias, gain, batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, f, s);
 }
 
 int nnk_conv_tile(int batch, int H, int W, int C_in, int C_out, int K, int stride, int pad, int flip) {
@@ -155,17 +162,23 @@ int nnk_conv_input_grad_by_columns(int batch, int H, int W, int C_in, int C_out,
     return 1.25 * (product + pass) + 2.0 < direct;
 }
 
-void nnk_conv_input_grad(float* dx, const float* dy, const float* w, const float* gain, int batch, int H, int W,
-    int C_in, int C_out, int K, int pad, const NnConvFusion* f, hipStream_t s) {
+void nnk_conv_input_grad_as(int columns, int staging, float* dx, const float* dy, const float* w, const float* gain,
+    int batch, int H, int W, int C_in, int C_out, int K, int pad, const NnConvFusion* f, hipStream_t s) {
     const char* what = "conv2d input gradient";
     NNK_REQUIRE(nnk_conv_fits(batch, H, W, C_in, C_out, K, H + 2 * pad - K + 1, W + 2 * pad - K + 1), what, "%s: tensor exceeds the 32-bit index range", what);
     if (batch <= 0) return;
     const ConvShape sh = dgrad_shape(batch, H, W, C_in, C_out, K, pad);
     ConvEpi ep{};
     ep.gain = gain;
-    if (f) nnk_conv_input_grad_fused(dx, dy, w, sh, ep, *f, s);
-    else conv_launch<true, kXeNone>(dx, dy, w, sh, ep, s);
+    const ConvPick pick{columns, staging};
+    if (f) nnk_conv_input_grad_fused(dx, dy, w, sh, ep, *f, s, pick);
+    else conv_launch<true, kXeNone>(dx, dy, w, sh, ep, s, pick);
     nnk_after_launch(what, s);
+}
+
+void nnk_conv_input_grad(float* dx, const float* dy, const float* w, const float* gain, int batch, int H, int W,
+    int C_in, int C_out, int K, int pad, const NnConvFusion* f, hipStream_t s) {
+    nnk_conv_input_grad_as(-1, -1, dx, dy, w, gain, batch, H, W, C_in, C_out, K, pad, f, s);
 }
 
 size_t nnk_conv_weight_grad_workspace(int batch, int C_in, int C_out, int K, int H_out, int W_out) {
@@ -175,8 +188,9 @@ size_t nnk_conv_weight_grad_workspace(int batch, int C_in, int C_out, int K, int
     return S > 1 ? (size_t)S * (K * K * C_in + 1) * C_out : 0;
 }
 
-void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy, int batch, int H, int W, int C_in,
-    int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace, hipStream_t s) {
+void nnk_conv_weight_grad_as(int tiled, int loads, float* gw, float* gb, const float* x, const float* dy, int batch,
+    int H, int W, int C_in, int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace,
+    hipStream_t s) {
     const char* what = "conv2d weight gradient";
     NNK_REQUIRE(nnk_conv_fits(batch, H, W, C_in, C_out, K, H_out, W_out), what, "%s: tensor exceeds the 32-bit index range", what);
     const int KKC = K * K * C_in;
@@ -187,20 +201,25 @@ void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy,
     }
     const ConvShape sh{batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, batch * H_out * W_out, KKC,
         FastDiv((uint32_t)W_out), FastDiv((uint32_t)H_out)};
-    if (wgrad_small_wins(sh)) {
+    if (tiled < 0 ? wgrad_small_wins(sh) : !tiled) {
         nnk_wgrad_small(gw, gb, x, dy, sh, s);
     } else if (const size_t n = workspace || !nnk_capturing(s) ? 0 : wgrad_scratch(sh, gb != nullptr)) {
         // A capture cannot allocate: the block that the same call left on the stream
         // when it ran eagerly, so that a replay gives what it gave, bit for bit; a
         // stream that has none takes the small tiles, which need none.
         float* part = nnk_scratch_cached(n, s);
-        if (part) wgrad_run(what, gw, gb, x, dy, sh, part, s);
+        if (part) wgrad_run(what, gw, gb, x, dy, sh, part, s, ConvPick{-1, loads});
         else nnk_wgrad_small(gw, gb, x, dy, sh, s);
         nnk_scratch_release(part, s);
     } else {
-        wgrad_run(what, gw, gb, x, dy, sh, workspace, s);
+        wgrad_run(what, gw, gb, x, dy, sh, workspace, s, ConvPick{-1, loads});
     }
     nnk_after_launch(what, s);
+}
+
+void nnk_conv_weight_grad(float* gw, float* gb, const float* x, const float* dy, int batch, int H, int W, int C_in,
+    int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace, hipStream_t s) {
+    nnk_conv_weight_grad_as(-1, -1, gw, gb, x, dy, batch, H, W, C_in, C_out, K, stride, pad, H_out, W_out, workspace, s);
 }
 
 }  // extern "C"

@@ -20,7 +20,7 @@ bool act_fusable(int act) { return act == ACT_SILU || act == ACT_MP_SILU; }
 }  // namespace
 
 void nnk_conv_forward_fused(float* Y, const float* X, const float* Wt, const ConvShape& sh, ConvEpi ep,
-    const NnConvFusion& f, hipStream_t s) {
+    const NnConvFusion& f, hipStream_t s, ConvPick pick) {
     ep.res = f.res;
     ep.wa = f.res_w;
     ep.wb = f.out_w;
@@ -28,18 +28,18 @@ void nnk_conv_forward_fused(float* Y, const float* X, const float* Wt, const Con
     ep.y2 = f.y2;
     ep.hw = FastDiv((uint32_t)(sh.Ho * sh.Wo));
     ep.mp = f.act == ACT_MP_SILU;
-    if (f.res) conv_launch<false, kXeRes>(Y, X, Wt, sh, ep, s);
-    else conv_launch<false, kXeMod>(Y, X, Wt, sh, ep, s);
+    if (f.res) conv_launch<false, kXeRes>(Y, X, Wt, sh, ep, s, pick);
+    else conv_launch<false, kXeMod>(Y, X, Wt, sh, ep, s, pick);
 }
 
 void nnk_conv_input_grad_fused(float* dX, const float* dY, const float* Wt, const ConvShape& sh, ConvEpi ep,
-    const NnConvFusion& f, hipStream_t s) {
+    const NnConvFusion& f, hipStream_t s, ConvPick pick) {
     ep.res = f.res;
     ep.xa = f.act_in;
     ep.wa = f.res_w;
     ep.wb = f.out_w;
     ep.mp = f.act == ACT_MP_SILU;
-    conv_launch<true, kXeActG | kXeRes>(dX, dY, Wt, sh, ep, s);
+    conv_launch<true, kXeActG | kXeRes>(dX, dY, Wt, sh, ep, s, pick);
 }
 
 extern "C" {

@@ -40,6 +40,18 @@ size_t nnk_conv_weight_grad_workspace(int batch, int C_in, int C_out, int K, int
    tiles; whether a weight gradient takes the tiled kernel. */
 int nnk_conv_tile(int batch, int H, int W, int C_in, int C_out, int K, int stride, int pad, int flip);
 int nnk_conv_weight_grad_tiled(int batch, int H, int W, int C_in, int C_out, int K, int stride, int pad);
+/* The three products in a named form, for tests: columns as nnk_conv_tile gives
+   them, tiled as nnk_conv_weight_grad_tiled, staging 0 halo rows, 1 gathered, 2
+   ragged, loads 0 fours, 1 pairs, 2 singles of pixels (a more special one than the
+   shape allows is not taken); negative: as the call without a name. */
+void nnk_conv_forward_as(int columns, int staging, float* y, const float* x, const float* w, const float* bias,
+    const float* gain, int batch, int H, int W, int C_in, int C_out, int K, int stride, int pad, int H_out, int W_out,
+    const NnConvFusion* f, hipStream_t s);
+void nnk_conv_input_grad_as(int columns, int staging, float* dx, const float* dy, const float* w, const float* gain,
+    int batch, int H, int W, int C_in, int C_out, int K, int pad, const NnConvFusion* f, hipStream_t s);
+void nnk_conv_weight_grad_as(int tiled, int loads, float* gw, float* gb, const float* x, const float* dy, int batch,
+    int H, int W, int C_in, int C_out, int K, int stride, int pad, int H_out, int W_out, float* workspace,
+    hipStream_t s);
 /* The same sums on the fp32 matrix cores, for conv2d modules with a gain
    (csrc/k_igemm_f32.hip says why): channel counts, alignment and index range as
    the launchers of nn_hip.h, outputs times gain[0].  f (may be NULL): res, or cond

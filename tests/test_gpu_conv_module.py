@@ -144,8 +144,10 @@ def test_small_tiles_fused_epilogues(L, nn, rng, geom):
 COLUMNS = [
     # B, H, W, C_in, C_out, K, stride, pad, mp: input gradients by columns
     (64, 32, 32, 3, 64, 3, 1, 1, 0),   # an image in
-    (20, 11, 11, 8, 448, 5, 1, 2, 1),  # a long k range, gain in the product's epilogue
+    (20, 11, 11, 8, 448, 5, 1, 2, 1),  # a long k range, with a gain: the library's products
+    (20, 11, 11, 8, 448, 5, 1, 2, 0),  # ... and without
     (3, 9, 8, 40, 24, 3, 2, 1, 1),     # strided: the library product
+    (3, 9, 8, 40, 24, 3, 2, 1, 0),
     (2, 10, 7, 5, 33, 5, 3, 0, 0),     # stride past the padding: pixels that no column reaches
 ]
 
