@@ -28,6 +28,31 @@ struct Slab {
     FastDiv dcw, dcpg;
 };
 
+// Total of a and b over the workgroup, on every thread: a slab of one group (ONE)
+// needs no sums by channel for it.  One thread adding a group's channels one by
+// one took longer than all else from about 100 channels on: forward + backward
+// [1, 1, 1, 1024] in one group 48 -> 17 us, [64, 8, 8, 1000] 111 -> 69.  l is [2][TPB /
+// 64]; the barriers order it after earlier uses of l.
+template <int TPB>
+__device__ __forceinline__ void slab_sum2(float& a, float& b, float* l) {
+    a = wave_sum(a);
+    b = wave_sum(b);
+    const int w = threadIdx.x / kWave;
+    __syncthreads();
+    if (threadIdx.x % kWave == 0) {
+        l[w] = a;
+        l[TPB / kWave + w] = b;
+    }
+    __syncthreads();
+    a = l[0];
+    b = l[TPB / kWave];
+#pragma unroll
+    for (int i = 1; i < TPB / kWave; ++i) {
+        a += l[i];
+        b += l[TPB / kWave + i];
+    }
+}
+
 // red[0..TPB) holds the threads' values (0 past pstep * cw); leaves in out[s *
 // cw + c], s < seg, the sums of channel c over the pixels s, s + seg, ...
 __device__ __forceinline__ void channel_segments(float* out, const float* red, const Slab& sl) {
@@ -41,7 +66,7 @@ __device__ __forceinline__ void channel_segments(float* out, const float* red, c
     }
 }
 
-template <int TPB, int NV, int ACT>
+template <int TPB, int NV, bool ONE, int ACT>
 __global__ __launch_bounds__(TPB) void gn_fwd_slab(float* __restrict__ y, float* __restrict__ mu_out,
     float* __restrict__ rstd_out, const float* __restrict__ x, const float* __restrict__ gamma,
     const float* __restrict__ beta, Slab sl, float eps) {
@@ -66,6 +91,11 @@ __global__ __launch_bounds__(TPB) void gn_fwd_slab(float* __restrict__ y, float*
     const float n = (float)(sl.HW * sl.cpg);
     // the group's total of s, per thread's own group
     auto group_total = [&](float s) {
+        if constexpr (ONE) {
+            float z = 0.0f;
+            slab_sum2<TPB>(s, z, red);
+            return s;
+        }
         __syncthreads();
         red[threadIdx.x] = s;
         __syncthreads();
@@ -111,7 +141,7 @@ __global__ __launch_bounds__(TPB) void gn_fwd_slab(float* __restrict__ y, float*
     }
 }
 
-template <int TPB, int NV, int ACT>
+template <int TPB, int NV, bool ONE, int ACT>
 __global__ __launch_bounds__(TPB) void gn_bwd_slab(float* __restrict__ dx, float* __restrict__ part_g,
     float* __restrict__ part_b, const float* __restrict__ dy, const float* __restrict__ x,
     const float* __restrict__ gamma, const float* __restrict__ beta, const float* __restrict__ mu,
@@ -165,8 +195,8 @@ __global__ __launch_bounds__(TPB) void gn_bwd_slab(float* __restrict__ dx, float
     channel_segments(part[1], red[1], sl);
     __syncthreads();
     // channel totals (into red), then the group's sums of d gamma and of d gamma xhat
+    float a = 0.0f, e = 0.0f;
     if ((int)threadIdx.x < ng * sl.cpg) {
-        float a = 0.0f, e = 0.0f;
         for (int q = 0; q < sl.seg; ++q) {
             a += part[0][q * sl.cw + (int)threadIdx.x];
             e += part[1][q * sl.cw + (int)threadIdx.x];
@@ -174,22 +204,30 @@ __global__ __launch_bounds__(TPB) void gn_bwd_slab(float* __restrict__ dx, float
         const int cc = g0 * sl.cpg + (int)threadIdx.x;
         part_g[(size_t)b * sl.C + cc] = a;
         part_b[(size_t)b * sl.C + cc] = e;
-        red[0][threadIdx.x] = a * gamma[cc];
-        red[1][threadIdx.x] = e * gamma[cc];
+        a *= gamma[cc];
+        e *= gamma[cc];
+        red[0][threadIdx.x] = a;
+        red[1][threadIdx.x] = e;
     }
-    __syncthreads();
-    if ((int)threadIdx.x < ng) {
-        float a = 0.0f, e = 0.0f;
-        for (int i = 0; i < sl.cpg; ++i) {
-            a += red[0][(int)threadIdx.x * sl.cpg + i];
-            e += red[1][(int)threadIdx.x * sl.cpg + i];
+    if constexpr (ONE) {
+        slab_sum2<TPB>(a, e, stat[0]);
+    } else {
+        __syncthreads();
+        if ((int)threadIdx.x < ng) {
+            a = e = 0.0f;
+            for (int i = 0; i < sl.cpg; ++i) {
+                a += red[0][(int)threadIdx.x * sl.cpg + i];
+                e += red[1][(int)threadIdx.x * sl.cpg + i];
+            }
+            stat[0][threadIdx.x] = a;
+            stat[1][threadIdx.x] = e;
         }
-        stat[0][threadIdx.x] = a;
-        stat[1][threadIdx.x] = e;
+        __syncthreads();
+        a = stat[0][gl];
+        e = stat[1][gl];
     }
-    __syncthreads();
     const float inv_n = 1.0f / (float)(sl.HW * sl.cpg);
-    const float pgx = stat[0][gl], m1 = stat[1][gl] * inv_n;
+    const float pgx = a, m1 = e * inv_n;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const int p = (int)p0 + k * sl.pstep;
@@ -244,12 +282,18 @@ SlabPlan plan(int B, int G, int HW, int C) {
 
 bool nnk_gn_slab_takes(int HW, int C, int G) { return C / G <= 1024 && HW <= 1 << 30; }
 
-#define NNK_SLAB(KERNEL, ...)                                                                  \
-    NNK_ACT_DISPATCH(act, A, {                                                                 \
-        if (p.cfg == 0) KERNEL<256, 4, A><<<p.grid, 256, 0, s>>>(__VA_ARGS__);                 \
-        else if (p.cfg == 1) KERNEL<256, 16, A><<<p.grid, 256, 0, s>>>(__VA_ARGS__);           \
-        else if (p.cfg == 2) KERNEL<1024, 16, A><<<p.grid, 1024, 0, s>>>(__VA_ARGS__);         \
-        else KERNEL<1024, 32, A><<<p.grid, 1024, 0, s>>>(__VA_ARGS__);                         \
+// (a slab of one group has kernels of its own: the others lose 4 % to the branch)
+#define NNK_SLAB_ONE(KERNEL, TPB_, NV_, ...)                                              \
+    do {                                                                                 \
+        if (p.sl.gb == 1) KERNEL<TPB_, NV_, true, A><<<p.grid, TPB_, 0, s>>>(__VA_ARGS__); \
+        else KERNEL<TPB_, NV_, false, A><<<p.grid, TPB_, 0, s>>>(__VA_ARGS__);             \
+    } while (0)
+#define NNK_SLAB(KERNEL, ...)                                             \
+    NNK_ACT_DISPATCH(act, A, {                                            \
+        if (p.cfg == 0) NNK_SLAB_ONE(KERNEL, 256, 4, __VA_ARGS__);        \
+        else if (p.cfg == 1) NNK_SLAB_ONE(KERNEL, 256, 16, __VA_ARGS__);  \
+        else if (p.cfg == 2) NNK_SLAB_ONE(KERNEL, 1024, 16, __VA_ARGS__); \
+        else NNK_SLAB_ONE(KERNEL, 1024, 32, __VA_ARGS__);                 \
     })
 
 void nnk_gn_fwd_slab(int act, float* y, float* mu, float* rstd, const float* x, const float* gamma, const float* beta,
