@@ -523,8 +523,8 @@ void conv_launch(float* Y, const float* X, const float* Wt, const ConvShape& sh,
 // to 48 MFMAs).  So the stages are pipelined: three LDS buffers and one barrier a
 // stage, the next stage's fragment reads and splits and the one after's loads
 // spread between the MFMAs.  3x3 128 -> 128 at [128, 32, 32]: 264 us with two
-// barriers a stage, 247 so (337 on the fp32 MFMA); 256 -> 256 at [16, 64,
-// 64]: 484, 457.  The column sums of dY (a convolution's bias gradient) come from
+// barriers a stage, 247 so on one box (337 on the fp32 MFMA), 227 on a faster one;
+// 256 -> 256 at [16, 64, 64]: 484, 457, 442.  The column sums of dY (a convolution's bias gradient) come from
 // the rows that the workgroups of the first k tile hold anyway, instead of a
 // pass over dY of two launches (5 us and more).
 // ---------------------------------------------------------------------------
@@ -864,8 +864,8 @@ struct WgradPlan {
 inline int tile_n(int Cout) { return Cout > 64 ? 128 : 64; }
 
 // At most as many splits as one round of resident workgroups holds (two per CU
-// on 256 CUs) and as there are stages of rows.  A plan may have fewer, its rows
-// being whole stages, so the splits do not grow with M (3x3 64 -> 64: 52 at
+// on 256 CUs), of kWgM rows at least.  A plan may have fewer, its rows being
+// multiples of kWgM, so the splits do not grow with M (3x3 64 -> 64: 52 at
 // 3300 rows, 100 at 3200); this bound does, and sizes the workspaces, which
 // serve every smaller batch.
 inline int wgrad_most_splits(int M, int KKC, int Cout) {

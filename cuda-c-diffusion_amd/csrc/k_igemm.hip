@@ -15,29 +15,33 @@
 // fp32 products on the bf16 matrix cores.  v_mfma_f32_32x32x2f32 holds 134
 // TFLOP/s here, v_mfma_f32_32x32x16_bf16 1780 (register-only loops, 512
 // workgroups): 13 times.  Each fp32 operand is split exactly into three bf16
-// planes and six of the nine plane products are formed (igemm.h), 297 TFLOP/s
-// of fp32 products at most.  With data from memory a large bf16 product of the
-// vendor library holds 1250 TFLOP/s, because the clock falls to 1.7 GHz under
-// that load, so 208 is what to expect.  Measured: cfg3 forward (3x3, 128 -> 128,
-// [128, 32, 32]) 320 -> 191 us (202 TFLOP/s), 256 -> 256 at [16, 64, 64] 627 ->
-// 351 us (220), their input gradients 317 -> 193 and 620 -> 359 us, their weight
-// gradients 337 -> 254 and 657 -> 454 us; the forward's matrix cores are busy 0.69
-// of the time at 1.67 GHz, the weight gradient's 0.46 (it splits each operand
+// planes and six of the nine plane products are formed (conv_common.h), 297
+// TFLOP/s of fp32 products at most.  With data from memory a large bf16 product of
+// the vendor library holds 1250 TFLOP/s, because the clock falls to 1.7 GHz under
+// that load, so 208 is what to expect.  Measured, each kernel by itself: 3x3, 128 ->
+// 128 at [128, 32, 32] forward 320 -> 184 us (210 TFLOP/s), 256 -> 256 at [16, 64,
+// 64] 627 -> 355 us (218), their input gradients 317 -> 188 and 620 -> 358 us, their
+// weight gradients (with the sum of the splits) 337 -> 227 and 657 -> 442 us, 5 %
+// more on boxes that clock lower; the forward's matrix cores are busy 0.69 of the
+// time at 1.67 GHz, the weight gradient's 0.46 (it splits each operand
 // again in all nine k tiles, and decodes pixels).  On the way: the fp32 kernel's
 // staging (both operands through LDS per tap, a split of each) 230-260 us;
 // activations staged once per 32 channels for all taps, weights split in
 // registers by the one wave that needs them 205-214; the next step's loads and
-// splits between the MFMAs 191.  Error against 64 bits: below the fp32 MFMA's
-// at every size measured (igemm.h).
+// splits between the MFMAs 184-191.  Error against 64 bits: below the fp32 MFMA's
+// at every size measured (conv_common.h).  Convolutions with a trained gain stay on
+// the fp32 MFMA all the same (k_igemm_f32.hip).
 //
 // Lane layout of v_mfma_f32_32x32x16_bf16 (checked on the device): lane l
 // supplies A[l % 32][8 (l / 32) .. + 7] and B[8 (l / 32) .. + 7][l % 32];
 // accumulator register r of lane l holds D[8 (r / 4) + 4 (l / 32) + r % 4][l %
 // 32].
 //
-// Summation order: each output is a fixed-order sum (slices of 32 channels,
-// taps, halves of 16), the same on every run and in both staging forms; it
-// differs from a library GEMM's order by rounding only.
+// Summation order: each output is a fixed-order sum, the same on every run: in the
+// tiled kernels (igemm.h) slices of 32 channels, taps, halves of 16, in every staging
+// form; in the small tiles (k_conv_small.hip) a wave's taps and channels, then the
+// waves.  Which of them a shape takes is fixed too (conv_tile, small_us).  Orders
+// differ from each other and from a library GEMM's by rounding only.
 #include "igemm.h"
 
 #include "conv_api.h"

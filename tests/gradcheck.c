@@ -443,9 +443,10 @@ int nn_gradcheck_run(int verbose)
     fails += check_module("conv1x1_mp", conv2d_create(&g_ctx, 4, 6, 1, 1, 0, 5, 5, B, 1, 1.0f), B, 2e-2);
     fails += check_module("conv3x3_s2", conv2d_create(&g_ctx, 4, 4, 3, 2, 1, 7, 7, B, 0, 1.0f), B, 2e-2);
     fails += check_module("linear", linear_create(&g_ctx, 12, 8), B, 2e-2);
-    /* channel counts that take the implicit-GEMM forward, weight gradient and
-       (C_in % 128 == 0, stride 1) input gradient; forced, since at these few
-       pixels the module's cost model would pick im2col + rocBLAS */
+    /* channel counts at which the modules with a gain take the fp32 matrix-core
+       kernels each way (input gradient: stride 1); forced, since at these few pixels
+       their cost model would pick im2col + rocBLAS.  Those without one take the
+       matrix-core kernels anyway */
     setenv("NNHIP_CONV_PATH", "implicit", 1);
     fails += check_module("conv3x3_implicit", conv2d_create(&g_ctx, 128, 128, 3, 1, 1, 4, 4, B, 0, 1.0f), B, 2e-2);
     fails += check_module("conv3x3_implicit_mp", conv2d_create(&g_ctx, 128, 128, 3, 1, 1, 4, 4, B, 1, 1.0f), B,
