@@ -169,13 +169,25 @@ def test_weight_gradient_workspace_serves_smaller_batches(nn, ci, co, k, hw):
     """A module's workspace has the size for its max_batch and serves every
     smaller batch, whose rows may be split into more parts."""
     L = nn.lib()
-    own = L.dll.nnk_conv_weight_grad_workspace
-    own.argtypes, own.restype = [ctypes.c_int] * 6, ctypes.c_size_t
-    for size in (L.nnhip_conv2d_wgrad_workspace, own):
+    own, f32 = L.dll.nnk_conv_weight_grad_workspace, L.dll.nnk_conv_f32_weight_grad_workspace
+    for f in (own, f32):
+        f.argtypes, f.restype = [ctypes.c_int] * 6, ctypes.c_size_t
+    for size in (L.nnhip_conv2d_wgrad_workspace, own, f32):
         sizes = [size(b, ci, co, k, hw, hw) for b in range(1, 400)]
         assert sizes == sorted(sizes)
         # as many parts as there are stages of 32 rows, until the device is full
         assert sizes[39] >= min(512 // (-(-k * k * ci // 128) * -(-co // 128)), -(-40 * hw * hw // 32)) * k * k * ci * co
+        assert size is not f32 or all(a >= s for s, a in zip(_f32_splits(ci, co, k, hw), sizes))
+
+
+def _f32_splits(ci, co, k, hw):
+    """Floats of partial sums that each batch from 1 on writes: its rows in multiples of 32."""
+    tiles = -(-k * k * ci // 128) * (co // (64 if co % 128 else 128))
+    for b in range(1, 400):
+        m = b * hw * hw
+        most = min(max(1, 512 // tiles), -(-m // 32))
+        rows = -(-(-(-m // most)) // 32) * 32
+        yield -(-m // rows) * k * k * ci * co if m > rows else 0
 
 
 def test_convolution_kernels_stay_in_their_index_range(nn):

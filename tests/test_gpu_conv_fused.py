@@ -11,7 +11,8 @@ the pass it replaces, so the comparison is bit for bit:
 The separate launches themselves are checked against the oracle by
 test_gpu_conv_implicit.py, test_gpu_spatial.py and test_gpu_elementwise.py.
 Geometries cover a partial row tile, both output-channel tile widths, stride 2
-and the EDM block's cfg2 shape."""
+and the EDM block's cfg2 shape, each in the form that the rules choose (the small
+ones in the small tiles; test_gpu_conv_forms.py names the forms)."""
 from __future__ import annotations
 
 import ctypes as C

@@ -10,7 +10,8 @@ reference's sequences restated on the CPU in double:
   of the oracle's im2col, summed in double.
 Bar 1e-5 relative to max(|ref|, sqrt(sum of the squared products)) per
 output (each output is a sum of many products), plus the refusal of shapes
-the kernels do not take."""
+the kernels do not take.  Each geometry runs in the form that the rules choose, the
+small ones in the small tiles; test_gpu_conv_forms.py names the forms."""
 from __future__ import annotations
 
 import numpy as np

@@ -1,4 +1,4 @@
-"""The products of the conv2d, linear and mp_linear modules (host/conv_api.h) at
+"""The products of the conv2d and linear modules (host/conv_api.h) at
 any channel counts and alignment, at the edges of the small tiles (32 x 32
 outputs and 16 k a step, or 16 x 16 and 32 k, 4 / 8 / 16 waves) and of the tiled kernels' ragged forms,
 against double; bar as in test_gpu_conv_implicit.py.  Geometries past each rule

@@ -3,7 +3,9 @@ convolutions' matrix-core kernels: operands that are infinite, NaN or so large
 that they round to infinity in bf16, operands too small for the split, a mean
 error that sums would show, and the edges of the staging (halo rows at image
 borders and between samples, tiles past the end, widths that leave the halo
-form).  Reference: the same sums in double.  Bar for finite values as in
+form), by the launchers and so in the form that the rules choose: for shapes as
+small as these the small tiles.  test_gpu_conv_forms.py runs them in every form.
+Reference: the same sums in double.  Bar for finite values as in
 test_gpu_conv_implicit.py: 1e-5 relative to max(|ref|, sqrt(sum of the squared
 products))."""
 from __future__ import annotations

@@ -139,3 +139,50 @@ def test_mp_linear_is_the_library_product(L, shape):
     terms = (wn * wn * ((x64 * x64).T @ (g64 * g64))).sum()
     assert abs(m.get(1, True)[0] - (wn * (x64.T @ g64)).sum()) <= TOL * np.sqrt(terms)
     m.free()
+
+
+@pytest.mark.parametrize("geom", [(3, 5, 7, 32, 128, 3, 1), (2, 9, 9, 64, 64, 3, 1), (2, 8, 8, 64, 192, 1, 0), (1, 9, 9, 128, 64, 5, 2)],
+                         ids=lambda g: "x".join(map(str, g)))
+def test_fused_epilogues_of_the_fp32_kernels(L, nn, rng, geom):
+    """Tiles that end within the tensor and both tile widths: the neighbours in the epilogue against the separate
+    launches, bit for bit."""
+    B, H, W, Ci, Co, K, p = geom
+    print(f"[case] fp32 kernels' epilogues {geom}", flush=True)
+    d, P, I = L.dll, C.c_void_p, C.c_int
+    d.nnk_conv_f32_forward.argtypes, d.nnk_conv_f32_forward.restype = [P] * 4 + [I] * 10 + [P, P], None
+    d.nnk_conv_f32_input_grad.argtypes, d.nnk_conv_f32_input_grad.restype = [P] * 4 + [I] * 7 + [P, P], None
+    n, ni = B * H * W * Co, B * H * W * Ci
+
+    def dev(*shape, scale=1.0):
+        return L.to_device((scale * rng.standard_normal(shape)).astype(np.float32))
+
+    xd, wd, cond, res = dev(ni), dev(K * K * Ci, Co, scale=0.1), dev(B, Co, scale=0.5), dev(n)
+    gain = L.to_device(np.array([0.91], np.float32))
+    y, want, got, y2 = L.alloc(n), L.alloc(n), L.alloc(n), L.alloc(n)
+    geo = (B, H, W, Ci, Co, K, 1, p, H, W)
+    d.nnk_conv_f32_forward(y.p, xd.p, wd.p, gain.p, *geo, None, None)
+    f = nn.NnConvFusion(cond=cond.p, y2=y2.p, act=nn.ACT_MP_SILU)
+    d.nnk_conv_f32_forward(got.p, xd.p, wd.p, gain.p, *geo, C.addressof(f), None)
+    L.launch_spatial_modulate_act_forward(want.p, y.p, cond.p, B, H * W, 1, Co, nn.ACT_MP_SILU, None)
+    L.sync()
+    L.check("modulate")
+    assert_bits_equal(got.download(), y.download(), "y")
+    assert_bits_equal(y2.download(), want.download(), "y2")
+    f = nn.NnConvFusion(res=res.p, res_w=0.83, out_w=0.55)
+    d.nnk_conv_f32_forward(got.p, xd.p, wd.p, gain.p, *geo, C.addressof(f), None)
+    L.launch_weighted_sum(want.p, res.p, y.p, 0.83, 0.55, n, None)
+    L.sync()
+    assert_bits_equal(got.download(), want.download(), "residual")
+    if Ci % 64 or Co % 32:
+        return
+    gd, act, resi, dx, t = dev(n), dev(ni), dev(ni), L.alloc(ni), L.alloc(ni)
+    d.nnk_conv_f32_input_grad(dx.p, gd.p, wd.p, gain.p, B, H, W, Ci, Co, K, p, None, None)
+    f = nn.NnConvFusion(act_in=act.p, act=nn.ACT_MP_SILU, res=resi.p, res_w=0.83, out_w=1.0)
+    d.nnk_conv_f32_input_grad(t.p, gd.p, wd.p, gain.p, B, H, W, Ci, Co, K, p, C.addressof(f), None)
+    L.sync()
+    L.check("activation gradient")
+    fused = t.download()
+    L.launch_activation_backward(t.p, dx.p, act.p, ni, nn.ACT_MP_SILU, None)
+    L.launch_weighted_sum(t.p, resi.p, t.p, 0.83, 1.0, ni, None)
+    L.sync()
+    assert_bits_equal(fused, t.download(), "input gradient")
